@@ -22,7 +22,8 @@
 //  * tiled (n_e > 64, prefill): MFMA-bound.  Persistent workgroups walk a device-computed
 //    list of 256x256 output tiles; A (gathered x rows / activation rows) and B (weight rows)
 //    tiles of 64 along K are staged by direct global->LDS loads into a swizzled,
-//    double-buffered LDS layout.  v_mfma_f32_32x32x16_bf16, eight wavefronts of 128x64.
+//    double-buffered LDS layout.  v_mfma_f32_16x16x32_bf16, eight wavefronts, the two of a SIMD
+//    taking turns on the matrix core and on memory.
 // Phase 1 ("up") computes the gate and up projections together and applies silu(g)*u in the
 // epilogue; phase 2 ("down") applies the routing weight in the epilogue and writes the
 // per-(token, expert) row that the combine kernel sums.
@@ -126,7 +127,7 @@ __device__ __forceinline__ const T* uniform_ptr(const T* p) {
 // 16-byte global->LDS direct load of each lane: global address sbase + voff (wave-uniform base
 // in scalar registers, 32-bit lane byte offset), LDS byte address lds + 16 * lane.  Issued as
 // inline asm so that the address keeps this form wherever the load is scheduled; the compiler
-// does not track these loads, their completion is awaited with wait_vmcnt0.  The asm writes
+// does not track these loads, their completion is awaited with wait_cnt / wait_vmcnt.  The asm writes
 // m0 (the LDS base of the direct load); nothing else in these kernels uses m0.  An LDS direct
 // load needs one wait state between the SALU write of m0 and its issue (the s_nop), which the
 // compiler's hazard pass would add for its own instructions but cannot see inside the asm.
@@ -139,25 +140,18 @@ __device__ __forceinline__ void dma16(const char* sbase, uint32_t voff, uint32_t
       : "v"(voff), "s"(sbase), "s"(lds)
       : "memory", "m0");
 }
-// wait until at most N of this wavefront's vector-memory operations are outstanding
-__device__ __forceinline__ void wait_vmcnt0() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 typedef __attribute__((address_space(3))) char lds_char;
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return (uint32_t)(uintptr_t)(lds_char*)p;
 }
-// LDS fragment read issued as inline asm: the compiler cannot see that it reads memory that
-// the in-flight direct loads write, so it does not insert a vmcnt(0) drain in front of it.
-// Completion is awaited explicitly with lds_wait, which also ties the fragment registers.
-template <int OFF>
-__device__ __forceinline__ void ds_read16(bf16x8& v, uint32_t addr) {
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF) : "memory");
-}
-__device__ __forceinline__ void lds_wait(bf16x8 (&a)[4], bf16x8 (&b)[2]) {
-  asm volatile("s_waitcnt lgkmcnt(0)"
-               : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1])
-               :
-               : "memory");
+// wait until at most VM vector-memory operations (the direct loads among them) and no LDS reads
+// of this wavefront are outstanding, in a form whose LDS part the compiler knows of
+template <int VM>
+__device__ __forceinline__ void wait_cnt() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt((VM & 15) | (7 << 4) | ((VM >> 4) << 14));
+  asm volatile("" ::: "memory");
 }
 // workgroup barrier without the release/acquire fence of __syncthreads (which would drain
 // the direct loads of the later stages); LDS visibility is established by the explicit waits
@@ -1184,22 +1178,54 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void f
 // Tiled kernels
 // =============================================================================================
 
-// Output tile 256 x 256 per workgroup (the wavefront layout is described at ffn_tiled).
-// Phase 1's 256 B rows are 128 gate rows and the 128 up rows of the same intermediate columns,
-// so every wavefront owns matching gate/up accumulators and the SwiGLU runs in registers.
+// Output tile 256 x 256 per workgroup, eight wavefronts, two per SIMD.  Bound by the matrix cores
+// (and, under them, by the clock that the power limit leaves: 1.6-1.7 GHz).
 //
-// Operand staging: global -> LDS direct loads (global_load_lds_dwordx4, no VGPR round trip).
-// A stage holds BK = 64 columns of K: 256 A rows and 256 B rows of 128 bytes.  One direct
-// load moves 8 full rows (64 lanes x 16 B, lane l -> row l / 8, LDS slot l % 8), which keeps
-// the global side fully coalesced.  Inside a row the 16-byte chunk c is stored at slot
-// c ^ ((row >> 1) & 7): the MFMA fragment read (32 rows x one chunk per half-wavefront) then
-// touches 16 distinct 16-byte bank groups in every 16 lanes, i.e. no LDS bank conflicts.
-// Two stages (2 x 64 KiB): the loads of stage kt+1 run while stage kt is multiplied.
-constexpr int BM = 256, BN = 256, BK = 64, STAGES = 2;
-constexpr int kRowBytes = BK * 2;                                // 128
-constexpr int kOperandBytes = 256 * kRowBytes;                   // 32 KiB per operand tile
-constexpr int kStageBytes = 2 * kOperandBytes;                   // A then B
-constexpr int kTileLds = STAGES * kStageBytes / 2;               // bf16 elements (128 KiB)
+// Halves and quadrants.  A stage holds BK = 64 columns of K: 256 A rows and 256 B rows of 128
+// bytes, each operand cut into two halves of 128 rows (16 KiB).  Wavefront (wm, wn) = (w / 4,
+// w % 4) computes in each of the four quadrants (A half, B half) the 64 rows 32 i + 16 wm + [0, 16)
+// (i < 4) by the 32 columns 32 wn + [0, 32): 16 v_mfma_f32_16x16x32_bf16, 256 cycles.  In phase 1
+// the B halves are 128 gate rows and the 128 up rows of the same intermediate columns, so every
+// wavefront owns matching gate / up accumulators and the SwiGLU runs in registers.
+//
+// Ping-pong.  A stage is four phases, each a memory segment (the LDS reads of one half's
+// fragments, the direct loads of another half) and a matrix segment (one quadrant's products), a
+// barrier after each.  The wavefronts wm = 1 run one segment behind those of wm = 0, the other
+// wavefront of the same SIMD: while one multiplies, its partner reads fragments and issues loads,
+// and the two never compete for the matrix core or for the LDS.
+//
+//   phase            1        2        3        4
+//   reads            A0(k)    B1(k)    A1(k)    B0(k+1)
+//   loads            B0(k+2)  A0(k+2)  B1(k+2)  A1(k+2)    (into the half read one phase before)
+//   multiplies       A0 B0    A0 B1    A1 B0    A1 B1
+//
+// Loads in flight.  Each half is loaded seven phases (about 2.2 us) before it is read, into the
+// buffer that the previous phase read: two stages of LDS (128 KiB) hold up to seven halves in
+// flight.  A wavefront issues two loads a phase, so "at most 12 outstanding" before the barrier
+// says that its share of the half read next has landed; nothing in the loop waits for all loads.
+// Before this schedule (one barrier and a full drain of the loads per stage, both wavefronts of a
+// SIMD waiting together) a stage took 1.7 us of the 1.31 us it takes now.  One dense expert of
+// 65,536 rows, H x I = 2048 x 768: up 352 -> 300 us (1173 -> 1372 TFLOP/s), down 233 -> 209 us
+// (883 -> 986); 2048 x 1408: up 1177 -> 1390, down 1048 -> 1208; 2048 x 4096 down 1240 -> 1467.
+// The same products are summed in the same K order as before: results are bit-identical.
+//
+// Operand staging: global -> LDS direct loads (global_load_lds_dwordx4, no VGPR round trip).  One
+// load moves 8 full rows (64 lanes x 16 B, lane l -> row l / 8, LDS slot l % 8), fully coalesced.
+// Inside a row the 16-byte chunk c is stored at slot c ^ swizzle(row); with two 128-byte rows per
+// 256-byte bank line, the 16 rows that a quarter of a wavefront reads then touch 16 distinct
+// 16-byte bank groups.  The rows are 16 consecutive ones for A, and {8 g + 4 c + [0, 4)} for B
+// (below), hence the two swizzles.
+//
+// The products take the weight rows as first operand and the token rows as second: a lane then
+// holds four consecutive weight rows (output columns) of one token row.  The B fragments of the
+// column tiles c = 0, 1 take the weight rows 8 g + 4 c + [0, 4) (g < 4), so that the two tiles
+// give a lane eight consecutive columns: the epilogue packs them into one 16-byte store, with no
+// LDS staging, one row address and one routing weight per 16-row tile.
+constexpr int BM = 256, BN = 256, BK = 64;
+constexpr int kRowBytes = BK * 2;                  // 128
+constexpr int kHalfBytes = 128 * kRowBytes;        // half an operand tile of one stage: 16 KiB
+__device__ __forceinline__ int swz_a(int row) { return (row >> 1) & 7; }
+__device__ __forceinline__ int swz_b(int row) { return ((row >> 1) & 1) | (((row >> 3) & 3) << 1); }
 
 struct TileTable {
   int32_t cum[kListMax + 1];  // cumulative M tiles over list entries
@@ -1262,22 +1288,16 @@ __device__ __forceinline__ int find_entry(const TileTable& tt, int m) {
   return lo;
 }
 
-// MODE 0: A = gathered x rows (K = H); B rows 0..127 = Wg[i0 ..], 128..255 = Wu[i0 ..];
-//         epilogue act[p, i0 + c] = bf16(silu(bf16(g)) * bf16(u)).
-// MODE 1: A = activation rows (K = I); B rows = Wd[h0 ..];
+// MODE 0: A = gathered x rows (K = H); B half 0 = gate rows i0 .. +128, half 1 = the up rows of
+//         the same columns; epilogue act[p, i0 + c] = bf16(silu(bf16(g)) * bf16(u)).
+// MODE 1: A = activation rows (K = I); B half h = down rows h0 + 128 h .. +128;
 //         epilogue out[row(p), h0 + c] = bf16(bf16(y) * w(p)).
-//
-// Eight wavefronts, two per SIMD: wavefront (wm, wn) = (w / 4, w % 4) computes rows
-// 128 wm .. +128 of the tile and a quarter of its columns (MODE 0: gate and up columns
-// 32 wn .. +32, MODE 1: columns 64 wn .. +64), 4 x 2 tiles of 32x32 (128 accumulators).
-// A wavefront that stalls -- issuing its direct loads while the address unit drains the
-// others', or waiting for LDS fragments -- leaves its SIMD to the other wavefront's MFMAs.
 constexpr int kTiledThreads = 512;
 template <int MODE>
-__global__ __launch_bounds__(kTiledThreads, 1) void ffn_tiled(FfnArgs a) {
+__global__ __launch_bounds__(kTiledThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void ffn_tiled(FfnArgs a) {
   __shared__ TileTable tt;
-  __shared__ __attribute__((aligned(1024))) bf16_t smem[kTileLds];
-  __shared__ int64_t orow_s[BM];   // phase 2: byte offset of each tile row's output row
+  __shared__ __attribute__((aligned(1024))) char smem[8 * kHalfBytes];
+  __shared__ int64_t orow_s[BM];   // phase 2: element offset of each tile row's output row
   __shared__ float wt_s[BM];
   build_tile_table(a, tt);
   const int64_t K = MODE == 0 ? a.H : a.I;
@@ -1286,8 +1306,18 @@ __global__ __launch_bounds__(kTiledThreads, 1) void ffn_tiled(FfnArgs a) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 2, wn = wave & 3;
-  const int KT = (int)(K / BK);
-  const int l32 = lane & 31;
+  const int KT = (int)(K / BK);   // even: H and I are multiples of 128
+  const int j16 = lane & 15, g4 = lane >> 4;
+
+  // fragment reads (byte address of K step ks; tile i / c, half and slot go into the offset)
+  const uint32_t smem0 = lds_addr(smem);
+  uint32_t a_addr[2], b_addr[2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+    const int arow = 16 * wm + j16, brow = 32 * wn + 8 * (j16 >> 2) + (j16 & 3);
+    a_addr[ks] = (uint32_t)(arow * kRowBytes + (((4 * ks + g4) ^ swz_a(arow)) << 4));
+    b_addr[ks] = (uint32_t)(4 * kHalfBytes + brow * kRowBytes + (((4 * ks + g4) ^ swz_b(brow)) << 4));
+  }
 
   // XCD-aware order: workgroup b runs on XCD b % 8 (round-robin dispatch), so in each round
   // of gridDim tiles the workgroups of one XCD take a contiguous run of tiles.  Tiles of one
@@ -1303,49 +1333,35 @@ __global__ __launch_bounds__(kTiledThreads, 1) void ffn_tiled(FfnArgs a) {
     const int m0 = (mt_global - tt.cum[li]) * BM;
     const bf16_t* slot = a.cache + (int64_t)a.list.slot[li] * 3 * a.H * a.I;
 
-    // Direct loads: this wavefront moves tile rows 32*wave + 8*q + lane/8 (q < 4) of A and of
-    // B, lane slot lane % 8 holding chunk (lane % 8) ^ ((row >> 1) & 7).  Rows past the
-    // expert's last row load a valid row instead: each output row depends only on its own A
-    // row, and those rows are never stored.
+    // Direct loads: of each half this wavefront moves rows 16 wave + 8 q + lane / 8 (q < 2), lane
+    // slot lane % 8 holding the row's chunk (lane % 8) ^ swizzle(row).  Rows past the expert's
+    // last row load its first row instead: each output row depends only on its own A row, and
+    // those rows are never stored.
     const int r8 = lane >> 3, slot8 = lane & 7;
-    // byte offsets of this lane's A rows (+ chunk) from abase: < 2^32 (host-checked sizes)
-    uint32_t aoff[4];
+    uint32_t aoff[2][2], boff[2];   // byte offsets: < 2^32 (host-checked sizes)
     const char* abase = reinterpret_cast<const char*>(MODE == 0 ? a.x : a.act);
     const uint32_t lda = (uint32_t)(MODE == 0 ? a.H : a.I);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int row = 32 * wave + 8 * q + r8;
-      const int chunk = slot8 ^ ((row >> 1) & 7);
-      const int r = m0 + row;
-      const bool ok = r < n;
-      const uint32_t t = MODE == 0 ? (uint32_t)a.rows[start + (ok ? r : 0)]
-                                   : (uint32_t)(start + (ok ? r : 0));
-      aoff[q] = (t * lda + (uint32_t)(chunk * 8)) * 2u;
-    }
-    // B rows of this wavefront: 32*wave .. +32 (MODE 0: waves 0-3 gate rows, 4-7 up rows)
-    const int64_t ldb = MODE == 0 ? a.H : a.I;
-    const int brow0 = 32 * wave;
-    const char* bbase = reinterpret_cast<const char*>(uniform_ptr(
-        MODE == 0 ? slot + (brow0 < 128 ? (int64_t)(ntile * 128 + brow0) * a.H
-                                        : a.H * a.I + (int64_t)(ntile * 128 + brow0 - 128) * a.H)
-                  : slot + 2 * a.H * a.I + (int64_t)(ntile * BN + brow0) * a.I));
-    uint32_t boff[4];
+    for (int q = 0; q < 2; ++q) {
+      const int row = 16 * wave + 8 * q + r8;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int row = brow0 + 8 * q + r8;
-      boff[q] = (uint32_t)(((8 * q + r8) * ldb + (slot8 ^ ((row >> 1) & 7)) * 8) * 2);
+      for (int h = 0; h < 2; ++h) {
+        const int r = m0 + 128 * h + row;
+        const bool ok = r < n;
+        const uint32_t t = MODE == 0 ? (uint32_t)a.rows[start + (ok ? r : 0)]
+                                     : (uint32_t)(start + (ok ? r : 0));
+        aoff[h][q] = (t * lda + (uint32_t)((slot8 ^ swz_a(row)) * 8)) * 2u;
+      }
+      boff[q] = (uint32_t)(((uint32_t)(8 * q + r8) * (uint32_t)K + (uint32_t)((slot8 ^ swz_b(row)) * 8)) * 2u);
     }
-    const uint32_t lds_smem = lds_addr(smem);
-    // Rows past the expert's last one (the partial last M tile of an expert) are not computed:
-    // in such a tile the A direct loads of 8-row groups that lie wholly past it are skipped,
-    // and so are the MFMAs of 32-row blocks that do.  Their LDS rows then hold stale data, which
-    // only reaches output rows that are never stored.  Full tiles run a copy of the loop
-    // without these tests.
+    const char* bbase[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      bbase[h] = reinterpret_cast<const char*>(uniform_ptr(
+          MODE == 0 ? slot + (int64_t)h * a.H * a.I + (int64_t)(ntile * 128 + 16 * wave) * a.H
+                    : slot + 2 * a.H * a.I + (int64_t)(ntile * BN + 128 * h + 16 * wave) * a.I));
     const int vrows = n - m0;                                          // > 0
-    const int nfa = __builtin_amdgcn_readfirstlane(
-        vrows >= wm * 128 + 128 ? 4 : (vrows > wm * 128 ? (vrows - wm * 128 + 31) / 32 : 0));
-    // per-row output row and routing weight for the phase-2 epilogue; run after the first
-    // stage's direct loads are issued, so that its dependent loads overlap them
+    // per-row output row and routing weight for the phase-2 epilogue
     auto row_meta = [&]() {
       if (MODE == 1) {
         for (int r = tid; r < BM; r += kTiledThreads) {
@@ -1356,7 +1372,7 @@ __global__ __launch_bounds__(kTiledThreads, 1) void ffn_tiled(FfnArgs a) {
             const int64_t p = start + rr;
             const int64_t t = a.rows[p], j = a.cols[p];
             wt = bf16_to_f32(a.w[t * a.k + j]);
-            orow = (a.out_mode == 0 ? t * a.k + j : p) * a.H * 2;   // byte offset of the row
+            orow = (a.out_mode == 0 ? t * a.k + j : p) * a.H;
           }
           orow_s[r] = orow;
           wt_s[r] = wt;
@@ -1364,189 +1380,182 @@ __global__ __launch_bounds__(kTiledThreads, 1) void ffn_tiled(FfnArgs a) {
       }
     };
 
-    floatx16 acc[4][2];
+    floatx4 acc[2][2][4][2];   // [A half][B half][16-row tile][16-column tile]
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int ha = 0; ha < 2; ++ha)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int hb = 0; hb < 2; ++hb)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-
-    // Fragment addresses.  Lane l reads row (first row of the fragment) + l % 32, chunk
-    // 2*sub + l / 32, at byte row*128 + ((chunk ^ ((row >> 1) & 7)) << 4); fragment rows are
-    // multiples of 32 apart, so the swizzle term only depends on the lane and the sub-step.
-    // A fragments i: rows wm*128 + 32 i.  B fragments j: MODE 0 gate rows 32 wn (j = 0) and
-    // up rows 128 + 32 wn (j = 1); MODE 1 rows 64 wn + 32 j.
-    const uint32_t smem_base = lds_addr(smem);
-    const int swz = (l32 >> 1) & 7, half = lane >> 5;
-    uint32_t a_addr[4], b_addr[4];
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int sub = 0; sub < 4; ++sub) {
-      const uint32_t slotb = (uint32_t)((((2 * sub + half) ^ swz)) << 4);
-      a_addr[sub] = smem_base + (uint32_t)((wm * 128 + l32) * kRowBytes) + slotb;
-      b_addr[sub] = smem_base + kOperandBytes + (uint32_t)(((MODE == 0 ? wn * 32 : wn * 64) + l32) * kRowBytes) + slotb;
+          for (int c = 0; c < 2; ++c) acc[ha][hb][i][c] = floatx4{0, 0, 0, 0};
+    // 16-row tiles of each A half that hold rows of the expert (the others' products are skipped
+    // in a partial tile: their output rows are never stored)
+    int nf[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int v = vrows - 128 * h - 16 * wm;
+      nf[h] = __builtin_amdgcn_readfirstlane(v >= 128 ? 4 : (v > 0 ? (v + 31) / 32 : 0));
     }
-    auto rd = [&](int kt, int sub, bf16x8 (&fa)[4], bf16x8 (&fb)[2]) {
-      const uint32_t so = (uint32_t)((kt % STAGES) * kStageBytes);
-      const uint32_t ab = a_addr[sub] + so, bb = b_addr[sub] + so;
-      ds_read16<0 * 4096>(fa[0], ab);
-      ds_read16<1 * 4096>(fa[1], ab);
-      ds_read16<2 * 4096>(fa[2], ab);
-      ds_read16<3 * 4096>(fa[3], ab);
-      ds_read16<0>(fb[0], bb);
-      ds_read16<MODE == 0 ? 16384 : 4096>(fb[1], bb);
+
+    bf16x8 ft[4][2], fw[2][2][2];
+    auto dma_a = [&](int kt, int h, int s) {
+      const uint32_t dst = smem0 + (uint32_t)((2 * h + s) * kHalfBytes + 16 * wave * kRowBytes);
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        dma16(abase + kt * BK * 2, aoff[h][q], dst + (uint32_t)(8 * q * kRowBytes));
+    };
+    auto dma_b = [&](int kt, int h, int s) {
+      const uint32_t dst = smem0 + (uint32_t)((4 + 2 * h + s) * kHalfBytes + 16 * wave * kRowBytes);
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        dma16(bbase[h] + kt * BK * 2, boff[q], dst + (uint32_t)(8 * q * kRowBytes));
+    };
+    auto read_a = [&](auto h, auto s) {
+      constexpr int off = (2 * decltype(h)::value + decltype(s)::value) * kHalfBytes;
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          ft[i][ks] = *reinterpret_cast<const bf16x8*>(smem + a_addr[ks] + off + i * 32 * kRowBytes);
+    };
+    auto read_b = [&](auto h, auto s) {
+      constexpr int H = decltype(h)::value, off = (2 * H + decltype(s)::value) * kHalfBytes;
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+          fw[H][c][ks] = *reinterpret_cast<const bf16x8*>(smem + b_addr[ks] + off + c * 4 * kRowBytes);
     };
     auto pipeline = [&](auto part) {
-    constexpr bool PARTIAL = decltype(part)::value;
-    // direct load n (< 8) of stage kt: A rows 32 wave + 8n of this wavefront for n < 4, B rows
-    // 32 wave + 8 (n - 4) for n >= 4
-    auto dma = [&](int kt, int n) {
-      const uint32_t st = lds_smem + (uint32_t)((kt % STAGES) * kStageBytes + 32 * wave * kRowBytes);
-      const int q = n & 3;
-      if (n < 4) {
-        if (!PARTIAL || 32 * wave + 8 * q < vrows)
-          dma16(abase + kt * BK * 2, aoff[q], st + (uint32_t)(8 * q * kRowBytes));
-      } else {
-        dma16(bbase + kt * BK * 2, boff[q], st + (uint32_t)(kOperandBytes + 8 * q * kRowBytes));
+      constexpr bool PARTIAL = decltype(part)::value;
+      auto mma = [&](auto ha, auto hb) {
+        constexpr int A = decltype(ha)::value, B = decltype(hb)::value;
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (!PARTIAL || i < nf[A]) {
+#pragma unroll
+              for (int c = 0; c < 2; ++c)
+                acc[A][B][i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[B][c][ks], ft[i][ks],
+                                                                         acc[A][B][i][c], 0, 0, 0);
+            }
+        __builtin_amdgcn_s_setprio(0);
+        wg_barrier();
+      };
+      // end of a memory segment: the loads of the next segment's half have landed (at most N
+      // younger ones in flight), this segment's fragments are in registers
+      auto mem_end = [&](auto nn) {
+        wait_cnt<decltype(nn)::value>();
+        wg_barrier();
+      };
+      typedef std::integral_constant<int, 0> I0;
+      typedef std::integral_constant<int, 1> I1;
+      // stage k in slot S; LAST: the last two stages issue no loads
+      auto stage = [&](int k, auto ss, auto tail) {
+        constexpr int S = decltype(ss)::value;
+        constexpr int T = decltype(tail)::value;   // 0, or 1 / 2 for the last but one / last stage
+        typedef std::integral_constant<int, S> IS;
+        typedef std::integral_constant<int, 1 - S> IO;
+        auto left = [&](auto ph) {   // loads in flight after phase ph's memory segment
+          constexpr int v = T == 0 ? 12 : 12 - 2 * (4 * (T - 1) + decltype(ph)::value + 1);
+          return std::integral_constant<int, (v > 0 ? v : 0)>{};
+        };
+        read_a(I0{}, IS{});
+        if constexpr (T == 0) dma_b(k + 2, 0, S);
+        mem_end(left(std::integral_constant<int, 0>{}));
+        mma(I0{}, I0{});
+        read_b(I1{}, IS{});
+        if constexpr (T == 0) dma_a(k + 2, 0, S);
+        mem_end(left(std::integral_constant<int, 1>{}));
+        mma(I0{}, I1{});
+        read_a(I1{}, IS{});
+        if constexpr (T == 0) dma_b(k + 2, 1, S);
+        mem_end(left(std::integral_constant<int, 2>{}));
+        mma(I1{}, I0{});
+        if constexpr (T < 2) read_b(I0{}, IO{});
+        if constexpr (T == 0) dma_a(k + 2, 1, S);
+        mem_end(left(std::integral_constant<int, 3>{}));
+        mma(I1{}, I1{});
+      };
+      // prologue: both stages' halves in the order in which they are read
+      dma_b(0, 0, 0);
+      dma_a(0, 0, 0);
+      dma_b(0, 1, 0);
+      dma_a(0, 1, 0);
+      dma_b(1, 0, 1);
+      dma_a(1, 0, 1);
+      dma_b(1, 1, 1);
+      dma_a(1, 1, 1);
+      asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+      wg_barrier();
+      read_b(I0{}, I0{});
+      // every wavefront has read B half 0 of stage 0 before stage 0's first loads replace it
+      wait_cnt<12>();
+      wg_barrier();
+      if (wm == 1) wg_barrier();   // the second group runs one segment behind the first
+      int k = 0;
+      for (; k + 2 < KT; k += 2) {
+        stage(k, I0{}, I0{});
+        stage(k + 1, I1{}, I0{});
       }
+      stage(k, I0{}, I1{});
+      stage(k + 1, I1{}, std::integral_constant<int, 2>{});
+      if (wm == 0) wg_barrier();
     };
-    auto issue = [&](int kt) {
-#pragma unroll
-      for (int n = 0; n < 8; ++n) dma(kt, n);
-    };
-    auto mma = [&](const bf16x8 (&fa)[4], const bf16x8 (&fb)[2]) {
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (!PARTIAL || i < nfa) {
-#pragma unroll
-          for (int j = 0; j < 2; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
-        }
-      __builtin_amdgcn_sched_barrier(0);
-    };
-    // pipeline: stage kt+1 streams in while stage kt is multiplied; the fragments of the next
-    // sub-step are read while the MFMAs of the current one run
-    bf16x8 f0a[4], f0b[2], f1a[4], f1b[2];
-    issue(0);
     row_meta();
-    wait_vmcnt0();
-    wg_barrier();
-    if (1 < KT) issue(1);
-    rd(0, 0, f0a, f0b);
-    lds_wait(f0a, f0b);
-    for (int kt = 0; kt < KT; ++kt) {
-      rd(kt, 1, f1a, f1b);
-      mma(f0a, f0b);
-      lds_wait(f1a, f1b);
-      rd(kt, 2, f0a, f0b);
-      mma(f1a, f1b);
-      lds_wait(f0a, f0b);
-      rd(kt, 3, f1a, f1b);
-      mma(f0a, f0b);
-      lds_wait(f1a, f1b);  // stage kt fully read by this wavefront
-      const bool more = kt + 1 < KT;
-      if (more) {
-        wait_vmcnt0();   // this wavefront's loads of stage kt+1 landed
-        wg_barrier();    // ... everyone's; and stage kt is no longer read by anyone
-        // stage kt+2 into the buffer stage kt just freed.  The two wavefronts of a SIMD (wm 0
-        // and 1) issue their direct loads one MFMA group apart, so that one runs its MFMAs
-        // while the other waits for the address unit to take its loads.
-        if (kt + 2 < KT && wm == 0) issue(kt + 2);
-        rd(kt + 1, 0, f0a, f0b);
-      }
-      mma(f1a, f1b);
-      if (more) {
-        if (kt + 2 < KT && wm == 1) issue(kt + 2);
-        lds_wait(f0a, f0b);
-      }
-    }
-    };
     if (vrows >= BM)
       pipeline(std::false_type{});
     else
       pipeline(std::true_type{});
-    // 32x32 accumulator layout: column = lane & 31, row(v) = (v / 4) * 8 + (lane / 32) * 4 + v % 4.
-    if constexpr (MODE == 1) {
-      // phase-2 epilogue, straight from the accumulators: for each pair of rows (v, v + 1) a
-      // lane rounds both of its column's values at once (v_cvt_pk_bf16_f32), applies the rows'
-      // routing weights and rounds again into one packed word (row v low, row v + 1 high),
-      // swaps that word with its neighbour lane (DPP quad_perm [1,0,3,2]) and picks two adjacent
-      // columns of one row with one byte permute -- the even lane row v (its own low half, the
-      // neighbour's low half), the odd lane row v + 1 (the neighbour's high half, its own high
-      // half) -- stored as 4 bytes.  This is the issue-bound part of a phase-2 tile (all eight
-      // wavefronts run it at once), so each row pair costs one address and about nine VALU
-      // instructions per 32-column block.  No LDS staging and no barrier before the stores;
-      // the barrier after them keeps the row table until every wavefront has read it.
-      const bool odd = lane & 1;
-      const uint32_t pick = odd ? 0x03020706u : 0x05040100u;
-      char* const obase = reinterpret_cast<char*>(a.out) +
-                          ((int64_t)ntile * BN + wn * 64 + (l32 & ~1)) * 2;
+    // 16x16 accumulator layout (first operand: weight rows): column = token row lane & 15, rows
+    // (lane >> 4) * 4 + q.  The weight rows of tiles c = 0, 1 interleave in groups of four (see
+    // b_addr), so a lane holds 8 consecutive output columns of one token row: one 16-byte store.
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
+        const int r = 128 * h + 32 * i + 16 * wm + j16;
+        if constexpr (MODE == 0) {
+          u32x4 y;
 #pragma unroll
-        for (int vp = 0; vp < 8; ++vp) {
-          const int v0 = 2 * vp;
-          const int r0 = wm * 128 + i * 32 + (v0 >> 2) * 8 + (lane >> 5) * 4 + (v0 & 3);  // even
-          const float w0 = wt_s[r0], w1 = wt_s[r0 + 1];
-          const int r = odd ? r0 + 1 : r0;
-          char* const rowp = obase + orow_s[r];
-          const bool ok = m0 + r < n;
+          for (int c = 0; c < 2; ++c)
 #pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            const uint32_t g = pk_bf16(acc[i][j][v0], acc[i][j][v0 + 1]);
-            const uint32_t y = pk_bf16(__uint_as_float(g << 16) * w0,
-                                       __uint_as_float(g & 0xffff0000u) * w1);
-            const uint32_t yn =
-                (uint32_t)__builtin_amdgcn_update_dpp((int)y, (int)y, 0xB1, 0xf, 0xf, false);
-            if (ok)
-              *reinterpret_cast<uint32_t*>(rowp + j * 64) = __builtin_amdgcn_perm(yn, y, pick);
+            for (int q = 0; q < 4; q += 2) {
+              const floatx4& g = acc[h][0][i][c];
+              const floatx4& u = acc[h][1][i][c];
+              const uint32_t gp = pk_bf16(g[q], g[q + 1]), up = pk_bf16(u[q], u[q + 1]);
+              const float s0 = silu_mul(__uint_as_float(gp << 16), __uint_as_float(up << 16));
+              const float s1 = silu_mul(__uint_as_float(gp & 0xffff0000u), __uint_as_float(up & 0xffff0000u));
+              y[2 * c + q / 2] = pk_bf16(s0, s1);
+            }
+          if (r < vrows)
+            *reinterpret_cast<u32x4*>(&a.act[(start + m0 + r) * a.I + ntile * 128 + wn * 32 + 8 * g4]) = y;
+        } else {
+          const float wt = wt_s[r];
+          bf16_t* const o = a.out + orow_s[r] + ntile * BN + wn * 32 + 8 * g4;
+#pragma unroll
+          for (int hb = 0; hb < 2; ++hb) {
+            u32x4 y;
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+#pragma unroll
+              for (int q = 0; q < 4; q += 2) {
+                const uint32_t v = pk_bf16(acc[h][hb][i][c][q], acc[h][hb][i][c][q + 1]);
+                y[2 * c + q / 2] = pk_bf16(__uint_as_float(v << 16) * wt,
+                                           __uint_as_float(v & 0xffff0000u) * wt);
+              }
+            if (r < vrows) *reinterpret_cast<u32x4*>(o + 128 * hb) = y;
           }
         }
       }
+    // the row table is free again once every wavefront has read it (the stores stay in flight)
+    if (MODE == 1) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       wg_barrier();
-      continue;
     }
-    __syncthreads();  // all fragment reads done before the staging area is reused
-
-    // phase-1 epilogue: act[p, i0 + c] = bf16(silu(bf16 g) * bf16 u), the bf16 tile staged in
-    // LDS (128 columns), then 16-byte row stores.  g and u are rounded by one packed
-    // conversion; the results of rows (v, v + 1) of a column are packed likewise, swapped with
-    // the neighbour lane and byte-permuted into two adjacent columns of one row (as in the
-    // phase-2 epilogue), so that each LDS write carries two outputs.
-    constexpr int OC = 128, OLD = OC + 8, CPR = OC / 8;   // CPR: 16-byte chunks per row
-    bf16_t* os = smem;
-    const bool odd = lane & 1;
-    const uint32_t pick = odd ? 0x03020706u : 0x05040100u;
-    const int col = wn * 32 + (l32 & ~1);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-#pragma unroll
-      for (int vp = 0; vp < 8; ++vp) {
-        const int v0 = 2 * vp;
-        const int r0 = wm * 128 + i * 32 + (v0 >> 2) * 8 + (lane >> 5) * 4 + (v0 & 3);  // even
-        const uint32_t gu0 = pk_bf16(acc[i][0][v0], acc[i][1][v0]);
-        const uint32_t gu1 = pk_bf16(acc[i][0][v0 + 1], acc[i][1][v0 + 1]);
-        const float s0 = silu_mul(__uint_as_float(gu0 << 16), __uint_as_float(gu0 & 0xffff0000u));
-        const float s1 = silu_mul(__uint_as_float(gu1 << 16), __uint_as_float(gu1 & 0xffff0000u));
-        const uint32_t y = pk_bf16(s0, s1);
-        const uint32_t yn =
-            (uint32_t)__builtin_amdgcn_update_dpp((int)y, (int)y, 0xB1, 0xf, 0xf, false);
-        const int r = odd ? r0 + 1 : r0;
-        *reinterpret_cast<uint32_t*>(&os[r * OLD + col]) = __builtin_amdgcn_perm(yn, y, pick);
-      }
-    }
-    __syncthreads();
-    for (int c = tid; c < BM * CPR; c += kTiledThreads) {
-      const int r = c / CPR, cc = (c % CPR) * 8;
-      if (m0 + r >= n) continue;
-      const u32x4 v = *reinterpret_cast<const u32x4*>(&os[r * OLD + cc]);
-      *reinterpret_cast<u32x4*>(&a.act[(start + m0 + r) * a.I + ntile * 128 + cc]) = v;
-    }
-    // the staging reads are complete (their values are in the stores); the stores stay in
-    // flight across the barrier (__syncthreads would wait for them)
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    wg_barrier();
   }
 }
 

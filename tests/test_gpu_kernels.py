@@ -376,6 +376,50 @@ def test_small_expert_kernels_vs_oracle(device, H, I, counts, split):
                                    msg=lambda m: f'expert {e} ({c} rows): {m}')
 
 
+@pytest.mark.parametrize('H,I,counts', [
+    # K of 2 and 4 stages; rows around the 16-, 128- and 256-row edges of a tile
+    (256, 128, [65, 127, 128, 129, 144, 241, 255, 256, 257, 513]),
+    # K of 6 (down) and 8 (up) stages, several column tiles
+    (512, 384, [66, 80, 200, 300, 385]),
+])
+@pytest.mark.parametrize('out_mode', [0, 1])
+def test_tiled_kernels_edges(device, H, I, counts, out_mode):
+    """Experts of more than 64 rows at the edges of the tiled kernels' 256-row tiles, into an
+    output that starts one element past an aligned address; rows of an unlisted expert stay as
+    they were.  Tolerance: the bf16 roundings of y and of y * w (2^-8 each) and of the rows the
+    down projection sums (gate, up, activation), as in the tests above."""
+    ops = _ops()
+    E = len(counts)
+    rows_w = _pool(E, H, I, seed=H + E)
+    g = torch.Generator().manual_seed(E)
+    ids = np.concatenate([np.full(c, e, np.int64) for e, c in enumerate(counts)])
+    ids = ids[np.random.default_rng(E).permutation(len(ids))]
+    T = len(ids)
+    sel = torch.from_numpy(ids).view(T, 1)
+    w = (torch.rand((T, 1), generator=g) + 0.5).to(torch.bfloat16)
+    x = torch.randn((T, H), generator=g).to(torch.bfloat16)
+    lay = ops.layout(sel.to(device), w.to(device), E)
+    act = torch.empty((T, I), dtype=torch.bfloat16, device=device)
+    flat = torch.full((T * H + 1,), float('nan'), dtype=torch.bfloat16, device=device)
+    out = flat[1:].view(T, H)
+    listed = np.arange(E - 1)
+    ops.expert_ffn(rows_w.to(device), x.to(device), lay.w_sorted, lay.starts, lay.rows, lay.cols,
+                   listed, np.arange(E, dtype=np.int32), H, I, act, out, out_mode=out_mode,
+                   max_rows=max(counts), counts=counts, experts=E)
+    torch.cuda.synchronize()
+    got, starts = out.cpu().float(), np.concatenate([[0], np.cumsum(counts)])
+    for e, c in enumerate(counts):
+        r = torch.from_numpy(np.nonzero(ids == e)[0])
+        mine = got[r] if out_mode == 0 else got[starts[e]:starts[e + 1]]
+        if e == E - 1:
+            assert torch.isnan(mine).all()
+            continue
+        ref = execute_experts_ref([rows_w[e]], x, w, [r], [torch.zeros(c, dtype=torch.long)], H, I)[0]
+        torch.testing.assert_close(mine, ref.float(), rtol=2e-2, atol=1e-2,
+                                   msg=lambda m: f'expert {e} ({c} rows): {m}')
+    assert torch.isnan(flat[0].cpu())
+
+
 def _list_rows_counts_400():
     # 400 experts: the small ones fill more than one launch's list of 256, and the 17-64-row
     # experts (issued first) outnumber it, so the split falls among them
