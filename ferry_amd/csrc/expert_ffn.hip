@@ -42,6 +42,7 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kListMax = 256;   // experts per launch (longer lists are split by the host)
@@ -1234,7 +1235,8 @@ struct TileTable {
   int32_t rows[kListMax];
 };
 
-// Wavefront 0 builds the cumulative M-tile counts of the big experts of the list.
+// Wavefront 0 builds the cumulative counts of M tiles of ROWS rows of the big experts of the list.
+template <int ROWS>
 __device__ void build_tile_table(const FfnArgs& a, TileTable& tt) {
   if (threadIdx.x < 64) {
     const int lane = threadIdx.x;
@@ -1248,7 +1250,7 @@ __device__ void build_tile_table(const FfnArgs& a, TileTable& tt) {
         const int e = a.list.expert[li];
         const int64_t s0 = a.starts[e];
         const int64_t n = a.starts[e + 1] - s0;
-        c = n > kSkinnyMax ? (int)((n + BM - 1) / BM) : 0;
+        c = n > kSkinnyMax ? (int)((n + ROWS - 1) / ROWS) : 0;
         tt.start[li] = s0;
         tt.rows[li] = (int32_t)n;
       }
@@ -1299,7 +1301,7 @@ __global__ __launch_bounds__(kTiledThreads) __attribute__((amdgpu_waves_per_eu(2
   __shared__ __attribute__((aligned(1024))) char smem[8 * kHalfBytes];
   __shared__ int64_t orow_s[BM];   // phase 2: element offset of each tile row's output row
   __shared__ float wt_s[BM];
-  build_tile_table(a, tt);
+  build_tile_table<BM>(a, tt);
   const int64_t K = MODE == 0 ? a.H : a.I;
   const int ntn = MODE == 0 ? (int)(a.I / 128) : (int)(a.H / BN);
   const int total = tt.total * ntn;
@@ -1559,6 +1561,248 @@ __global__ __launch_bounds__(kTiledThreads) __attribute__((amdgpu_waves_per_eu(2
   }
 }
 
+// Smaller tiles, for lists that leave CUs idle (or a nearly empty last round) with 256 x 256 ones
+// (choose_tile): TM = 16 WM MI rows by TN = 16 WN NI weight rows per workgroup of WM x WN
+// wavefronts, each with MI x NI 16 x 16 accumulators.  Such a launch is one or two rounds of tiles,
+// so a tile's latency is what counts: its stages (64 columns of K) stream through an LDS ring as
+// deep as 144 KiB allows (3 to 6 stages for the five shapes below), the loads of a stage spread
+// between the matrix instructions; a wavefront's fragments of the next 32 columns are read while
+// the current ones are multiplied.  The loads of one CU reach it at about 64 bytes a clock, which a
+// 64 x 64 tile needs for 256 clocks of 128 clocks of products a stage: below that size nothing is
+// gained.  Stage time at full occupancy, us (256 x 256: 1.3): 256 x 128 and 128 x 256 0.8,
+// 128 x 128 0.5, 64 x 128 0.38, 64 x 64 0.3.  128 x 128 with four wavefronts of 64 x 64 took 0.6
+// (a wavefront alone on its SIMD stalls on its loads' issue), with eight of 64 x 32 0.52.
+// Products, K order, operand layout in LDS and roundings are those of ffn_tiled, so the outputs
+// do not depend on the tile.
+
+// 4-byte global->LDS direct load of each lane (LDS byte address lds + 4 * lane), as dma16
+__device__ __forceinline__ void dma4(const char* sbase, uint32_t voff, uint32_t lds) {
+  asm volatile(
+      "s_mov_b32 m0, %2\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dword %0, %1"
+      :
+      : "v"(voff), "s"(sbase), "s"(lds)
+      : "memory", "m0");
+}
+// wait until at most y groups of LPS vector-memory operations are outstanding (y wave-uniform,
+// values above V count as V)
+template <int V, int LPS>
+__device__ __forceinline__ void wait_groups(int y) {
+  if constexpr (V == 0) {
+    wait_cnt<0>();
+  } else {
+    if (y >= V)
+      wait_cnt<V * LPS>();
+    else
+      wait_groups<V - 1, LPS>(y);
+  }
+}
+
+template <int MODE, int WM, int WN, int MI, int NI>
+__global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(WM * WN / 4, WM * WN / 4))) void ffn_tile(FfnArgs a) {
+  constexpr int W = WM * WN;
+  constexpr int TM = 16 * WM * MI, TN = 16 * WN * NI;    // tile rows and weight rows
+  constexpr int kStage = (TM + TN) * kRowBytes;
+  constexpr int SST = 147456 / kStage;                   // stages: 128 or 144 KiB
+  constexpr int LA = TM / (8 * W), LB = TN / (8 * W);    // direct loads per wavefront and stage
+  constexpr int LPS = LA + LB;
+  // phase 1 with one gate and one up tile per wavefront: weight rows in order (else interleaved)
+  constexpr bool INORD = MODE == 0 && NI == 2;
+  __shared__ TileTable tt;
+  __shared__ __attribute__((aligned(1024))) char smem[SST * kStage];
+  __shared__ __attribute__((aligned(256))) int32_t row_s[MODE == 1 ? TM : 1], col_s[MODE == 1 ? TM : 1];
+  __shared__ int32_t orow_s[MODE == 1 ? TM : 1];
+  __shared__ float wt_s[MODE == 1 ? TM : 1];
+  build_tile_table<TM>(a, tt);
+  const int64_t K = MODE == 0 ? a.H : a.I;
+  const int ntn = MODE == 0 ? (int)(a.I / (TN / 2)) : (int)(a.H / TN);
+  const int total = tt.total * ntn;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int KT = (int)(K / BK);   // at least 2
+  const int j16 = lane & 15, g4 = lane >> 4;
+  const uint32_t smem0 = lds_addr(smem);
+  auto swz_w = [](int row) { return INORD ? swz_a(row) : swz_b(row); };
+  // fragment reads: K step ks of A tile i (rows 32 i + 16 wm + j16) and of weight tile c.  Phase 1:
+  // gate columns (TN / 4) wn + ... for c < NI / 2, the same up columns for the others; phase 2:
+  // columns (TN / 2) wn + ...; pairs of tiles interleaved as in ffn_tiled
+  uint32_t a_addr[2], b_addr[2];
+  constexpr int kPair = (MODE == 0 ? TN / 2 : 32) * kRowBytes;   // from tiles c < NI / 2 to the others
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+    const int arow = 16 * wm + j16;
+    const int brow = INORD ? 16 * wn + j16 : 16 * (MODE == 0 ? NI / 2 : NI) * wn + 8 * (j16 >> 2) + (j16 & 3);
+    a_addr[ks] = (uint32_t)(arow * kRowBytes + (((4 * ks + g4) ^ swz_a(arow)) << 4));
+    b_addr[ks] = (uint32_t)((TM + brow) * kRowBytes + (((4 * ks + g4) ^ swz_w(brow)) << 4));
+  }
+  const int per_xcd = gridDim.x % 8 == 0 ? (int)gridDim.x / 8 : 0;
+  const int lslot = per_xcd ? (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8) : (int)blockIdx.x;
+  for (int tile = lslot; tile < total; tile += gridDim.x) {
+    const int mt_global = tile / ntn, ntile = tile % ntn;
+    const int li = find_entry(tt, mt_global);
+    const int64_t start = tt.start[li];
+    const int n = tt.rows[li];
+    const int m0 = (mt_global - tt.cum[li]) * TM;
+    const int vrows = n - m0;   // > 0
+    const bf16_t* slot = a.cache + (int64_t)a.list.slot[li] * 3 * a.H * a.I;
+    // direct loads: this wavefront moves A rows 8 MI wave + 8 q + lane / 8 (q < MI) and weight rows
+    // 8 NI wave + 8 q + lane / 8 (q < NI)
+    const int r8 = lane >> 3, slot8 = lane & 7;
+    uint32_t aoff[LA], boff[LB];
+    const char* abase = reinterpret_cast<const char*>(MODE == 0 ? a.x : a.act);
+    const uint32_t lda = (uint32_t)K;
+#pragma unroll
+    for (int q = 0; q < LA; ++q) {
+      const int row = 8 * LA * wave + 8 * q + r8;
+      const int r = m0 + row;
+      const bool ok = r < n;
+      const uint32_t t = MODE == 0 ? (uint32_t)a.rows[start + (ok ? r : 0)]
+                                   : (uint32_t)(start + (ok ? r : 0));
+      aoff[q] = (t * lda + (uint32_t)((slot8 ^ swz_a(row)) * 8)) * 2u;
+    }
+#pragma unroll
+    for (int q = 0; q < LB; ++q) {
+      const int row = 8 * LB * wave + 8 * q + r8;
+      boff[q] = (uint32_t)(((uint32_t)(8 * q + r8) * (uint32_t)K + (uint32_t)((slot8 ^ swz_w(row)) * 8)) * 2u);
+    }
+    // phase 1: the first TN / 2 weight rows are gate, the others up columns (TN / 2) ntile + ...
+    const int brow0 = 8 * LB * wave;
+    const char* bbase = reinterpret_cast<const char*>(uniform_ptr(
+        MODE == 0 ? slot + (brow0 < TN / 2 ? (int64_t)(ntile * (TN / 2) + brow0) * a.H
+                                           : a.H * a.I + (int64_t)(ntile * (TN / 2) + brow0 - TN / 2) * a.H)
+                  : slot + 2 * a.H * a.I + (int64_t)(ntile * TN + brow0) * a.I));
+    if (MODE == 1 && 64 * wave < TM) {
+      // the tile rows' token and slot indices (low words) of rows 64 wave + lane: the oldest loads
+      // of the tile, so they have landed when the first stage has
+      const int r = 64 * wave + lane;
+      const int64_t p = start + m0;
+      const uint32_t off = (uint32_t)((r < vrows ? r : 0) * 8);
+      dma4(reinterpret_cast<const char*>(uniform_ptr(a.rows + p)), off, lds_addr(row_s) + 256 * wave);
+      dma4(reinterpret_cast<const char*>(uniform_ptr(a.cols + p)), off, lds_addr(col_s) + 256 * wave);
+    }
+    floatx4 acc[MI][NI];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int c = 0; c < NI; ++c) acc[i][c] = floatx4{0, 0, 0, 0};
+    // 16-row tiles of this wavefront that hold rows of the expert
+    const int v = vrows - 16 * wm;
+    const int nf = __builtin_amdgcn_readfirstlane(v <= 0 ? 0 : ((v + 16 * WM - 1) / (16 * WM) < MI ? (v + 16 * WM - 1) / (16 * WM) : MI));
+    auto dma = [&](int kt, int sl, auto qq) {   // load q of stage kt into slot sl: A rows for q < MI
+      constexpr int q = decltype(qq)::value;
+      const uint32_t dst = smem0 + (uint32_t)(sl * kStage);
+      if constexpr (q < LA)
+        dma16(abase + kt * BK * 2, aoff[q], dst + (uint32_t)((8 * LA * wave + 8 * q) * kRowBytes));
+      else
+        dma16(bbase + kt * BK * 2, boff[q - LA], dst + (uint32_t)((TM + 8 * LB * wave + 8 * (q - LA)) * kRowBytes));
+    };
+    auto read = [&](int sl, int ks, bf16x8 (&ft)[MI], bf16x8 (&fw)[NI]) {
+      const char* st = smem + sl * kStage;
+#pragma unroll
+      for (int c = 0; c < NI; ++c)
+        fw[c] = *reinterpret_cast<const bf16x8*>(
+            st + b_addr[ks] + (INORD ? c * kPair : (c >> 1) * kPair + (c & 1) * 4 * kRowBytes));
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+        ft[i] = *reinterpret_cast<const bf16x8*>(st + a_addr[ks] + i * 16 * WM * kRowBytes);
+    };
+    auto mma = [&](int i, const bf16x8 (&ft)[MI], const bf16x8 (&fw)[NI]) {
+      if (i < nf) {
+#pragma unroll
+        for (int c = 0; c < NI; ++c)
+          acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[c], ft[i], acc[i][c], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    bf16x8 t0[MI], w0[NI], t1[MI], w1[NI];
+    for (int k = 0; k < (SST < KT ? SST : KT); ++k)
+      static_for<0, LPS>([&](auto q) { dma(k, k, q); });
+    wait_groups<SST - 1, LPS>(KT - 1);
+    wg_barrier();
+    // phase 2: the output row and routing weight of row tid, loaded under the K loop
+    int32_t my_orow = 0;
+    float my_wt = 0.f;
+    if (MODE == 1 && tid < TM) {
+      const int64_t tj = (int64_t)row_s[tid] * a.k + col_s[tid];
+      my_wt = bf16_to_f32(a.w[tj]);
+      my_orow = a.out_mode == 0 ? (int32_t)tj : (int32_t)(start + m0 + tid);
+    }
+    read(0, 0, t0, w0);
+    int cur = 0;   // slot of stage k
+    for (int k = 0; k < KT; ++k) {
+      const int nxt = cur + 1 == SST ? 0 : cur + 1;
+      read(cur, 1, t1, w1);
+#pragma unroll
+      for (int i = 0; i < MI; ++i) mma(i, t0, w0);
+      // stage k is read by this wavefront, its loads of stage k + 1 have landed
+      wait_groups<SST - 2, LPS>(KT - 2 - k);
+      wg_barrier();
+      if (k + 1 < KT) read(nxt, 0, t0, w0);
+      const bool more = k + SST < KT;
+      static_for<0, MI>([&](auto ii) {
+        constexpr int i = decltype(ii)::value;
+        if (more)   // a share of the loads into the buffer of stage k
+          static_for<i * LPS / MI, (i + 1) * LPS / MI>([&](auto q) { dma(k + SST, cur, q); });
+        mma(i, t1, w1);
+      });
+      cur = nxt;
+    }
+    if (MODE == 1) {
+      if (tid < TM) {
+        orow_s[tid] = my_orow;
+        wt_s[tid] = my_wt;
+      }
+      __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      const int r = 16 * WM * i + 16 * wm + j16;
+      if constexpr (MODE == 0) {
+        uint32_t y[NI];
+#pragma unroll
+        for (int c = 0; c < NI / 2; ++c)
+#pragma unroll
+          for (int q = 0; q < 4; q += 2) {
+            const uint32_t gp = pk_bf16(acc[i][c][q], acc[i][c][q + 1]);
+            const uint32_t up = pk_bf16(acc[i][NI / 2 + c][q], acc[i][NI / 2 + c][q + 1]);
+            const float s0 = silu_mul(__uint_as_float(gp << 16), __uint_as_float(up << 16));
+            const float s1 = silu_mul(__uint_as_float(gp & 0xffff0000u), __uint_as_float(up & 0xffff0000u));
+            y[2 * c + q / 2] = pk_bf16(s0, s1);
+          }
+        bf16_t* const o = a.act + (start + m0 + r) * a.I + ntile * (TN / 2) + wn * (8 * NI) + 2 * NI * g4;
+        if (r < vrows) {
+          if constexpr (NI == 4)
+            *reinterpret_cast<u32x4*>(o) = u32x4{y[0], y[1], y[2], y[3]};
+          else
+            *reinterpret_cast<u32x2*>(o) = u32x2{y[0], y[1]};
+        }
+      } else {
+        const float wt = wt_s[r];
+        bf16_t* const o = a.out + (int64_t)orow_s[r] * a.H + ntile * TN + wn * (16 * NI) + 8 * g4;
+#pragma unroll
+        for (int hb = 0; hb < NI / 2; ++hb) {
+          u32x4 y;
+#pragma unroll
+          for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int q = 0; q < 4; q += 2) {
+              const uint32_t v2 = pk_bf16(acc[i][2 * hb + c][q], acc[i][2 * hb + c][q + 1]);
+              y[2 * c + q / 2] = pk_bf16(__uint_as_float(v2 << 16) * wt,
+                                         __uint_as_float(v2 & 0xffff0000u) * wt);
+            }
+          if (r < vrows) *reinterpret_cast<u32x4*>(o + 32 * hb) = y;
+        }
+      }
+    }
+    if (MODE == 1) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      wg_barrier();
+    }
+  }
+}
+
 int g_num_cus = 0;
 
 // Device addresses of g_sync / g_sync_timeouts on each device (resolved on first use there).
@@ -1600,10 +1844,15 @@ int ffn_timeouts_address(int32_t** timeouts) {
 
 using namespace ferry;
 
+// M tiles of a list's experts with more than 64 rows, for tiles of 64 << i rows (0: row counts
+// unknown)
+struct MTiles {
+  int64_t n[3] = {0, 0, 0};
+};
 static int ffn_launch_list(FfnArgs& args, const int32_t* expert_list, const int32_t* slot_of,
                            int32_t n_list, int32_t n_mid, int64_t maxn, int64_t min_rows,
-                           int64_t pairs, int32_t phases, int64_t hidden, int64_t inter,
-                           hipStream_t s);
+                           int64_t pairs, const MTiles& mt, int32_t phases, int64_t hidden,
+                           int64_t inter, hipStream_t s);
 
 extern "C" int ferry_expert_ffn(const void* cache, int64_t cache_rows, int64_t hidden,
                                 int64_t inter, const void* x, int64_t rows_in, int64_t topk,
@@ -1679,9 +1928,10 @@ extern "C" int ferry_expert_ffn(const void* cache, int64_t cache_rows, int64_t h
   // without rows are left out.
   if (!list_rows)
     return ffn_launch_list(args, expert_list, slot_of, n_list, n_list, max_rows_per_expert,
-                           min_rows_per_expert, rows_in * topk, phases, hidden, inter, s);
+                           min_rows_per_expert, rows_in * topk, MTiles{}, phases, hidden, inter, s);
   std::vector<int32_t> small, big;
   int32_t n_mid = 0;
+  MTiles mt;
   int64_t small_max = 0, small_min = kSkinnyMax, big_max = 0, big_min = INT64_MAX;
   for (int pass = 0; pass < 2; ++pass)   // 17-64 rows, then 1-16 rows
     for (int32_t i = 0; i < n_list; ++i) {
@@ -1696,16 +1946,75 @@ extern "C" int ferry_expert_ffn(const void* cache, int64_t cache_rows, int64_t h
         big.push_back(expert_list[i]);
         big_max = r > big_max ? r : big_max;
         big_min = r < big_min ? r : big_min;
+        for (int i = 0; i < 3; ++i) mt.n[i] += ceil_div(r, 64 << i);
       }
     }
   if (!small.empty()) {
     const int rc = ffn_launch_list(args, small.data(), slot_of, (int32_t)small.size(), n_mid,
-                                   small_max, small_min, rows_in * topk, phases, hidden, inter, s);
+                                   small_max, small_min, rows_in * topk, MTiles{}, phases, hidden,
+                                   inter, s);
     if (rc != 0) return rc;
   }
   if (!big.empty())
     return ffn_launch_list(args, big.data(), slot_of, (int32_t)big.size(), 0, big_max, big_min,
-                           rows_in * topk, phases, hidden, inter, s);
+                           rows_in * topk, mt, phases, hidden, inter, s);
+  return 0;
+}
+
+// Which tile a list's tiled experts take: the one whose rounds of one tile per CU cost least.  A
+// tile costs kt stages of K plus a fixed part (tile table, row indices, first loads, epilogue); the
+// figures are fitted to 2 x 67 launches (1-64 experts of 65-4096 rows, H x I = 2048 x 768 / 1408 /
+// 2816), over which the choice costs 0.8 % more than the best tile on average, 16 % at worst (64
+// experts of 65 rows, 1.5 rounds).  A small tile has less latency, a large one less traffic per
+// product; so a list that leaves CUs idle with large tiles takes smaller ones.  us, 256 x 256 ->
+// chosen: shared expert (2048 x 2816) of 256 rows 39.9 -> 18.3 up, 47.4 -> 18.7 down, of 777 rows
+// 50.6 -> 33.0 and 52.3 -> 22.0; 8 experts (2048 x 1408) of 128 rows 39.5 -> 26.0 and 28.5 -> 15.4;
+// 24 experts (2048 x 768) of 100 rows 46.0 -> 41.9.  No choice beats reading the list's weights at
+// 4.5 TB/s, and the 256 x 256 tile is preferred by 5 % (its loop is the better one when full).
+// Lists without row counts take 256 x 256 tiles.
+struct TileCost {
+  int rows_log, cols;    // 64 << rows_log rows, weight rows
+  double stage, fixed;   // us
+};
+static const TileCost kTiles[] = {{2, 256, 1.3, 7.0}, {2, 128, 0.8, 6.0}, {1, 256, 0.8, 6.0},
+                                  {1, 128, 0.5, 5.0}, {0, 128, 0.38, 4.0}, {0, 64, 0.3, 3.5}};
+static int choose_tile(const MTiles& mt, int64_t experts, int64_t cols, int64_t k, int64_t cus) {
+  const double read = (double)(experts * cols * k * 2) / 4.5e6 + 1.0;
+  int best = 0;
+  double least = 0;
+  for (int i = 0; i < 6; ++i) {
+    const int64_t tiles = mt.n[kTiles[i].rows_log] * (cols / kTiles[i].cols);
+    const double t = (double)ceil_div(tiles, cus) * ((double)(k / BK) * kTiles[i].stage + kTiles[i].fixed);
+    const double cost = (t > read ? t : read) * (i == 0 ? 0.95 : 1.0);
+    if (i == 0 || cost < least) best = i, least = cost;
+  }
+  return best;
+}
+
+// The tiled experts of a list, one phase (MODE 0: up, 1: down).
+template <int MODE>
+static int tiled_launch(const FfnArgs& args, const MTiles& mt, int64_t pairs, int64_t cus, hipStream_t s) {
+  const char* name = MODE == 0 ? "ffn_tiled_up" : "ffn_tiled_down";
+  const int64_t cols = MODE == 0 ? 2 * args.I : args.H;   // weight rows of an expert
+  const int c = mt.n[0] == 0 ? 0 : choose_tile(mt, args.list.n, cols, MODE == 0 ? args.H : args.I, cus);
+  auto go = [&](auto kernel, int threads, int64_t tiles) {
+    launch(name, kernel, dim3((unsigned)(tiles < cus ? tiles : cus)), dim3(threads), 0, s, args);
+  };
+  const int64_t tiles = mt.n[kTiles[c].rows_log] * (cols / kTiles[c].cols);
+  switch (c) {
+    case 0:
+      // M tiles over experts with > 64 rows when the row counts are unknown:
+      // sum ceil(n/BM) <= pairs/BM + (experts with > 64 rows), and those are <= pairs/65
+      go(ffn_tiled<MODE>, kTiledThreads,
+         mt.n[0] ? tiles : (pairs / BM + pairs / (kSkinnyMax + 1) + 1) * (cols / BN));
+      break;
+    case 1: go(ffn_tile<MODE, 4, 2, 4, 4>, 512, tiles); break;
+    case 2: go(ffn_tile<MODE, 2, 4, 4, 4>, 512, tiles); break;
+    case 3: go(ffn_tile<MODE, 4, 2, 2, 4>, 512, tiles); break;
+    case 4: go(ffn_tile<MODE, 2, 4, 2, 2>, 512, tiles); break;
+    default: go(ffn_tile<MODE, 2, 2, 2, 2>, 256, tiles);
+  }
+  FERRY_LAUNCHED(name);
   return 0;
 }
 
@@ -1714,8 +2023,8 @@ extern "C" int ferry_expert_ffn(const void* cache, int64_t cache_rows, int64_t h
 // the bounds allow no expert of more than 16 rows, n_mid = n_list when unknown).
 static int ffn_launch_list(FfnArgs& args, const int32_t* expert_list, const int32_t* slot_of,
                            int32_t n_list, int32_t n_mid, int64_t maxn, int64_t min_rows,
-                           int64_t pairs, int32_t phases, int64_t hidden, int64_t inter,
-                           hipStream_t s) {
+                           int64_t pairs, const MTiles& mt, int32_t phases, int64_t hidden,
+                           int64_t inter, hipStream_t s) {
   const bool any_small = min_rows <= kSkinnyMax;
   for (int32_t off = 0; off < n_list; off += kListMax) {
     const int32_t cnt = (n_list - off) < kListMax ? (n_list - off) : kListMax;
@@ -1727,9 +2036,7 @@ static int ffn_launch_list(FfnArgs& args, const int32_t* expert_list, const int3
       args.list.slot[i] = i < cnt ? slot_of[expert_list[off + i]] : 0;
     }
     const bool any_big = maxn > kSkinnyMax;
-    // M tiles over experts with > 64 rows: sum ceil(n/BM) <= pairs/BM + (experts with > 64 rows)
-    const int64_t tile_bound = pairs / BM + pairs / (kSkinnyMax + 1) + 1;  // and those are <= pairs/65
-    const int64_t grid_cap = (int64_t)g_num_cus;  // one 256x256 workgroup per CU
+    const int64_t grid_cap = (int64_t)g_num_cus;  // one tiled workgroup per CU
     if (phases == 3 && any_small && !any_big && maxn <= 16 && inter / 16 <= kMaxUpWgs) {
       // decode: both phases in one launch, each expert's down projection as soon as its up
       // projection is stored
@@ -1761,10 +2068,8 @@ static int ffn_launch_list(FfnArgs& args, const int32_t* expert_list, const int3
         FERRY_LAUNCHED("ffn_up_skinny");
       }
       if (any_big) {
-        const int64_t t1 = tile_bound * (inter / 128);
-        launch("ffn_tiled_up", ffn_tiled<0>, dim3((unsigned)(t1 < grid_cap ? t1 : grid_cap)),
-                           dim3(kTiledThreads), 0, s, args);
-        FERRY_LAUNCHED("ffn_tiled<up>");
+        const int rc = tiled_launch<0>(args, mt, pairs, grid_cap, s);
+        if (rc != 0) return rc;
       }
     }
     if (phases & 2) {
@@ -1778,10 +2083,8 @@ static int ffn_launch_list(FfnArgs& args, const int32_t* expert_list, const int3
         FERRY_LAUNCHED("ffn_down_skinny");
       }
       if (any_big) {
-        const int64_t t2 = tile_bound * (hidden / BN);
-        launch("ffn_tiled_down", ffn_tiled<1>, dim3((unsigned)(t2 < grid_cap ? t2 : grid_cap)),
-                           dim3(kTiledThreads), 0, s, args);
-        FERRY_LAUNCHED("ffn_tiled<down>");
+        const int rc = tiled_launch<1>(args, mt, pairs, grid_cap, s);
+        if (rc != 0) return rc;
       }
     }
   }

@@ -420,6 +420,35 @@ def test_tiled_kernels_edges(device, H, I, counts, out_mode):
     assert torch.isnan(flat[0].cpu())
 
 
+@pytest.mark.parametrize('E,n', [(1, 65), (5, 257), (20, 65), (40, 65), (60, 65), (80, 65), (40, 129),
+                                 (30, 257), (80, 129)])
+def test_tiled_kernels_tile_shapes_bit_identical(device, E, n):
+    """Given the row counts, a list's tiled experts take the tile that suits their number: these
+    lists of n to n + 15 rows reach all six, in both phases (on 256 CUs).  Each sums the same
+    products in the same order: the bits of the call without counts (256 x 256 tiles)."""
+    ops = _ops()
+    H, I = 512, 384
+    counts = [n + (7 * e) % 16 for e in range(E)]
+    cache = _pool(E, H, I, seed=E + n).to(device)
+    g = torch.Generator().manual_seed(E)
+    ids = np.concatenate([np.full(c, e, np.int64) for e, c in enumerate(counts)])
+    ids = ids[np.random.default_rng(E).permutation(len(ids))]
+    T = len(ids)
+    w = (torch.rand((T, 1), generator=g) + 0.5).to(torch.bfloat16).to(device)
+    x = torch.randn((T, H), generator=g).to(torch.bfloat16).to(device)
+    lay = ops.layout(torch.from_numpy(ids).view(T, 1).to(device), w, E)
+    outs = []
+    for c in (None, counts):
+        act = torch.full((T, I), float('nan'), dtype=torch.bfloat16, device=device)
+        part = torch.full((T, H), float('nan'), dtype=torch.bfloat16, device=device)
+        ops.expert_ffn(cache, x, lay.w_sorted, lay.starts, lay.rows, lay.cols, np.arange(E),
+                       np.arange(E, dtype=np.int32), H, I, act, part, max_rows=T, counts=c)
+        outs.append((act.cpu(), part.cpu()))
+    assert not torch.isnan(outs[0][1].float()).any()
+    for a, b in zip(*outs):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
 def _list_rows_counts_400():
     # 400 experts: the small ones fill more than one launch's list of 256, and the 17-64-row
     # experts (issued first) outnumber it, so the split falls among them
