@@ -117,13 +117,15 @@ __device__ __forceinline__ bf16x8 load_act8(const bf16_t* p) {
 // Memory helpers shared by the kernels below
 // =============================================================================================
 
-// a wave-uniform pointer moved to scalar registers
+// a wave-uniform value / pointer moved to scalar registers
+__device__ __forceinline__ int64_t uniform64(int64_t v) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)v >> 32));
+  return (int64_t)(((uint64_t)hi << 32) | lo);
+}
 template <typename T>
 __device__ __forceinline__ const T* uniform_ptr(const T* p) {
-  const uint64_t v = (uint64_t)(uintptr_t)p;
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
-  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-  return (const T*)(uintptr_t)(((uint64_t)hi << 32) | lo);
+  return (const T*)(uintptr_t)uniform64((int64_t)(uintptr_t)p);
 }
 // 16-byte global->LDS direct load of each lane: global address sbase + voff (wave-uniform base
 // in scalar registers, 32-bit lane byte offset), LDS byte address lds + 16 * lane.  Issued as
@@ -145,6 +147,30 @@ __device__ __forceinline__ void dma16(const char* sbase, uint32_t voff, uint32_t
 typedef __attribute__((address_space(3))) char lds_char;
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return (uint32_t)(uintptr_t)(lds_char*)p;
+}
+// 4-byte global->LDS direct load of each lane (LDS byte address lds + 4 * lane), as dma16
+__device__ __forceinline__ void dma4(const char* sbase, uint32_t voff, uint32_t lds) {
+  asm volatile(
+      "s_mov_b32 m0, %2\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dword %0, %1"
+      :
+      : "v"(voff), "s"(sbase), "s"(lds)
+      : "memory", "m0");
+}
+// 2-byte load of each lane, zero-extended to 4 bytes in LDS (address lds + 4 * lane)
+__device__ __forceinline__ void dma2(const char* sbase, uint32_t voff, uint32_t lds) {
+  asm volatile(
+      "s_mov_b32 m0, %2\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_ushort %0, %1"
+      :
+      : "v"(voff), "s"(sbase), "s"(lds)
+      : "memory", "m0");
+}
+// 16 bytes at LDS byte address addr (constant parts of it go into the instruction's offset)
+__device__ __forceinline__ bf16x8 lds_read16(uint32_t addr) {
+  return *reinterpret_cast<__attribute__((address_space(3))) const bf16x8*>((uintptr_t)addr);
 }
 // wait until at most VM vector-memory operations (the direct loads among them) and no LDS reads
 // of this wavefront are outstanding, in a form whose LDS part the compiler knows of
@@ -1205,9 +1231,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void f
 // flight.  A wavefront issues two loads a phase, so "at most 12 outstanding" before the barrier
 // says that its share of the half read next has landed; nothing in the loop waits for all loads.
 // Before this schedule (one barrier and a full drain of the loads per stage, both wavefronts of a
-// SIMD waiting together) a stage took 1.7 us of the 1.31 us it takes now.  One dense expert of
-// 65,536 rows, H x I = 2048 x 768: up 352 -> 300 us (1173 -> 1372 TFLOP/s), down 233 -> 209 us
-// (883 -> 986); 2048 x 1408: up 1177 -> 1390, down 1048 -> 1208; 2048 x 4096 down 1240 -> 1467.
+// SIMD waiting together) a stage took 1.7 us, now 1.31.  One dense expert of
+// 65,536 rows, H x I = 2048 x 768: up 352 -> 299 us (1173 -> 1380 TFLOP/s), down 233 -> 197 us
+// (883 -> 1049); 2048 x 1408: up 1177 -> 1411, down 1048 -> 1232; 2048 x 4096 down 1240 -> 1488.  Of
+// that, running on across tiles gives 2 % (up) and 2-6 % (down); each tile still spends about 6.5 us
+// outside its stages, most of it the SwiGLU of the up epilogue (two quarter-rate transcendentals for
+// each of a lane's 64 outputs).
 // The same products are summed in the same K order as before: results are bit-identical.
 //
 // Operand staging: global -> LDS direct loads (global_load_lds_dwordx4, no VGPR round trip).  One
@@ -1229,7 +1258,7 @@ __device__ __forceinline__ int swz_a(int row) { return (row >> 1) & 7; }
 __device__ __forceinline__ int swz_b(int row) { return ((row >> 1) & 1) | (((row >> 3) & 3) << 1); }
 
 struct TileTable {
-  int32_t cum[kListMax + 1];  // cumulative M tiles over list entries
+  __attribute__((aligned(16))) int32_t cum[kListMax + 1];  // cumulative M tiles over list entries
   int32_t total;
   int64_t start[kListMax];    // per list entry: its expert's first grouped row, and row count
   int32_t rows[kListMax];
@@ -1277,17 +1306,14 @@ __device__ void build_tile_table(const FfnArgs& a, TileTable& tt) {
   __syncthreads();
 }
 
-// largest li with cum[li] <= m (cum is non-decreasing)
+// largest li with cum[li] <= m (cum is non-decreasing), by a whole wavefront: the entries that hold
+// at most m, counted with ballots over four entries a lane
 __device__ __forceinline__ int find_entry(const TileTable& tt, int m) {
-  int lo = 0, hi = kListMax;  // cum[lo] <= m < cum[hi]
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (tt.cum[mid] <= m)
-      lo = mid;
-    else
-      hi = mid;
-  }
-  return lo;
+  const u32x4 c = *reinterpret_cast<const u32x4*>(&tt.cum[(threadIdx.x & 63) * 4]);
+  int le = 0;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) le += __popcll(__ballot((int)c[q] <= m));
+  return le - 1;
 }
 
 // MODE 0: A = gathered x rows (K = H); B half 0 = gate rows i0 .. +128, half 1 = the up rows of
@@ -1299,12 +1325,15 @@ template <int MODE>
 __global__ __launch_bounds__(kTiledThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void ffn_tiled(FfnArgs a) {
   __shared__ TileTable tt;
   __shared__ __attribute__((aligned(1024))) char smem[8 * kHalfBytes];
-  __shared__ int64_t orow_s[BM];   // phase 2: element offset of each tile row's output row
-  __shared__ float wt_s[BM];
+  // per tile row, two sets taken in turn: phase 1 the token (source row), phase 2 the token and
+  // slot index, and from them the output row and the routing weight (bf16 bits)
+  __shared__ __attribute__((aligned(256))) int32_t row_s[2][BM], col_s[MODE == 1 ? 2 : 1][MODE == 1 ? BM : 1];
+  __shared__ __attribute__((aligned(256))) int32_t orow_s[MODE == 1 ? 2 : 1][MODE == 1 ? BM : 1],
+      wt_s[MODE == 1 ? 2 : 1][MODE == 1 ? BM : 1];
   build_tile_table<BM>(a, tt);
   const int64_t K = MODE == 0 ? a.H : a.I;
   const int ntn = MODE == 0 ? (int)(a.I / 128) : (int)(a.H / BN);
-  const int total = tt.total * ntn;
+  const int total = __builtin_amdgcn_readfirstlane(tt.total) * ntn;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 2, wn = wave & 3;
@@ -1317,9 +1346,76 @@ __global__ __launch_bounds__(kTiledThreads) __attribute__((amdgpu_waves_per_eu(2
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks) {
     const int arow = 16 * wm + j16, brow = 32 * wn + 8 * (j16 >> 2) + (j16 & 3);
-    a_addr[ks] = (uint32_t)(arow * kRowBytes + (((4 * ks + g4) ^ swz_a(arow)) << 4));
-    b_addr[ks] = (uint32_t)(4 * kHalfBytes + brow * kRowBytes + (((4 * ks + g4) ^ swz_b(brow)) << 4));
+    a_addr[ks] = smem0 + (uint32_t)(arow * kRowBytes + (((4 * ks + g4) ^ swz_a(arow)) << 4));
+    b_addr[ks] = smem0 + (uint32_t)(4 * kHalfBytes + brow * kRowBytes + (((4 * ks + g4) ^ swz_b(brow)) << 4));
   }
+  // Direct loads: of each half this wavefront moves rows 16 wave + 8 q + lane / 8 (q < 2), lane
+  // slot lane % 8 holding the row's chunk (lane % 8) ^ swizzle(row).  Rows past the expert's last
+  // row load its first row instead: each output row depends only on its own A row, and those rows
+  // are never stored.
+  const int r8 = lane >> 3, slot8 = lane & 7;
+  uint32_t aoff[2][2], boff[2];   // byte offsets: < 2^32 (host-checked sizes)
+  const char* const abase = reinterpret_cast<const char*>(MODE == 0 ? a.x : a.act);
+#pragma unroll
+  for (int q = 0; q < 2; ++q)
+    boff[q] = ((uint32_t)(8 * q + r8) * (uint32_t)K + (uint32_t)((slot8 ^ swz_b(16 * wave + 8 * q + r8)) * 8)) * 2u;
+
+  const int64_t bhalf = MODE == 0 ? a.H * a.I * 2 : 128 * a.I * 2;   // bytes from B half 0 to half 1
+  struct Tile {
+    int64_t start;       // the expert's first grouped row
+    int m0, vrows, ntile;
+    const char* bbase;   // B half 0, rows 16 wave ...
+  };
+  auto locate = [&](int tile) {
+    Tile t;
+    const int mt_global = tile / ntn;
+    t.ntile = tile - mt_global * ntn;
+    const int li = __builtin_amdgcn_readfirstlane(find_entry(tt, mt_global));
+    t.start = uniform64(tt.start[li]);
+    t.m0 = (mt_global - __builtin_amdgcn_readfirstlane(tt.cum[li])) * BM;
+    t.vrows = __builtin_amdgcn_readfirstlane(tt.rows[li]) - t.m0;   // > 0
+    const bf16_t* slot = a.cache + (int64_t)a.list.slot[li] * 3 * a.H * a.I;
+    t.bbase = reinterpret_cast<const char*>(uniform_ptr(
+        MODE == 0 ? slot + (int64_t)(t.ntile * 128 + 16 * wave) * a.H
+                  : slot + 2 * a.H * a.I + (int64_t)(t.ntile * BN + 16 * wave) * a.I));
+    return t;
+  };
+  // the tile rows' indices (low words; rows past the last: the first row's) into set p, direct
+  // loads of the wavefronts 0 .. 3, 64 rows each
+  auto load_rows = [&](const Tile& t, int p) {
+    if (wave < 4) {
+      const int r = 64 * wave + lane;
+      const uint32_t off = (uint32_t)((r < t.vrows ? r : 0) * 8);
+      const int64_t at = t.start + t.m0;
+      dma4(reinterpret_cast<const char*>(uniform_ptr(a.rows + at)), off, lds_addr(row_s[p]) + 256 * wave);
+      if constexpr (MODE == 1)
+        dma4(reinterpret_cast<const char*>(uniform_ptr(a.cols + at)), off, lds_addr(col_s[p]) + 256 * wave);
+    }
+  };
+  auto dma_a = [&](int kt, int h, int s) {
+    const uint32_t dst = smem0 + (uint32_t)((2 * h + s) * kHalfBytes + 16 * wave * kRowBytes);
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      dma16(abase + kt * BK * 2, aoff[h][q], dst + (uint32_t)(8 * q * kRowBytes));
+  };
+  auto dma_b = [&](const char* b, int h, int s) {   // b: the stage's columns of B half 0
+    const uint32_t dst = smem0 + (uint32_t)((4 + 2 * h + s) * kHalfBytes + 16 * wave * kRowBytes);
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      dma16(b + (h ? bhalf : 0), boff[q], dst + (uint32_t)(8 * q * kRowBytes));
+  };
+  // A offsets of a tile whose row indices are in set p
+  auto set_aoff = [&](const Tile& t, int p) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int row = 16 * wave + 8 * q + r8, r = 128 * h + row;
+        const uint32_t src = MODE == 0 ? (uint32_t)row_s[p][r]
+                                       : (uint32_t)(t.start + t.m0 + (r < t.vrows ? r : 0));
+        aoff[h][q] = (src * (uint32_t)K + (uint32_t)((slot8 ^ swz_a(row)) * 8)) * 2u;
+      }
+  };
 
   // XCD-aware order: workgroup b runs on XCD b % 8 (round-robin dispatch), so in each round
   // of gridDim tiles the workgroups of one XCD take a contiguous run of tiles.  Tiles of one
@@ -1327,70 +1423,62 @@ __global__ __launch_bounds__(kTiledThreads) __attribute__((amdgpu_waves_per_eu(2
   // A and B slices are shared in that XCD's L2.
   const int per_xcd = gridDim.x % 8 == 0 ? (int)gridDim.x / 8 : 0;
   const int lslot = per_xcd ? (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8) : (int)blockIdx.x;
-  for (int tile = lslot; tile < total; tile += gridDim.x) {
-    const int mt_global = tile / ntn, ntile = tile % ntn;
-    const int li = find_entry(tt, mt_global);
-    const int64_t start = tt.start[li];
-    const int n = tt.rows[li];
-    const int m0 = (mt_global - tt.cum[li]) * BM;
-    const bf16_t* slot = a.cache + (int64_t)a.list.slot[li] * 3 * a.H * a.I;
-
-    // Direct loads: of each half this wavefront moves rows 16 wave + 8 q + lane / 8 (q < 2), lane
-    // slot lane % 8 holding the row's chunk (lane % 8) ^ swizzle(row).  Rows past the expert's
-    // last row load its first row instead: each output row depends only on its own A row, and
-    // those rows are never stored.
-    const int r8 = lane >> 3, slot8 = lane & 7;
-    uint32_t aoff[2][2], boff[2];   // byte offsets: < 2^32 (host-checked sizes)
-    const char* abase = reinterpret_cast<const char*>(MODE == 0 ? a.x : a.act);
-    const uint32_t lda = (uint32_t)(MODE == 0 ? a.H : a.I);
+  if (lslot >= total) return;
+  typedef std::integral_constant<int, 0> I0;
+  typedef std::integral_constant<int, 1> I1;
+  bf16x8 ft[4][2], fw[2][2][2];
+  auto read_a = [&](auto h, auto s) {
+    constexpr int off = (2 * decltype(h)::value + decltype(s)::value) * kHalfBytes;
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int row = 16 * wave + 8 * q + r8;
+    for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int r = m0 + 128 * h + row;
-        const bool ok = r < n;
-        const uint32_t t = MODE == 0 ? (uint32_t)a.rows[start + (ok ? r : 0)]
-                                     : (uint32_t)(start + (ok ? r : 0));
-        aoff[h][q] = (t * lda + (uint32_t)((slot8 ^ swz_a(row)) * 8)) * 2u;
+      for (int i = 0; i < 4; ++i) ft[i][ks] = lds_read16(a_addr[ks] + off + i * 32 * kRowBytes);
+  };
+  auto read_b = [&](auto h, auto s) {
+    constexpr int H = decltype(h)::value, off = (2 * H + decltype(s)::value) * kHalfBytes;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) fw[H][c][ks] = lds_read16(b_addr[ks] + off + c * 4 * kRowBytes);
+  };
+  // the first tile's first two stages, halves in the order in which they are read
+  Tile cur = locate(lslot);
+  load_rows(cur, 0);
+  wait_cnt<0>();
+  wg_barrier();
+  set_aoff(cur, 0);
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    dma_b(cur.bbase + k * BK * 2, 0, k);
+    dma_a(k, 0, k);
+    dma_b(cur.bbase + k * BK * 2, 1, k);
+    dma_a(k, 1, k);
+  }
+  wait_cnt<12>();   // B half 0 and A half 0 of stage 0 have landed
+  wg_barrier();
+  read_b(I0{}, I0{});
+  // every wavefront has read B half 0 of stage 0 before stage 0's first loads replace it
+  wait_cnt<12>();
+  wg_barrier();
+  if (wm == 1) wg_barrier();   // the second group runs one segment behind the first
+  int set = 0;
+  for (int tile = lslot; tile < total; tile += gridDim.x, set ^= 1) {
+    // the tile after this one; after the last tile its own first stages are loaded again
+    const bool more = tile + (int)gridDim.x < total;
+    Tile next = cur;
+    if (more) next = locate(tile + gridDim.x);
+    load_rows(next, set ^ 1);
+    if constexpr (MODE == 1) {
+      // output row and routing weight of tile row tid, in LDS before the epilogue reads them
+      if (wave < 4) {
+        const int64_t tj = (int64_t)row_s[set][tid] * a.k + col_s[set][tid];
+        dma2(reinterpret_cast<const char*>(a.w), (uint32_t)(tj * 2), lds_addr(wt_s[set]) + 256 * wave);
+        orow_s[set][tid] = a.out_mode == 0 ? (int32_t)tj : (int32_t)(cur.start + cur.m0 + tid);
       }
-      boff[q] = (uint32_t)(((uint32_t)(8 * q + r8) * (uint32_t)K + (uint32_t)((slot8 ^ swz_b(row)) * 8)) * 2u);
     }
-    const char* bbase[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-      bbase[h] = reinterpret_cast<const char*>(uniform_ptr(
-          MODE == 0 ? slot + (int64_t)h * a.H * a.I + (int64_t)(ntile * 128 + 16 * wave) * a.H
-                    : slot + 2 * a.H * a.I + (int64_t)(ntile * BN + 128 * h + 16 * wave) * a.I));
-    const int vrows = n - m0;                                          // > 0
-    // per-row output row and routing weight for the phase-2 epilogue
-    auto row_meta = [&]() {
-      if (MODE == 1) {
-        for (int r = tid; r < BM; r += kTiledThreads) {
-          const int rr = m0 + r;
-          int64_t orow = 0;
-          float wt = 0.f;
-          if (rr < n) {
-            const int64_t p = start + rr;
-            const int64_t t = a.rows[p], j = a.cols[p];
-            wt = bf16_to_f32(a.w[t * a.k + j]);
-            orow = (a.out_mode == 0 ? t * a.k + j : p) * a.H;
-          }
-          orow_s[r] = orow;
-          wt_s[r] = wt;
-        }
-      }
-    };
+    const int vrows = cur.vrows, ntile = cur.ntile;
+    const int64_t row0 = cur.start + cur.m0;
 
-    floatx4 acc[2][2][4][2];   // [A half][B half][16-row tile][16-column tile]
-#pragma unroll
-    for (int ha = 0; ha < 2; ++ha)
-#pragma unroll
-      for (int hb = 0; hb < 2; ++hb)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int c = 0; c < 2; ++c) acc[ha][hb][i][c] = floatx4{0, 0, 0, 0};
     // 16-row tiles of each A half that hold rows of the expert (the others' products are skipped
     // in a partial tile: their output rows are never stored)
     int nf[2];
@@ -1400,126 +1488,99 @@ __global__ __launch_bounds__(kTiledThreads) __attribute__((amdgpu_waves_per_eu(2
       nf[h] = __builtin_amdgcn_readfirstlane(v >= 128 ? 4 : (v > 0 ? (v + 31) / 32 : 0));
     }
 
-    bf16x8 ft[4][2], fw[2][2][2];
-    auto dma_a = [&](int kt, int h, int s) {
-      const uint32_t dst = smem0 + (uint32_t)((2 * h + s) * kHalfBytes + 16 * wave * kRowBytes);
-#pragma unroll
-      for (int q = 0; q < 2; ++q)
-        dma16(abase + kt * BK * 2, aoff[h][q], dst + (uint32_t)(8 * q * kRowBytes));
-    };
-    auto dma_b = [&](int kt, int h, int s) {
-      const uint32_t dst = smem0 + (uint32_t)((4 + 2 * h + s) * kHalfBytes + 16 * wave * kRowBytes);
-#pragma unroll
-      for (int q = 0; q < 2; ++q)
-        dma16(bbase[h] + kt * BK * 2, boff[q], dst + (uint32_t)(8 * q * kRowBytes));
-    };
-    auto read_a = [&](auto h, auto s) {
-      constexpr int off = (2 * decltype(h)::value + decltype(s)::value) * kHalfBytes;
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          ft[i][ks] = *reinterpret_cast<const bf16x8*>(smem + a_addr[ks] + off + i * 32 * kRowBytes);
-    };
-    auto read_b = [&](auto h, auto s) {
-      constexpr int H = decltype(h)::value, off = (2 * H + decltype(s)::value) * kHalfBytes;
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-        for (int c = 0; c < 2; ++c)
-          fw[H][c][ks] = *reinterpret_cast<const bf16x8*>(smem + b_addr[ks] + off + c * 4 * kRowBytes);
-    };
     auto pipeline = [&](auto part) {
       constexpr bool PARTIAL = decltype(part)::value;
-      auto mma = [&](auto ha, auto hb) {
-        constexpr int A = decltype(ha)::value, B = decltype(hb)::value;
-        __builtin_amdgcn_s_setprio(1);
+      floatx4 acc[2][2][4][2];   // [A half][B half][16-row tile][16-column tile]
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
+      for (int ha = 0; ha < 2; ++ha)
+#pragma unroll
+        for (int hb = 0; hb < 2; ++hb)
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            if (!PARTIAL || i < nf[A]) {
 #pragma unroll
-              for (int c = 0; c < 2; ++c)
-                acc[A][B][i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[B][c][ks], ft[i][ks],
-                                                                         acc[A][B][i][c], 0, 0, 0);
+            for (int c = 0; c < 2; ++c) acc[ha][hb][i][c] = floatx4{0, 0, 0, 0};
+      auto mma = [&](auto ha, auto hb) {
+        constexpr int A = decltype(ha)::value, B = decltype(hb)::value;
+        auto tile_row = [&](int i, int ks) {
+#pragma unroll
+          for (int c = 0; c < 2; ++c)
+            acc[A][B][i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[B][c][ks], ft[i][ks],
+                                                                     acc[A][B][i][c], 0, 0, 0);
+        };
+        __builtin_amdgcn_s_setprio(1);
+        if constexpr (!PARTIAL) {
+#pragma unroll
+          for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) tile_row(i, ks);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; i += 2)
+            if (i < nf[A]) {
+#pragma unroll
+              for (int ks = 0; ks < 2; ++ks) {
+                tile_row(i, ks);
+                tile_row(i + 1, ks);
+              }
             }
+        }
         __builtin_amdgcn_s_setprio(0);
         wg_barrier();
       };
-      // end of a memory segment: the loads of the next segment's half have landed (at most N
-      // younger ones in flight), this segment's fragments are in registers
-      auto mem_end = [&](auto nn) {
-        wait_cnt<decltype(nn)::value>();
+      // end of a memory segment: the loads of the next segment's half have landed (the 12 loads of
+      // the six halves after it may be in flight), this segment's fragments are in registers
+      auto mem_end = [&]() {
+        wait_cnt<12>();
         wg_barrier();
       };
-      typedef std::integral_constant<int, 0> I0;
-      typedef std::integral_constant<int, 1> I1;
-      // stage k in slot S; LAST: the last two stages issue no loads
-      auto stage = [&](int k, auto ss, auto tail) {
+      // a stage in slot S; its loads are those of stage kl (A) and at bl (B)
+      auto stage = [&](const char* bl, int kl, auto ss) {
         constexpr int S = decltype(ss)::value;
-        constexpr int T = decltype(tail)::value;   // 0, or 1 / 2 for the last but one / last stage
         typedef std::integral_constant<int, S> IS;
         typedef std::integral_constant<int, 1 - S> IO;
-        auto left = [&](auto ph) {   // loads in flight after phase ph's memory segment
-          constexpr int v = T == 0 ? 12 : 12 - 2 * (4 * (T - 1) + decltype(ph)::value + 1);
-          return std::integral_constant<int, (v > 0 ? v : 0)>{};
-        };
         read_a(I0{}, IS{});
-        if constexpr (T == 0) dma_b(k + 2, 0, S);
-        mem_end(left(std::integral_constant<int, 0>{}));
+        dma_b(bl, 0, S);
+        mem_end();
         mma(I0{}, I0{});
         read_b(I1{}, IS{});
-        if constexpr (T == 0) dma_a(k + 2, 0, S);
-        mem_end(left(std::integral_constant<int, 1>{}));
+        dma_a(kl, 0, S);
+        mem_end();
         mma(I0{}, I1{});
         read_a(I1{}, IS{});
-        if constexpr (T == 0) dma_b(k + 2, 1, S);
-        mem_end(left(std::integral_constant<int, 2>{}));
+        dma_b(bl, 1, S);
+        mem_end();
         mma(I1{}, I0{});
-        if constexpr (T < 2) read_b(I0{}, IO{});
-        if constexpr (T == 0) dma_a(k + 2, 1, S);
-        mem_end(left(std::integral_constant<int, 3>{}));
+        read_b(I0{}, IO{});
+        dma_a(kl, 1, S);
+        mem_end();
         mma(I1{}, I1{});
       };
-      // prologue: both stages' halves in the order in which they are read
-      dma_b(0, 0, 0);
-      dma_a(0, 0, 0);
-      dma_b(0, 1, 0);
-      dma_a(0, 1, 0);
-      dma_b(1, 0, 1);
-      dma_a(1, 0, 1);
-      dma_b(1, 1, 1);
-      dma_a(1, 1, 1);
-      asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
-      wg_barrier();
-      read_b(I0{}, I0{});
-      // every wavefront has read B half 0 of stage 0 before stage 0's first loads replace it
-      wait_cnt<12>();
-      wg_barrier();
-      if (wm == 1) wg_barrier();   // the second group runs one segment behind the first
-      int k = 0;
-      for (; k + 2 < KT; k += 2) {
-        stage(k, I0{}, I0{});
-        stage(k + 1, I1{}, I0{});
+      const char* bnext = cur.bbase + 2 * BK * 2;   // B half 0 of the stage loaded next
+      int kl = 2;
+      for (int k = 0; k < KT; k += 2) {
+        if (k + 2 == KT) {   // the last two stages load the next tile's first two
+          set_aoff(next, set ^ 1);
+          bnext = next.bbase;
+          kl = 0;
+        }
+        bnext = uniform_ptr(bnext);
+        stage(bnext, kl, I0{});
+        stage(bnext + BK * 2, kl + 1, I1{});
+        bnext += 2 * BK * 2;
+        kl += 2;
       }
-      stage(k, I0{}, I1{});
-      stage(k + 1, I1{}, std::integral_constant<int, 2>{});
-      if (wm == 0) wg_barrier();
-    };
-    row_meta();
-    if (vrows >= BM)
-      pipeline(std::false_type{});
-    else
-      pipeline(std::true_type{});
     // 16x16 accumulator layout (first operand: weight rows): column = token row lane & 15, rows
     // (lane >> 4) * 4 + q.  The weight rows of tiles c = 0, 1 interleave in groups of four (see
     // b_addr), so a lane holds 8 consecutive output columns of one token row: one 16-byte store.
+    // the lane's row, opaque here so that the stores' addresses are computed now and not kept in
+    // registers through the loop
+    int erow = 16 * wm + j16;
+    asm volatile("" : "+v"(erow));
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int r = 128 * h + 32 * i + 16 * wm + j16;
+        const int r = 128 * h + 32 * i + erow;
         if constexpr (MODE == 0) {
           u32x4 y;
 #pragma unroll
@@ -1534,10 +1595,10 @@ __global__ __launch_bounds__(kTiledThreads) __attribute__((amdgpu_waves_per_eu(2
               y[2 * c + q / 2] = pk_bf16(s0, s1);
             }
           if (r < vrows)
-            *reinterpret_cast<u32x4*>(&a.act[(start + m0 + r) * a.I + ntile * 128 + wn * 32 + 8 * g4]) = y;
+            *reinterpret_cast<u32x4*>(&a.act[(row0 + r) * a.I + ntile * 128 + wn * 32 + 8 * g4]) = y;
         } else {
-          const float wt = wt_s[r];
-          bf16_t* const o = a.out + orow_s[r] + ntile * BN + wn * 32 + 8 * g4;
+          const float wt = __uint_as_float((uint32_t)wt_s[set][r] << 16);
+          bf16_t* const o = a.out + (int64_t)orow_s[set][r] * a.H + ntile * BN + wn * 32 + 8 * g4;
 #pragma unroll
           for (int hb = 0; hb < 2; ++hb) {
             u32x4 y;
@@ -1553,19 +1614,22 @@ __global__ __launch_bounds__(kTiledThreads) __attribute__((amdgpu_waves_per_eu(2
           }
         }
       }
-    // the row table is free again once every wavefront has read it (the stores stay in flight)
-    if (MODE == 1) {
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      wg_barrier();
-    }
+    };
+    if (vrows >= BM)
+      pipeline(std::false_type{});
+    else
+      pipeline(std::true_type{});
+    cur = next;
   }
+  if (wm == 0) wg_barrier();
+  wait_cnt<0>();   // no load may write this workgroup's LDS after its end
 }
 
 // Smaller tiles, for lists that leave CUs idle (or a nearly empty last round) with 256 x 256 ones
 // (choose_tile): TM = 16 WM MI rows by TN = 16 WN NI weight rows per workgroup of WM x WN
 // wavefronts, each with MI x NI 16 x 16 accumulators.  Such a launch is one or two rounds of tiles,
 // so a tile's latency is what counts: its stages (64 columns of K) stream through an LDS ring as
-// deep as 144 KiB allows (3 to 6 stages for the five shapes below), the loads of a stage spread
+// deep as 144 KiB allows (3 to 9 stages for the five shapes below), the loads of a stage spread
 // between the matrix instructions; a wavefront's fragments of the next 32 columns are read while
 // the current ones are multiplied.  The loads of one CU reach it at about 64 bytes a clock, which a
 // 64 x 64 tile needs for 256 clocks of 128 clocks of products a stage: below that size nothing is
@@ -1575,16 +1639,6 @@ __global__ __launch_bounds__(kTiledThreads) __attribute__((amdgpu_waves_per_eu(2
 // Products, K order, operand layout in LDS and roundings are those of ffn_tiled, so the outputs
 // do not depend on the tile.
 
-// 4-byte global->LDS direct load of each lane (LDS byte address lds + 4 * lane), as dma16
-__device__ __forceinline__ void dma4(const char* sbase, uint32_t voff, uint32_t lds) {
-  asm volatile(
-      "s_mov_b32 m0, %2\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dword %0, %1"
-      :
-      : "v"(voff), "s"(sbase), "s"(lds)
-      : "memory", "m0");
-}
 // wait until at most y groups of LPS vector-memory operations are outstanding (y wave-uniform,
 // values above V count as V)
 template <int V, int LPS>
