@@ -8,12 +8,21 @@
 // an expert (:64-74).  The packet weights of pack_dispatch (ferry/csrc/expert_ops.cpp:57-60)
 // are the routing weights reordered into send_ids order.
 //
-// Design: tokens are processed in blocks of 1024 (16 wavefronts x 64 lanes, one token per
-// lane).  Within a wavefront the rank of a token among the earlier tokens that chose the
-// same expert is a popcount of a 64-bit per-expert lane mask built with LDS atomic ORs; the
-// wavefront and block offsets come from exclusive scans.  No global atomics are used, so the
-// permutation is deterministic.  A single block (T <= 1024) does everything in one launch;
-// larger T uses count -> scan -> scatter launches.
+// Design: one token per lane.  Within a wavefront the rank of a token among the earlier tokens that
+// chose the same expert is a popcount of a 64-bit per-expert lane mask built with LDS atomic ORs;
+// the wavefront and block offsets come from exclusive scans.  No global atomics are used, so the
+// permutation is deterministic.  Up to 512 tokens a single block (of as many wavefronts as the
+// tokens need) does everything in one launch; more take two: per-block histograms, then the
+// scatter, in which every block sums the histograms before its own.
+//
+// Both are bound by latency: a chain of LDS and L2 round trips on few wavefronts.  Hence the ID sort
+// in registers over 8 slots when k <= 8 (16 otherwise), scans across lanes rather than by one thread,
+// and blocks of 256 tokens where the histograms then stay small (256 blocks at 65,536 tokens
+// instead of 64 of 1024).  us, with one sort width, a one-thread scan, 1024-token blocks and a scan
+// launch of its own -> now: 16 tokens (k = 8, 128 experts) 10.2 -> 6.5; 512 tokens 15.8 -> 12.1; 1024
+// tokens 25.0 -> 13.4; 8192 tokens 34.9 -> 14.4; 65,536 tokens (k = 6, 64 experts) 39 -> 16.  The one
+// launch is left at 512 tokens, where both take 12 us: one CU then spends its time on the scattered
+// stores (22.5 us at 1024 tokens).
 #include "common.h"
 
 #include <mutex>
@@ -23,23 +32,25 @@ namespace {
 
 constexpr int kMaxE = 512;
 constexpr int kMaxK = 16;
-constexpr int kWaves = 16;
-constexpr int kBlockTokens = 64 * kWaves;
+constexpr int kSingleTokens = 512;    // most tokens of the one-launch layout
+constexpr int kMaxBlock = 1024;       // most tokens of a block of the two-launch layout
 
+template <int KM>
 struct TokenIds {
-  int32_t id[kMaxK];
-  bf16_t w[kMaxK];
+  int32_t id[KM];
+  bf16_t w[KM];
 };
 
-// Load one token's k IDs and weights and sort them by ID (IDs of a token are distinct, so any
+// Load one token's k <= KM IDs and weights and sort them by ID (IDs of a token are distinct, so any
 // sort gives the insertion-sort result); out-of-range entries carry the key kMaxE, padding
 // entries kMaxE + 1.  `bad` is set for a token with an out-of-range or a repeated ID: such a
 // token breaks the layout's contract (its entries would share one permutation slot).
+template <int KM>
 __device__ __forceinline__ void load_sorted(const int64_t* __restrict__ selected,
                                             const bf16_t* __restrict__ weights, int64_t t, int k,
-                                            int E, TokenIds& s, bool& bad) {
+                                            int E, TokenIds<KM>& s, bool& bad) {
 #pragma unroll
-  for (int j = 0; j < kMaxK; ++j) {
+  for (int j = 0; j < KM; ++j) {
     if (j < k) {
       int64_t e = selected[t * k + j];
       bad |= (e < 0 || e >= E);
@@ -50,11 +61,11 @@ __device__ __forceinline__ void load_sorted(const int64_t* __restrict__ selected
       s.w[j] = 0;
     }
   }
-  // odd-even transposition sort over kMaxK slots (static indices keep it in registers)
+  // odd-even transposition sort over KM slots (static indices keep it in registers)
 #pragma unroll
-  for (int r = 0; r < kMaxK; ++r) {
+  for (int r = 0; r < KM; ++r) {
 #pragma unroll
-    for (int j = r & 1; j + 1 < kMaxK; j += 2) {
+    for (int j = r & 1; j + 1 < KM; j += 2) {
       if (s.id[j] > s.id[j + 1]) {
         int32_t ti = s.id[j];
         s.id[j] = s.id[j + 1];
@@ -66,61 +77,99 @@ __device__ __forceinline__ void load_sorted(const int64_t* __restrict__ selected
     }
   }
 #pragma unroll
-  for (int j = 0; j + 1 < kMaxK; ++j) bad |= (j + 1 < k && s.id[j] < E && s.id[j] == s.id[j + 1]);
+  for (int j = 0; j + 1 < KM; ++j) bad |= (j + 1 < k && s.id[j] < E && s.id[j] == s.id[j + 1]);
 }
 
-struct LayoutShared {
-  unsigned long long mask[kWaves][kMaxE];  // lanes of the wavefront that chose expert e
-  int32_t wave_base[kWaves][kMaxE];        // exclusive prefix over wavefronts, per expert
+// LDS of a block of `waves` wavefronts, E experts: lane masks (the wavefront's lanes that chose
+// expert e), exclusive prefixes over the wavefronts, and two per-expert arrays
+struct BlockLds {
+  unsigned long long* mask;   // [waves][E]
+  int32_t* wave_base;         // [waves][E]
+  int32_t* count;             // [E]
+  int32_t* base;              // [E]
+  __device__ BlockLds(char* p, int waves, int E) {
+    mask = reinterpret_cast<unsigned long long*>(p);
+    wave_base = reinterpret_cast<int32_t*>(mask + waves * E);
+    count = wave_base + waves * E;
+    base = count + E;
+  }
+  static size_t bytes(int waves, int E) { return (size_t)E * (waves * 12 + 8); }
 };
 
-// Phase 1 of a block: build the lane masks of its tokens and the per-wavefront prefix.
-// Returns (in block_count[e], when non-null) the number of the block's tokens per expert.
-__device__ void block_masks(LayoutShared& sh, const int64_t* __restrict__ selected,
-                            const bf16_t* __restrict__ weights, int64_t tokens, int k, int E,
-                            int64_t t0, TokenIds& s, bool& valid, bool& bad,
-                            int32_t* block_count) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int i = threadIdx.x; i < kWaves * E; i += blockDim.x) sh.mask[i / E][i % E] = 0ull;
-  __syncthreads();
-  const int64_t t = t0 + threadIdx.x;
+// Phase 1 of a block: the lane masks of its tokens and the per-wavefront prefixes; count[e] (with
+// COUNT) is the number of the block's tokens per expert.
+template <int KM, bool COUNT>
+__device__ __forceinline__ void block_masks(const BlockLds& sh, const int64_t* __restrict__ selected,
+                                            const bf16_t* __restrict__ weights, int64_t tokens,
+                                            int k, int E, int64_t t, TokenIds<KM>& s, bool& valid,
+                                            bool& bad) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
   valid = t < tokens;
+  if (valid) load_sorted(selected, weights, t, k, E, s, bad);
+  for (int i = threadIdx.x; i < waves * E; i += blockDim.x) sh.mask[i] = 0ull;
+  __syncthreads();
   if (valid) {
-    load_sorted(selected, weights, t, k, E, s, bad);
 #pragma unroll
-    for (int j = 0; j < kMaxK; ++j)
-      if (j < k && s.id[j] < E) atomicOr(&sh.mask[wave][s.id[j]], 1ull << lane);
+    for (int j = 0; j < KM; ++j)
+      if (j < k && s.id[j] < E) atomicOr(&sh.mask[wave * E + s.id[j]], 1ull << lane);
   }
   __syncthreads();
   for (int e = threadIdx.x; e < E; e += blockDim.x) {
     int32_t run = 0;
-    for (int w = 0; w < kWaves; ++w) {
-      sh.wave_base[w][e] = run;
-      run += __popcll(sh.mask[w][e]);
+    for (int w = 0; w < waves; ++w) {
+      sh.wave_base[w * E + e] = run;
+      run += __popcll(sh.mask[w * E + e]);
     }
-    if (block_count) block_count[e] = run;
+    if (COUNT) sh.count[e] = run;
   }
   __syncthreads();
 }
 
+// Wavefront 0: exclusive prefix of count[0 .. E) into base (added to it with ADD), and into starts
+// (with its total at E) when given.
+template <bool ADD>
+__device__ __forceinline__ void scan_experts(const int32_t* count, int32_t* base, int E,
+                                             int64_t* __restrict__ starts) {
+  if (threadIdx.x >= 64) return;
+  const int lane = threadIdx.x;
+  int32_t carry = 0;
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    const int e = e0 + lane;
+    const int32_t c = e < E ? count[e] : 0;
+    int32_t incl = c;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int32_t v = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += v;
+    }
+    if (e < E) {
+      base[e] = (ADD ? base[e] : 0) + carry + incl - c;
+      if (starts) starts[e] = carry + incl - c;
+    }
+    carry += __shfl(incl, 63, 64);
+  }
+  if (lane == 0 && starts) starts[E] = carry;
+}
+
 // Phase 2 of a block: write the sorted IDs, packet weights and the permutation entries.
 // base[e] = grouped position of the block's first entry of expert e.
-__device__ void block_scatter(const LayoutShared& sh, const int32_t* base, int64_t t, int k,
-                              const TokenIds& s, int64_t* __restrict__ send_ids,
-                              bf16_t* __restrict__ w_sorted, int64_t* __restrict__ rows,
-                              int64_t* __restrict__ cols, int32_t* __restrict__ pair_pos,
-                              int E) {
+template <int KM>
+__device__ __forceinline__ void block_scatter(const BlockLds& sh, int64_t t, int k,
+                                              const TokenIds<KM>& s, int64_t* __restrict__ send_ids,
+                                              bf16_t* __restrict__ w_sorted,
+                                              int64_t* __restrict__ rows, int64_t* __restrict__ cols,
+                                              int32_t* __restrict__ pair_pos, int E) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
 #pragma unroll
-  for (int j = 0; j < kMaxK; ++j) {
+  for (int j = 0; j < KM; ++j) {
     if (j < k) {
       const int32_t e = s.id[j];
       send_ids[t * k + j] = e < E ? e : -1;
       if (w_sorted) w_sorted[t * k + j] = s.w[j];
       if (e < E) {
-        const int64_t pos =
-            (int64_t)base[e] + sh.wave_base[wave][e] + __popcll(sh.mask[wave][e] & below);
+        const int64_t pos = (int64_t)sh.base[e] + sh.wave_base[wave * E + e] +
+                            __popcll(sh.mask[wave * E + e] & below);
         rows[pos] = t;
         cols[pos] = j;
         if (pair_pos) pair_pos[t * k + j] = (int32_t)pos;
@@ -131,86 +180,108 @@ __device__ void block_scatter(const LayoutShared& sh, const int32_t* base, int64
   }
 }
 
-__global__ __launch_bounds__(kBlockTokens) void layout_single(
+template <int KM>
+__global__ __launch_bounds__(kSingleTokens) void layout_single(
     const int64_t* __restrict__ selected, const bf16_t* __restrict__ weights, int64_t tokens,
     int k, int E, int64_t* __restrict__ send_ids, bf16_t* __restrict__ w_sorted,
     int64_t* __restrict__ starts, int64_t* __restrict__ rows, int64_t* __restrict__ cols,
     int32_t* __restrict__ pair_pos, int32_t* __restrict__ err) {
-  __shared__ LayoutShared sh;
-  __shared__ int32_t count[kMaxE];
-  __shared__ int32_t base[kMaxE];
-  TokenIds s;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const BlockLds sh(lds, blockDim.x >> 6, E);
+  TokenIds<KM> s;
   bool valid, bad = false;
   if (threadIdx.x == 0) *err = 0;  // ordered before the atomics by the barriers below
-  block_masks(sh, selected, weights, tokens, k, E, 0, s, valid, bad, count);
-  if (threadIdx.x == 0) {
-    int32_t run = 0;
-    for (int e = 0; e < E; ++e) {
-      base[e] = run;
-      starts[e] = run;
-      run += count[e];
-    }
-    starts[E] = run;
-  }
+  block_masks<KM, true>(sh, selected, weights, tokens, k, E, threadIdx.x, s, valid, bad);
+  scan_experts<false>(sh.count, sh.base, E, starts);
   __syncthreads();
   if (valid) {
-    block_scatter(sh, base, threadIdx.x, k, s, send_ids, w_sorted, rows, cols, pair_pos, E);
+    block_scatter(sh, threadIdx.x, k, s, send_ids, w_sorted, rows, cols, pair_pos, E);
     if (bad) atomicAdd(err, 1);
   }
 }
 
-__global__ __launch_bounds__(kBlockTokens) void layout_count(
-    const int64_t* __restrict__ selected, int64_t tokens, int k, int E,
-    int32_t* __restrict__ block_hist) {
-  __shared__ LayoutShared sh;
-  TokenIds s;
-  bool valid, bad = false;
-  block_masks(sh, selected, nullptr, tokens, k, E, (int64_t)blockIdx.x * kBlockTokens, s, valid,
-              bad, block_hist + (int64_t)blockIdx.x * E);
-}
-
-// One block: per expert, exclusive prefix over blocks; starts = exclusive prefix of totals.
-__global__ __launch_bounds__(kMaxE) void layout_scan(int32_t* __restrict__ block_hist, int nblk,
-                                                     int E, int64_t* __restrict__ starts,
-                                                     int32_t* __restrict__ err) {
-  __shared__ int32_t total[kMaxE];
-  const int e = threadIdx.x;
-  if (e == 0) *err = 0;
-  if (e < E) {
-    int32_t run = 0;
-    for (int b = 0; b < nblk; ++b) {
-      const int32_t c = block_hist[(int64_t)b * E + e];
-      block_hist[(int64_t)b * E + e] = run;
-      run += c;
+// Per-expert counts of each block of block_tokens tokens; an expert that a token names twice
+// counts once (as its lane mask holds it once), IDs outside [0, E) do not count.
+constexpr int kCountThreads = 256;
+template <int KM>
+__global__ __launch_bounds__(kCountThreads) void layout_count(
+    const int64_t* __restrict__ selected, int64_t tokens, int k, int E, int block_tokens,
+    int32_t* __restrict__ block_hist, int32_t* __restrict__ err) {
+  __shared__ int32_t hist[kMaxE];
+  if (blockIdx.x == 0 && threadIdx.x == 0) *err = 0;
+  for (int e = threadIdx.x; e < E; e += kCountThreads) hist[e] = 0;
+  __syncthreads();
+  const int64_t t0 = (int64_t)blockIdx.x * block_tokens;
+  for (int i = threadIdx.x; i < block_tokens; i += kCountThreads) {
+    const int64_t t = t0 + i;
+    if (t >= tokens) break;
+    int64_t id[KM];
+#pragma unroll
+    for (int j = 0; j < KM; ++j) id[j] = j < k ? selected[t * k + j] : -1;
+#pragma unroll
+    for (int j = 0; j < KM; ++j) {
+      bool count = id[j] >= 0 && id[j] < E;
+#pragma unroll
+      for (int q = 0; q < j; ++q) count &= id[q] != id[j];
+      if (count) atomicAdd(&hist[id[j]], 1);
     }
-    total[e] = run;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int64_t run = 0;
-    for (int i = 0; i < E; ++i) {
-      starts[i] = run;
-      run += total[i];
-    }
-    starts[E] = run;
-  }
+  for (int e = threadIdx.x; e < E; e += kCountThreads) block_hist[(int64_t)blockIdx.x * E + e] = hist[e];
 }
 
-__global__ __launch_bounds__(kBlockTokens) void layout_scatter(
+template <int KM>
+__global__ __launch_bounds__(kMaxBlock) void layout_scatter(
     const int64_t* __restrict__ selected, const bf16_t* __restrict__ weights, int64_t tokens,
-    int k, int E, const int32_t* __restrict__ block_hist, const int64_t* __restrict__ starts,
+    int k, int E, const int32_t* __restrict__ block_hist, int64_t* __restrict__ starts,
     int64_t* __restrict__ send_ids, bf16_t* __restrict__ w_sorted, int64_t* __restrict__ rows,
     int64_t* __restrict__ cols, int32_t* __restrict__ pair_pos, int32_t* __restrict__ err) {
-  __shared__ LayoutShared sh;
-  __shared__ int32_t base[kMaxE];
-  TokenIds s;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const BlockLds sh(lds, blockDim.x >> 6, E);
+  const int nblk = gridDim.x, b = blockIdx.x;
+  // per expert: the entries of the blocks before this one (base) and of all blocks (count); the
+  // blocks are dealt to the threads of a column of experts (four a thread where E allows)
+  for (int e = threadIdx.x; e < E; e += blockDim.x) sh.count[e] = sh.base[e] = 0;
+  __syncthreads();
+  const bool vec = E % 4 == 0 && ((uintptr_t)block_hist & 15) == 0;
+  const int cols_n = vec ? E / 4 : E;
+  const int parts = (int)blockDim.x / cols_n > 1 ? (int)blockDim.x / cols_n : 1;
+  for (int c = threadIdx.x; c < cols_n * parts; c += blockDim.x) {
+    const int col = c % cols_n, part = c / cols_n;
+    if (vec) {
+      typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
+      i32x4 pre = {0, 0, 0, 0}, all = {0, 0, 0, 0};
+#pragma unroll 4
+      for (int q = part; q < nblk; q += parts) {
+        const i32x4 h = *reinterpret_cast<const i32x4*>(block_hist + (int64_t)q * E + 4 * col);
+        all += h;
+        if (q < b) pre += h;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        atomicAdd(&sh.base[4 * col + i], pre[i]);
+        atomicAdd(&sh.count[4 * col + i], all[i]);
+      }
+    } else {
+      int32_t pre = 0, all = 0;
+#pragma unroll 4
+      for (int q = part; q < nblk; q += parts) {
+        const int32_t h = block_hist[(int64_t)q * E + col];
+        all += h;
+        if (q < b) pre += h;
+      }
+      atomicAdd(&sh.base[col], pre);
+      atomicAdd(&sh.count[col], all);
+    }
+  }
+  __syncthreads();
+  scan_experts<true>(sh.count, sh.base, E, b == 0 ? starts : nullptr);
+  TokenIds<KM> s;
   bool valid, bad = false;
-  const int64_t t0 = (int64_t)blockIdx.x * kBlockTokens;
-  for (int e = threadIdx.x; e < E; e += blockDim.x)
-    base[e] = (int32_t)(starts[e] + block_hist[(int64_t)blockIdx.x * E + e]);
-  block_masks(sh, selected, weights, tokens, k, E, t0, s, valid, bad, nullptr);
+  const int64_t t = (int64_t)b * blockDim.x + threadIdx.x;
+  block_masks<KM, false>(sh, selected, weights, tokens, k, E, t, s, valid, bad);
   if (valid) {
-    block_scatter(sh, base, t0 + threadIdx.x, k, s, send_ids, w_sorted, rows, cols, pair_pos, E);
+    block_scatter(sh, t, k, s, send_ids, w_sorted, rows, cols, pair_pos, E);
     if (bad) atomicAdd(err, 1);
   }
 }
@@ -247,11 +318,19 @@ int scratch_address(void** out) {
 
 using namespace ferry;
 
+// Bytes of the error counter (256 B aligned) and of one histogram per block of block_tokens tokens.
+static int64_t layout_bytes(int64_t tokens, int64_t experts, int64_t block_tokens) {
+  return 256 + ceil_div(tokens > 0 ? tokens : 1, block_tokens) * experts * (int64_t)sizeof(int32_t);
+}
+// A workspace holds at least the histograms of 1024-token blocks.  Smaller blocks need more of them:
+// the recommended size has room for 256-token blocks as long as the histograms stay within 256 KiB
+// (which every block of the scatter reads); it grows with the number of tokens.
 extern "C" int64_t ferry_layout_workspace_bytes(int64_t tokens, int64_t topk, int64_t experts) {
   (void)topk;
-  const int64_t nblk = ceil_div(tokens > 0 ? tokens : 1, kBlockTokens);
-  // error counter (256 B aligned) + per-block histograms
-  return 256 + nblk * experts * (int64_t)sizeof(int32_t);
+  const int64_t need = layout_bytes(tokens, experts, kMaxBlock);
+  const int64_t fine = layout_bytes(tokens, experts, 256);
+  const int64_t room = fine < kScratchBytes ? fine : kScratchBytes;
+  return need > room ? need : room;
 }
 
 extern "C" int ferry_layout(const int64_t* selected, const void* weights_bf16, int64_t tokens,
@@ -266,9 +345,9 @@ extern "C" int ferry_layout(const int64_t* selected, const void* weights_bf16, i
                   "topk must be in [1, min(experts, %d)]", kMaxK);
   FERRY_CHECK_ARG(tokens * topk < (int64_t)1 << 31, "tokens*topk must be < 2^31");
   FERRY_CHECK_ARG(starts && workspace, "null pointer argument");
-  FERRY_CHECK_ARG(workspace_bytes >= ferry_layout_workspace_bytes(tokens, topk, experts),
+  FERRY_CHECK_ARG(workspace_bytes >= layout_bytes(tokens, experts, kMaxBlock),
                   "workspace too small (%lld < %lld bytes)", (long long)workspace_bytes,
-                  (long long)ferry_layout_workspace_bytes(tokens, topk, experts));
+                  (long long)layout_bytes(tokens, experts, kMaxBlock));
   FERRY_CHECK_ARG(tokens == 0 || (selected && send_ids && rows && cols), "null pointer argument");
   hipStream_t s = (hipStream_t)stream;
   int32_t* err = (int32_t*)workspace;
@@ -276,20 +355,26 @@ extern "C" int ferry_layout(const int64_t* selected, const void* weights_bf16, i
   const int k = (int)topk, E = (int)experts;
   const bf16_t* w = (const bf16_t*)weights_bf16;
   bf16_t* ws = (bf16_t*)w_sorted_bf16;
-  if (tokens <= kBlockTokens) {
-    launch("layout_single", layout_single, dim3(1), dim3(kBlockTokens), 0, s, selected, w, tokens, k,
-                       E, send_ids, ws, starts, rows, cols, pair_pos, err);
+  if (tokens <= kSingleTokens) {
+    const int waves = (int)ceil_div(tokens > 0 ? tokens : 1, 64);
+    launch("layout_single", k <= 8 ? layout_single<8> : layout_single<16>, dim3(1), dim3(64 * waves),
+           (uint32_t)BlockLds::bytes(waves, E), s, selected, w, tokens, k, E, send_ids, ws, starts,
+           rows, cols, pair_pos, err);
     FERRY_LAUNCHED("layout_single");
     return 0;
   }
-  const int nblk = (int)ceil_div(tokens, kBlockTokens);
-  launch("layout_count", layout_count, dim3(nblk), dim3(kBlockTokens), 0, s, selected, tokens, k, E,
-                     hist);
+  // the smallest blocks whose histograms fit the workspace and 256 KiB
+  int block = 256;
+  while (block < kMaxBlock && (layout_bytes(tokens, experts, block) > workspace_bytes ||
+                                   layout_bytes(tokens, experts, block) > kScratchBytes))
+    block *= 2;
+  const int nblk = (int)ceil_div(tokens, block);
+  launch("layout_count", k <= 8 ? layout_count<8> : layout_count<16>, dim3(nblk), dim3(kCountThreads),
+         0, s, selected, tokens, k, E, block, hist, err);
   FERRY_LAUNCHED("layout_count");
-  launch("layout_scan", layout_scan, dim3(1), dim3(kMaxE), 0, s, hist, nblk, E, starts, err);
-  FERRY_LAUNCHED("layout_scan");
-  launch("layout_scatter", layout_scatter, dim3(nblk), dim3(kBlockTokens), 0, s, selected, w, tokens, k,
-                     E, hist, starts, send_ids, ws, rows, cols, pair_pos, err);
+  launch("layout_scatter", k <= 8 ? layout_scatter<8> : layout_scatter<16>, dim3(nblk), dim3(block),
+         (uint32_t)BlockLds::bytes(block / 64, E), s, selected, w, tokens, k, E, hist, starts, send_ids,
+         ws, rows, cols, pair_pos, err);
   FERRY_LAUNCHED("layout_scatter");
   return 0;
 }
@@ -302,13 +387,13 @@ extern "C" int ferry_layout_noalloc(const int64_t* selected, const void* weights
   clear_error();
   FERRY_CHECK_ARG(tokens >= 0, "tokens must be >= 0");
   FERRY_CHECK_ARG(experts >= 1 && experts <= kMaxE, "experts must be in [1, %d]", kMaxE);
-  const int64_t need = ferry_layout_workspace_bytes(tokens, topk, experts);
+  const int64_t need = layout_bytes(tokens, experts, kMaxBlock);
   FERRY_CHECK_ARG(need <= kScratchBytes,
                   "layout_noalloc: %lld tokens x %lld experts need %lld scratch bytes, the static "
                   "buffer holds %lld (at most %lld tokens at this expert count)",
                   (long long)tokens, (long long)experts, (long long)need, (long long)kScratchBytes,
                   (long long)((kScratchBytes - 256) / (experts * (int64_t)sizeof(int32_t)) *
-                              kBlockTokens));
+                              kMaxBlock));
   void* ws = nullptr;
   const int rc = scratch_address(&ws);
   if (rc != 0) return rc;

@@ -170,7 +170,43 @@ def test_layout_bit_exact(device, T, E, k):
     assert np.array_equal(lay.pair_pos.cpu().numpy(), ref['pair_pos'])
 
 
-@pytest.mark.parametrize('T', [5, 3000])   # one-block and three-kernel layouts
+@pytest.mark.parametrize('T,E,k', [(1, 3, 3), (63, 130, 9), (65, 512, 16), (1024, 512, 16),
+                                   (1025, 5, 5), (2049, 130, 7), (66000, 512, 8), (140000, 64, 6)])
+def test_layout_blocks_and_workspaces(device, T, E, k):
+    """One launch and two, expert counts that are no multiple of 4 or 64, more than 8 IDs a token,
+    and the two-launch layout's 256-, 512- and 1024-token blocks: the recommended workspace and one
+    that only holds the histograms of 1024-token blocks give the same bits, equal to the closed
+    form."""
+    from ferry_amd._lib import last_error, lib
+    ops = _ops()
+    sel = torch.argsort(torch.rand((T, E), generator=torch.Generator().manual_seed(T)), dim=1)[:, :k]
+    sel = sel.contiguous()
+    w = torch.randn((T, k)).to(torch.bfloat16)
+    ref = layout_closed_form(sel.numpy(), E, w.view(torch.int16).numpy())
+    small = 256 + -(-T // 1024) * E * 4
+    assert small <= ops.layout_workspace_bytes(T, k, E)
+    lay = ops.layout(sel.to(device), w.to(device), E)
+    for nbytes in (lay.workspace.numel(), small):
+        for t in (lay.send_ids, lay.rows, lay.cols, lay.starts, lay.pair_pos):
+            t.fill_(-7)
+        seld, wd = sel.to(device), w.to(device)
+        rc = lib().ferry_layout(
+            seld.data_ptr(), wd.data_ptr(), T, k, E, lay.send_ids.data_ptr(), lay.w_sorted.data_ptr(),
+            lay.starts.data_ptr(), lay.rows.data_ptr(), lay.cols.data_ptr(), lay.pair_pos.data_ptr(),
+            lay.workspace.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, last_error()
+        assert ops.layout_errors(lay) == 0
+        assert np.array_equal(lay.send_ids.cpu().numpy(), ref['send_ids'])
+        assert np.array_equal(lay.w_sorted.cpu().view(torch.int16).numpy(), ref['w_sorted'])
+        assert np.array_equal(lay.starts.cpu().numpy(), ref['starts'])
+        assert np.array_equal(lay.rows.cpu().numpy(), ref['rows'])
+        assert np.array_equal(lay.cols.cpu().numpy(), ref['cols'])
+        assert np.array_equal(lay.pair_pos.cpu().numpy(), ref['pair_pos'])
+    assert lib().ferry_layout(seld.data_ptr(), wd.data_ptr(), T, k, E, *([lay.rows.data_ptr()] * 6),
+                              lay.workspace.data_ptr(), small - 4, None) != 0
+
+
+@pytest.mark.parametrize('T', [5, 3000])   # one-block and two-kernel layouts
 def test_layout_flags_invalid_ids(device, T):
     """Tokens with an out-of-range or a repeated expert ID are counted by the kernel and
     ``layout(check=True)`` raises; valid routing passes the check with a zero count."""
