@@ -17,19 +17,23 @@
 // a NaN or +inf logit has all-NaN probabilities, i.e. all elements compare equal.
 // Selection runs on order-preserving uint32 keys of the probabilities.
 //
-// Fast path (sorted output, nth_element regime, all top-k keys distinct and the k-th above
-// the (k+1)-th): the selection is unique and comes out in descending order; k wavefront
-// arg-max rounds find it.  Every other row replays the CPU algorithm exactly:
-//  * wavefront-parallel introselect: the row is held 4 keys per lane (position
-//    p = 64 * slot + lane); each median-of-3 / Hoare partition step is evaluated in one pass
-//    -- the j-th left stop (ascending position holding a key <= pivot) is exchanged with the
-//    j-th right stop (descending position holding a key >= pivot) while left < right, and
-//    the stops are ranked with ballots -- so a partition costs a few LDS round trips
-//    instead of a serial scan;
+// Every row replays the CPU algorithm exactly, on a whole wavefront:
+//  * introselect: the row is held 1, 2 or 4 keys per lane (position p = 64 * slot + lane); each
+//    median-of-3 / Hoare partition step is evaluated in one pass -- the j-th left stop (ascending
+//    position holding a key <= pivot) is exchanged with the j-th right stop (descending position
+//    holding a key >= pivot) while left < right, which every lane decides from the two ranks of
+//    its position (ballots), so a step costs one LDS round trip instead of a serial scan;
 //  * the final std::sort of the first k-1 entries (k - 1 <= 16) is an insertion sort, i.e.
 //    a stable descending sort, computed by ranking;
 //  * the rare remainder (introselect depth limit reached -> heap select; partial_sort regime
 //    k*64 <= n; k - 1 > 16) runs the sequential algorithm on lane 0 over the row in LDS.
+//
+// A decode call is bound by this chain's latency (one wavefront a row, a step of it about 1,000
+// clocks), a large batch by its instruction issue.  Finding sorted rows without ties by k arg-max
+// rounds first, and replaying the others with ranks staged in LDS, took 10.7 us for 16 rows (k = 8
+// of 128, bf16: a quarter of the rows have ties), 24.0 us for 8192 and, unsorted (k = 6 of 64, fp32),
+// 7.4 us for 256 and 108 us for 65,536 rows; now 7.6, 19.7, 5.4 and 68.8 us.  Always replaying costs
+// a single row without ties 5.0 -> 6.8 us.
 #include "common.h"
 
 // every rounding step below is the reference's: no contraction of a*b+c into one FMA
@@ -218,8 +222,6 @@ __device__ void sort_(Pair* a, int first, int last, int* stk) {
 // ---------------------------------------------------------------------------------------------
 struct WaveScratch {
   Pair stage[kMaxE];
-  int16_t lstop[kMaxE];
-  int16_t rstop[kMaxE];
   float prob[kMaxE];
   int32_t sel[kMaxK];
   int32_t stack[3 * kStack];
@@ -258,31 +260,42 @@ __device__ __forceinline__ int32_t idx_at(const int32_t (&ix)[NS], int p) {
 }
 template <int NS>
 __device__ __forceinline__ void set_at(uint32_t (&k)[NS], int32_t (&ix)[NS], int p, uint32_t kv,
-                                       int32_t iv, int lane) {
-  const bool mine = lane == (p & 63);
+                                       int32_t iv) {
   const int s = p >> 6;
-  // per-element selects (no indexed store, which would move the arrays to scratch)
+  // per-slot selects by a scalar mask (no indexed store, which would move the arrays to scratch)
 #pragma unroll
   for (int q = 0; q < NS; ++q) {
-    const bool hit = mine && q == s;
+    const bool hit = __builtin_amdgcn_inverse_ballot_w64(NS == 1 || q == s ? 1ull << (p & 63) : 0ull);
     k[q] = hit ? kv : k[q];
     ix[q] = hit ? iv : ix[q];
   }
 }
-template <int NS>
-__device__ __forceinline__ void swap_at(uint32_t (&k)[NS], int32_t (&ix)[NS], int a, int b,
-                                        int lane) {
-  const uint32_t ka = key_at(k, a), kb = key_at(k, b);
-  const int32_t ia = idx_at(ix, a), ib = idx_at(ix, b);
-  set_at(k, ix, a, kb, ib, lane);
-  set_at(k, ix, b, ka, ia, lane);
+
+// bits of the positions [lo, hi) that lie in slot s (lo, hi wave-uniform)
+__device__ __forceinline__ uint64_t slot_mask(int lo, int hi, int s) {
+  const int a = lo - 64 * s, b = hi - 64 * s;
+  const uint64_t below_b = b >= 64 ? ~0ull : (b <= 0 ? 0ull : (1ull << b) - 1);
+  const uint64_t below_a = a >= 64 ? ~0ull : (a <= 0 ? 0ull : (1ull << a) - 1);
+  return below_b & ~below_a;
+}
+__device__ __forceinline__ int lane_rank(uint64_t m) {   // set bits of m below this lane
+  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
 }
 
 // One std::__unguarded_partition_pivot step on [first, last); returns the cut.
+//
+// The j-th left stop L_j (ascending position in [first + 1, last) holding a key <= pivot) is
+// exchanged with the j-th right stop R_j (descending position in [first, last) holding a key >=
+// pivot) while L_j < R_j.  A left stop of rank j at position p is exchanged iff more than j right
+// stops lie above p (R_j > p), a right stop of rank j iff more than j left stops lie below it, so
+// every lane decides from two ranks, with ballots and scalar bit operations only; the exchanged
+// keys meet in LDS at their rank.  The cut is the first left stop not exchanged or the last right
+// stop exchanged, whichever is lower.
 template <int NS>
 __device__ __forceinline__ int wave_partition_pivot(uint32_t (&k)[NS], int32_t (&ix)[NS], int first, int last,
                                     int lane, WaveScratch& ws) {
   const int mid = first + (last - first) / 2;
+  uint32_t piv;
   {
     // __move_median_to_first(first, first + 1, mid, last - 1)
     const int a = first + 1, b = mid, c = last - 1;
@@ -293,78 +306,64 @@ __device__ __forceinline__ int wave_partition_pivot(uint32_t (&k)[NS], int32_t (
     } else {
       m = (ka > kc) ? a : (kb > kc) ? c : b;
     }
-    swap_at(k, ix, first, m, lane);
+    piv = m == a ? ka : (m == b ? kb : kc);
+    const uint32_t kf = key_at(k, first);
+    const int32_t xf = idx_at(ix, first), xm = idx_at(ix, m);
+    set_at(k, ix, m, kf, xf);
+    set_at(k, ix, first, piv, xm);
   }
-  const uint32_t piv = key_at(k, first);
-  // left stops: [first+1, last) with key <= pivot; right stops: [first, last) with key >= pivot
   uint64_t bl[NS], bg[NS];
-  bool le[NS], ge[NS];
+  int ng = 0;
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    const int pos = s * 64 + lane;
-    le[s] = pos > first && pos < last && k[s] <= piv;
-    ge[s] = pos >= first && pos < last && k[s] >= piv;
-    bl[s] = __ballot(le[s]);
-    bg[s] = __ballot(ge[s]);
+    bl[s] = __ballot(k[s] <= piv) & slot_mask(first + 1, last, s);
+    bg[s] = __ballot(k[s] >= piv) & slot_mask(first, last, s);
+    ng += __popcll(bg[s]);
   }
-  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  const uint64_t gt_mask = (lane == 63) ? 0ull : (~0ull << (lane + 1));
-  int nl = 0, ng = 0;
-  int rl[NS], rg[NS];
-  int below_l = 0;
+  uint64_t sl[NS], sr[NS];   // exchanged left / right stops
+  int rank[NS];              // of an exchanged stop, on its side
+  int below_l = 0, below_g = 0;
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    rl[s] = below_l + __popcll(bl[s] & lt_mask);
+    const int left = below_l + lane_rank(bl[s]);              // left stops below
+    const int upto = below_g + lane_rank(bg[s]);              // right stops below
+    const bool le = __builtin_amdgcn_inverse_ballot_w64(bl[s]), ge = __builtin_amdgcn_inverse_ballot_w64(bg[s]);
+    const int right = ng - upto - (ge ? 1 : 0);               // right stops above
+    sl[s] = __ballot(le && right > left);
+    sr[s] = __ballot(ge && left > right);
+    rank[s] = left < right ? left : right;
     below_l += __popcll(bl[s]);
+    below_g += __popcll(bg[s]);
   }
-  nl = below_l;
-  int above_g = 0;
+  int lnext = 0x7fffffff, rprev = 0x7fffffff;
 #pragma unroll
   for (int s = NS - 1; s >= 0; --s) {
-    rg[s] = above_g + __popcll(bg[s] & gt_mask);
-    above_g += __popcll(bg[s]);
+    const uint64_t l = bl[s] & ~sl[s];
+    if (l) lnext = 64 * s + __ffsll((long long)l) - 1;
+    if (sr[s]) rprev = 64 * s + __ffsll((long long)sr[s]) - 1;
   }
-  ng = above_g;
-#pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    const int pos = s * 64 + lane;
-    if (le[s]) ws.lstop[rl[s]] = (int16_t)pos;
-    if (ge[s]) ws.rstop[rg[s]] = (int16_t)pos;
-    if (pos < last) ws.stage[pos] = Pair{k[s], ix[s]};
-  }
-  wave_sync_lds();
-  // number of exchanges: prefix of m with lstop[m] < rstop[m]
-  const int mm = nl < ng ? nl : ng;
-  int nswap = 0;
-#pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    const int m = s * 64 + lane;
-    const bool f = m < mm && ws.lstop[m] < ws.rstop[m];
-    nswap += __popcll(__ballot(f));
-  }
-  int cut;
-  if (nswap == 0) {
-    cut = nl > 0 ? ws.lstop[0] : last - 1;
-  } else {
-    const int lnext = nswap < nl ? ws.lstop[nswap] : 0x7fffffff;
-    const int rprev = ws.rstop[nswap - 1];
-    cut = lnext < rprev ? lnext : rprev;
-  }
+  int cut = lnext < rprev ? lnext : rprev;
   // the median-of-3 pivot guarantees a left stop inside the range, so cut lies in
   // [first + 1, last - 1]; the clamp only keeps indices in range should that ever fail
   cut = cut < first + 1 ? first + 1 : (cut > last - 1 ? last - 1 : cut);
+  if (rprev != 0x7fffffff) {
 #pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    int src = -1;
-    if (le[s] && rl[s] < nswap) src = ws.rstop[rl[s]];
-    else if (ge[s] && rg[s] < nswap) src = ws.lstop[rg[s]];
-    if (src >= 0) {
-      const Pair p = ws.stage[src];
-      k[s] = p.v;
-      ix[s] = p.i;
+    for (int s = 0; s < NS; ++s) {
+      const bool l = __builtin_amdgcn_inverse_ballot_w64(sl[s]), r = __builtin_amdgcn_inverse_ballot_w64(sr[s]);
+      if (l || r) ws.stage[rank[s] + (r ? 32 * NS : 0)] = Pair{k[s], ix[s]};
     }
+    wave_sync_lds();
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const bool l = __builtin_amdgcn_inverse_ballot_w64(sl[s]), r = __builtin_amdgcn_inverse_ballot_w64(sr[s]);
+      if (l || r) {
+        const Pair p = ws.stage[rank[s] + (l ? 32 * NS : 0)];
+        k[s] = p.v;
+        ix[s] = p.i;
+      }
+    }
+    wave_sync_lds();
   }
-  wave_sync_lds();
   return cut;
 }
 
@@ -373,39 +372,28 @@ __device__ __forceinline__ int wave_partition_pivot(uint32_t (&k)[NS], int32_t (
 template <int NS>
 __device__ __forceinline__ void wave_insertion_sort(uint32_t (&k)[NS], int32_t (&ix)[NS], int first, int last,
                                     int lane, WaveScratch& ws) {
-  const int len = last - first;
-  if (len <= 1) return;
-#pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    const int pos = s * 64 + lane;
-    if (pos >= first && pos < last) ws.stage[pos] = Pair{k[s], ix[s]};
-  }
-  wave_sync_lds();
+  if (last - first <= 1) return;
   int dest[NS];
 #pragma unroll
+  for (int s = 0; s < NS; ++s) dest[s] = 0;
+  for (int q = first; q < last; ++q) {
+    const uint32_t kq = key_at(k, q);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) dest[s] += (kq > k[s]) || (kq == k[s] && q < s * 64 + lane);
+  }
+#pragma unroll
   for (int s = 0; s < NS; ++s) {
     const int pos = s * 64 + lane;
-    dest[s] = -1;
-    if (pos >= first && pos < last) {
-      int d = first;
-      for (int q = first; q < last; ++q) {
-        const uint32_t kq = ws.stage[q].v;
-        d += (kq > k[s]) || (kq == k[s] && q < pos);
-      }
-      dest[s] = d;
-    }
+    if (pos >= first && pos < last) ws.stage[dest[s]] = Pair{k[s], ix[s]};
   }
   wave_sync_lds();
 #pragma unroll
-  for (int s = 0; s < NS; ++s)
-    if (dest[s] >= 0) ws.stage[dest[s]] = Pair{k[s], ix[s]};
-  wave_sync_lds();
-#pragma unroll
   for (int s = 0; s < NS; ++s) {
     const int pos = s * 64 + lane;
     if (pos >= first && pos < last) {
-      k[s] = ws.stage[pos].v;
-      ix[s] = ws.stage[pos].i;
+      const Pair p = ws.stage[pos - first];
+      k[s] = p.v;
+      ix[s] = p.i;
     }
   }
   wave_sync_lds();
@@ -446,58 +434,33 @@ __device__ __forceinline__ void insertion_step(uint32_t (&k)[NS], int32_t (&ix)[
   wave_insertion_sort(k, ix, first, last, lane, ws);
 }
 
-// Exact CPU top-k selection of the row (n keys, position p = 64*s + lane); the chosen indices
-// are written to ws.sel[0..k).
+// Exact CPU top-k selection of the row (n keys, position p = 64*s + lane): lane j < kk returns
+// the j-th chosen index.
 template <int NS>
-__device__ __forceinline__ void exact_select(uint32_t (&k)[NS], int32_t (&ix)[NS], int n, int kk, bool sorted,
+__device__ __forceinline__ int exact_select(uint32_t (&k)[NS], int32_t (&ix)[NS], int n, int kk, bool sorted,
                              int lane, WaveScratch& ws) {
-  bool serial = kk * 64 <= n || (sorted && kk - 1 > 16);
-  if (!serial) {
+  const bool partial = kk * 64 <= n;                  // partial_sort regime
+  const bool long_sort = sorted && kk - 1 > 16;       // a final sort longer than 16
+  int first = 0, last = n, depth = lg2_(n) * 2;
+  if (!partial && !long_sort) {
     // std::nth_element(first, first + kk - 1, last)
     const int nth = kk - 1;
-    int first = 0, last = n;
-    int depth = lg2_(n) * 2;
-    if (nth != n) {
-      while (last - first > 3) {
-        if (depth == 0) {
-          serial = true;  // heap select from this state on lane 0
-          break;
-        }
-        --depth;
-        const int cut = partition_step(k, ix, first, last, lane, ws);
-        if (cut <= nth)
-          first = cut;
-        else
-          last = cut;
-      }
-      if (!serial) insertion_step(k, ix, first, last, lane, ws);
+    while (last - first > 3 && depth > 0) {
+      --depth;
+      const int cut = partition_step(k, ix, first, last, lane, ws);
+      if (cut <= nth)
+        first = cut;
+      else
+        last = cut;
     }
-    if (serial) {
-#pragma unroll
-      for (int s = 0; s < NS; ++s) {
-        const int pos = s * 64 + lane;
-        if (pos < n) ws.stage[pos] = Pair{k[s], ix[s]};
-      }
-      wave_sync_lds();
-      if (lane == 0) {
-        heap_select_(ws.stage + first, nth + 1 - first, last - first);
-        swap_(ws.stage, first, nth);
-        if (sorted) sort_(ws.stage, 0, kk - 1, ws.stack);
-        for (int j = 0; j < kk; ++j) ws.sel[j] = ws.stage[j].i;
-      }
-      wave_sync_lds();
-      return;
+    if (last - first <= 3) {
+      insertion_step(k, ix, first, last, lane, ws);
+      if (sorted) insertion_step(k, ix, 0, kk - 1, lane, ws);
+      return ix[0];
     }
-    if (sorted) insertion_step(k, ix, 0, kk - 1, lane, ws);
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      const int pos = s * 64 + lane;
-      if (pos < kk) ws.sel[pos] = ix[s];
-    }
-    wave_sync_lds();
-    return;
   }
-  // partial_sort regime, or a final sort longer than 16: sequential on lane 0
+  // sequential on lane 0, from the state reached: the depth limit's heap select on [first, last),
+  // or the whole of a partial_sort or of a selection with a long final sort
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
     const int pos = s * 64 + lane;
@@ -506,35 +469,31 @@ __device__ __forceinline__ void exact_select(uint32_t (&k)[NS], int32_t (&ix)[NS
   wave_sync_lds();
   if (lane == 0) {
     Pair* a = ws.stage;
-    if (kk * 64 <= n) {
+    const int nth = kk - 1;
+    if (partial) {
       heap_select_(a, kk, n);
       sort_heap_(a, kk);
     } else {
-      int first = 0, last = n, depth = lg2_(n) * 2;
-      const int nth = kk - 1;
-      bool done = false;
-      if (nth != n) {
-        while (last - first > 3) {
-          if (depth == 0) {
-            heap_select_(a + first, nth + 1 - first, last - first);
-            swap_(a, first, nth);
-            done = true;
-            break;
-          }
-          --depth;
-          const int cut = partition_pivot_(a, first, last);
-          if (cut <= nth)
-            first = cut;
-          else
-            last = cut;
-        }
-        if (!done) insertion_sort_(a, first, last);
+      while (last - first > 3 && depth > 0) {
+        --depth;
+        const int cut = partition_pivot_(a, first, last);
+        if (cut <= nth)
+          first = cut;
+        else
+          last = cut;
+      }
+      if (last - first > 3) {
+        heap_select_(a + first, nth + 1 - first, last - first);
+        swap_(a, first, nth);
+      } else {
+        insertion_sort_(a, first, last);
       }
       if (sorted) sort_(a, 0, kk - 1, ws.stack);
     }
     for (int j = 0; j < kk; ++j) ws.sel[j] = a[j].i;
   }
   wave_sync_lds();
+  return ws.sel[lane < kk ? lane : 0];
 }
 
 // Wavefront reductions through DPP lane moves (a few cycles each, against an LDS round trip
@@ -561,17 +520,6 @@ __device__ __forceinline__ float wave_max(float v) {
   v = fmaxf(v, dpp_asf(dpp_u<0x143, 0xc>(u, u)));
   return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), 63));
 }
-__device__ __forceinline__ uint32_t umax_(uint32_t a, uint32_t b) { return a > b ? a : b; }
-__device__ __forceinline__ uint32_t wave_max_u(uint32_t v) {
-  v = umax_(v, dpp_u<0xB1>(v, v));
-  v = umax_(v, dpp_u<0x4E>(v, v));
-  v = umax_(v, dpp_u<0x141>(v, v));
-  v = umax_(v, dpp_u<0x140>(v, v));
-  v = umax_(v, dpp_u<0x142, 0xa>(v, v));
-  v = umax_(v, dpp_u<0x143, 0xc>(v, v));
-  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
-}
-
 // SLEEF's single-precision exp with 1.0-ulp bound (xexpf of SLEEF 3, sleefsimdsp.c; the
 // published Cody-Waite reduction by ln 2 in two parts, a degree-6 polynomial for e^s - 1 - s in
 // Horner form with fused multiply-adds, and a two-step scaling by 2^q).  Restated from that
@@ -729,50 +677,24 @@ __global__ __launch_bounds__(64 * kWaves) void router_kernel(
       key[s] = e < n ? (row_bad ? 0xffffffffu : ordered_key(p)) : 0u;
       ix[s] = e;
     }
-    // fast path: kk arg-max rounds on distinct keys (nth_element regime, sorted output)
-    bool exact = !sorted || row_bad || kk * 64 <= n;
-    if (!exact) {
-      uint32_t cur[NS];
+    const int e = exact_select(key, ix, n, kk, sorted != 0, lane, ws);
+    if (tie_rows) {
+      // rows whose result depends on the algorithm's order: unsorted, NaN and partial_sort rows, and
+      // those with a chosen key that another element has too
+      bool tie = !sorted || row_bad || kk * 64 <= n;
+      for (int j = 0; j < kk && !tie; ++j) {
+        const uint32_t kj = ordered_key(ws.prob[__builtin_amdgcn_readlane(e, j)]);
+        int same = 0;
 #pragma unroll
-      for (int s = 0; s < NS; ++s) cur[s] = (s * 64 + lane < n) ? key[s] : 0u;
-      for (int r = 0; r < kk; ++r) {
-        uint32_t lm = cur[0];
-#pragma unroll
-        for (int s = 1; s < NS; ++s) lm = cur[s] > lm ? cur[s] : lm;
-        const uint32_t best = wave_max_u(lm);
-        int eq = 0, where = 0;
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-          const bool hit = (s * 64 + lane < n) && cur[s] == best;
-          eq += hit;
-          if (hit) where = s * 64 + lane;
-        }
-        const uint64_t hits = __ballot(eq > 0);
-        const int total = __popcll(hits) == 1 ? __builtin_amdgcn_readlane(eq, __ffsll((long long)hits) - 1) : 2;
-        if (total != 1 || best == 0u) {
-          exact = true;  // a tie decides membership or order
-          break;
-        }
-        const int owner = __ffsll((long long)hits) - 1;
-        const int pos = __builtin_amdgcn_readlane(where, owner);
-        if (lane == 0) ws.sel[r] = pos;
-#pragma unroll
-        for (int s = 0; s < NS; ++s) cur[s] = (lane == owner && s == (pos >> 6)) ? 0u : cur[s];
+        for (int s = 0; s < NS; ++s)
+          same += __popcll(__ballot(s * 64 + lane < n && ordered_key(ws.prob[s * 64 + lane]) == kj));
+        tie = same != 1;
       }
-      wave_sync_lds();
-    }
-    if (exact) {
-      exact_select(key, ix, n, kk, sorted != 0, lane, ws);
-      if (lane == 0 && tie_rows) atomicAdd(tie_rows, 1);
+      if (tie && lane == 0) atomicAdd(tie_rows, 1);
     }
     wave_sync_lds();
     // weights: lanes 0..kk-1 each own one selected expert
-    float wv = 0.f;
-    int e = 0;
-    if (lane < kk) {
-      e = ws.sel[lane];
-      wv = ws.prob[e];
-    }
+    const float wv = lane < kk ? ws.prob[e] : 0.f;
     const float tot = renorm ? topk_weight_sum(wv, kk) : 0.f;
     if (lane < kk) {
       float w = renorm ? wv / tot : wv;

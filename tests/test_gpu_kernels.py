@@ -55,6 +55,25 @@ def test_router_sorted_matches_torch_cpu_topk(device, E, k, dtype, ties):
         assert int(counter.item()) > 0, 'the exact tie path was not exercised'
 
 
+@pytest.mark.parametrize('E,k', [(63, 6), (64, 2), (65, 7), (127, 9), (128, 17), (129, 5), (192, 12),
+                                 (255, 8), (256, 17)])
+@pytest.mark.parametrize('sorted_', [False, True])
+@pytest.mark.parametrize('levels', [2, 5, 40])
+def test_router_partition_edges(device, E, k, sorted_, levels):
+    """Expert counts at the edges of the 64-key slots, rows of 2, 5 and 40 distinct logits (the
+    partition's stops then fill whole slots), ascending and descending rows among them: indices and
+    weights equal to torch's CPU topk, bit for bit."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(E * 64 + k)
+    x = torch.randint(levels, (257, E), generator=g).float() / 4
+    x[0] = x[0].sort()[0]
+    x[1] = x[1].sort(descending=True)[0]
+    w, idx = ops.router_topk(x.to(device), k, renorm=sorted_, sorted=sorted_)
+    ref_w, ref_idx, _ = (qwen3_router if sorted_ else deepseek_router)(x, k)
+    assert torch.equal(idx.cpu(), ref_idx)
+    assert torch.equal(w.cpu().view(torch.int16), ref_w.view(torch.int16))
+
+
 @pytest.mark.parametrize('E,k', [(64, 6), (128, 8), (16, 5), (128, 32), (256, 3)])
 @pytest.mark.parametrize('ties', [False, True])
 def test_router_unsorted_deepseek(device, E, k, ties):
