@@ -286,6 +286,28 @@ __global__ __launch_bounds__(kMaxBlock) void layout_scatter(
   }
 }
 
+// starts[0 .. n] from n sizes that come with the launch (no copy from host memory)
+struct Sizes {
+  int32_t v[kMaxE];
+};
+__global__ __launch_bounds__(64) void starts_kernel(Sizes sizes, int n, int64_t* __restrict__ starts) {
+  const int lane = threadIdx.x;
+  int64_t carry = 0;
+  for (int e0 = 0; e0 < n; e0 += 64) {
+    const int e = e0 + lane;
+    const int64_t c = e < n ? sizes.v[e] : 0;
+    int64_t incl = c;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int64_t v = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += v;
+    }
+    if (e < n) starts[e] = carry + incl - c;
+    carry += __shfl(incl, 63, 64);
+  }
+  if (lane == 0) starts[n] = carry;
+}
+
 // The workspace of ferry_layout_noalloc: a file-scope device array instead of caller memory.
 // Each GPU holds its own copy for the life of the process; its device address is looked up
 // once per device (hipGetSymbolAddress) and only that address is handed to kernels.  Nothing in
@@ -399,4 +421,19 @@ extern "C" int ferry_layout_noalloc(const int64_t* selected, const void* weights
   if (rc != 0) return rc;
   return ferry_layout(selected, weights_bf16, tokens, topk, experts, send_ids, w_sorted_bf16,
                       starts, rows, cols, pair_pos, ws, kScratchBytes, stream);
+}
+
+extern "C" int ferry_starts(const int32_t* sizes, int32_t n, int64_t* starts, void* stream) {
+  clear_error();
+  FERRY_CHECK_ARG(n >= 0 && n <= kMaxE, "n must be in [0, %d]", kMaxE);
+  FERRY_CHECK_ARG(starts && (n == 0 || sizes), "null pointer argument");
+  Sizes s;
+  for (int i = 0; i < n; ++i) {
+    FERRY_CHECK_ARG(sizes[i] >= 0, "sizes[%d] = %d is negative", i, sizes[i]);
+    s.v[i] = sizes[i];
+  }
+  for (int i = n; i < kMaxE; ++i) s.v[i] = 0;
+  launch("starts_kernel", starts_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, s, (int)n, starts);
+  FERRY_LAUNCHED("starts_kernel");
+  return 0;
 }

@@ -149,11 +149,35 @@ def layout(selected, weights, experts, out=None, check=False):
         lay.rows.data_ptr(), lay.cols.data_ptr(), lay.pair_pos.data_ptr(),
         lay.workspace.data_ptr(), lay.workspace.numel(), current_stream(dev)), 'layout')
     if check:
-        bad = layout_errors(lay)
-        if bad:
-            raise RuntimeError(f'layout: {bad} token(s) with an expert ID out of [0, {experts}) '
-                               'or repeated')
+        _raise_bad_tokens(layout_errors(lay), experts)
     return lay
+
+
+def layout_on_host(selected, weights, experts):
+    """``layout(..., check=True)`` and its ``starts`` on the host (int64 numpy [experts + 1]), read
+    back in one copy with the count of invalid tokens."""
+    T, k = selected.shape
+    dev = selected.device
+    head = -(-(experts + 1) * 8 // 256) * 256
+    buf = torch.empty(head + layout_workspace_bytes(T, k, experts), dtype=torch.uint8, device=dev)
+    lay = Layout()
+    lay.send_ids = torch.empty((T, k), dtype=torch.int64, device=dev)
+    lay.w_sorted = torch.empty((T, k), dtype=torch.bfloat16, device=dev)
+    lay.starts = buf[:(experts + 1) * 8].view(torch.int64)
+    lay.rows = torch.empty(T * k, dtype=torch.int64, device=dev)
+    lay.cols = torch.empty(T * k, dtype=torch.int64, device=dev)
+    lay.pair_pos = torch.empty(T * k, dtype=torch.int32, device=dev)
+    lay.workspace = buf[head:]
+    layout(selected, weights, experts, out=lay)
+    host = buf[:head + 4].cpu().numpy()
+    _raise_bad_tokens(int(host[head:].view(np.int32)[0]), experts)
+    return lay, host[:(experts + 1) * 8].view(np.int64)
+
+
+def _raise_bad_tokens(bad, experts):
+    if bad:
+        raise RuntimeError(f'layout: {bad} token(s) with an expert ID out of [0, {experts}) '
+                           'or repeated')
 
 
 PHASE_UP, PHASE_DOWN, PHASE_BOTH = 1, 2, 3
@@ -170,6 +194,7 @@ def expert_ffn(cache, x, w_sorted, starts, rows, cols, expert_list, slot_of, hid
     the row count of every expert, ``starts[e+1] - starts[e]``: the library then issues the
     experts with at most 64 rows (small-expert kernels, 17-64 rows first) and the larger ones
     (tiled kernels) as separate launches with exact row bounds, and skips experts without rows.
+    ``rows`` and ``cols`` are CUDA tensors or raw device addresses (ints).
     """
     R, k = w_sorted.shape
     el = np.ascontiguousarray(expert_list, dtype=np.int32)
@@ -177,8 +202,9 @@ def expert_ffn(cache, x, w_sorted, starts, rows, cols, expert_list, slot_of, hid
     E = int(experts if experts is not None else len(so))
     args = (_dev(cache, 'cache', torch.bfloat16), cache.shape[0], hidden, intermediate,
             _dev(x, 'x', torch.bfloat16), R, k, _dev(w_sorted, 'w_sorted', torch.bfloat16),
-            _dev(starts, 'starts', torch.int64), _dev(rows, 'rows', torch.int64),
-            _dev(cols, 'cols', torch.int64))
+            _dev(starts, 'starts', torch.int64),
+            rows if isinstance(rows, int) else _dev(rows, 'rows', torch.int64),
+            cols if isinstance(cols, int) else _dev(cols, 'cols', torch.int64))
     tail = (_dev(act, 'act', torch.bfloat16), _dev(out, 'out', torch.bfloat16), int(out_mode),
             int(phases), current_stream(x.device))
 
@@ -327,6 +353,27 @@ def history_ready_words(tokens, topk):
 # The reference's pybind names (ferry/csrc/expert_ops.cpp:144-157)
 # ------------------------------------------------------------------------------------------
 
+def _joined(tensors, dtype, device):
+    """(address, elements, owner) of the tensors one after the other, as ``dtype``: in place where
+    they already follow each other in memory (views that split one tensor), else concatenated.
+    ``owner`` keeps the memory alive."""
+    index, size = device.index, dtype.itemsize
+    start = end = None
+    for t in tensors:
+        n = t.numel()
+        if n == 0:
+            continue
+        at = t.data_ptr()
+        if start is None:
+            start = end = at
+        if at != end or t.dtype is not dtype or t.get_device() != index or not t.is_contiguous():
+            cat = torch.cat([u.reshape(-1) for u in tensors]).to(dtype).contiguous()
+            _dev(cat, 'tensors of a group list')
+            return cat.data_ptr(), cat.numel(), cat
+        end += n * size
+    return (0, 0, None) if start is None else (start, (end - start) // size, tensors)
+
+
 def execute_experts(cache, input, routing_weights, slots, rows, cols, hidden, intermediate):
     """Routed-expert MLPs of every (slot, rows, cols) group (expert_ops.cpp:16-45).
 
@@ -347,20 +394,24 @@ def execute_experts(cache, input, routing_weights, slots, rows, cols, hidden, in
         return []
     if G > MAX_EXPERTS:
         raise RuntimeError(f'at most {MAX_EXPERTS} groups per call')
-    for s in slots:
-        if not 0 <= int(s) < cache.shape[0]:
-            raise RuntimeError('slot out of range')
-    sizes = [int(r.numel()) for r in rows]
+    slots = np.asarray(slots, np.int64)
+    if slots.min() < 0 or slots.max() >= cache.shape[0]:
+        raise RuntimeError('slot out of range')
+    sizes = [r.numel() for r in rows]
     dev = input.device
-    starts = torch.tensor(np.concatenate([[0], np.cumsum(sizes)]), dtype=torch.int64, device=dev)
-    rows_cat = torch.cat([r.reshape(-1) for r in rows]).to(torch.int64).contiguous()
-    cols_cat = torch.cat([c.reshape(-1) for c in cols]).to(torch.int64).contiguous()
-    P = int(sum(sizes))
+    rows_at, P, _rows = _joined(rows, torch.int64, dev)
+    cols_at, n_cols, _cols = _joined(cols, torch.int64, dev)
+    if n_cols < P:
+        raise RuntimeError('cols must name a weight for every row')
+    starts = torch.empty(G + 1, dtype=torch.int64, device=dev)
+    counts = np.array(sizes, np.int32)
+    check(lib().ferry_starts(counts.ctypes.data, G, starts.data_ptr(), current_stream(dev)), 'starts')
     act = torch.empty((max(P, 1), intermediate), dtype=torch.bfloat16, device=dev)
     out = torch.empty((max(P, 1), hidden), dtype=torch.bfloat16, device=dev)
-    expert_ffn(cache, input.contiguous(), routing_weights.contiguous(), starts, rows_cat, cols_cat,
-               np.arange(G), np.asarray(slots, np.int32), hidden, intermediate, act, out,
-               out_mode=1, experts=G, counts=sizes)
+    if P:
+        expert_ffn(cache, input.contiguous(), routing_weights.contiguous(), starts, rows_at, cols_at,
+                   np.arange(G), slots, hidden, intermediate, act, out, out_mode=1, experts=G,
+                   counts=counts)
     return list(out[:P].split(sizes))
 
 
@@ -385,7 +436,7 @@ def pack_dispatch(hidden, selected, weights, send_idx, send_ids, experts):
 
 def unpack_dispatch(raw, hidden, topk):
     """Split packet rows back into bf16 [m, H] hidden states and [m, k] weights
-    (expert_ops.cpp:106-111), as two strided device copies."""
+    (expert_ops.cpp:106-111), on the ``ferry_unpack_dispatch`` kernel."""
     m = raw.shape[0]
     if raw.dim() != 2 or raw.shape[1] != 2 * hidden + 3 * topk:
         raise RuntimeError('raw must be uint8 [m, 2 * hidden + 3 * topk]')
@@ -401,17 +452,26 @@ def reduce_partials(parts, rows, received, hidden, like):
     """fp32 sum of expert outputs per received row, ascending group order, then bf16 (:76-83)."""
     if len(parts) == 0:
         return torch.zeros((received, hidden), dtype=torch.bfloat16, device=like.device)
-    part = torch.cat([p.reshape(-1, hidden) for p in parts]).to(torch.bfloat16).contiguous()
-    rows_cat = torch.cat([r.reshape(-1) for r in rows]).to(torch.int64)
-    # the j-th occurrence (in group order) of each row is its j-th term
-    order = torch.argsort(rows_cat, stable=True)
-    counts = torch.bincount(rows_cat, minlength=received)
-    k = max(int(counts.max().item()) if counts.numel() else 1, 1)
-    first = torch.cumsum(counts, 0) - counts
-    rank = torch.arange(order.numel(), device=like.device) - first[rows_cat[order]]
-    pair_pos = torch.full((received * k,), -1, dtype=torch.int32, device=like.device)
-    pair_pos[rows_cat[order] * k + rank] = order.to(torch.int32)
-    return combine(part, received, k, hidden, pair_pos=pair_pos)
+    dev = parts[0].device
+    part_at, n, _parts = _joined(parts, torch.bfloat16, dev)
+    if part_at % 16:
+        _parts = torch.cat([p.reshape(-1) for p in parts])
+        part_at = _parts.data_ptr()
+    if n % hidden:
+        raise RuntimeError('parts must hold rows of hidden elements')
+    rows_at, entries, _rows = _joined(rows, torch.int64, dev)
+    if entries > n // hidden:
+        raise RuntimeError('rows must not outnumber the rows of parts')
+    out = torch.empty((received, hidden), dtype=torch.bfloat16, device=dev)
+    ws = torch.empty(int(lib().ferry_reduce_rows_workspace_bytes(received)) // 4, dtype=torch.int32,
+                     device=dev)
+    check(lib().ferry_reduce_rows(part_at, entries, hidden, rows_at, received, out.data_ptr(),
+                                  ws.data_ptr(), ws.numel() * 4, current_stream(dev)),
+          'reduce_partials')
+    bad = int(ws[received].item())
+    if bad:
+        raise RuntimeError(f'reduce_partials: {bad} row(s) outside [0, {received})')
+    return out
 
 
 def scatter_returned(returned, send_idx, tokens):

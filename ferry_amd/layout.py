@@ -29,13 +29,12 @@ def device_layout(selected, destinations, tokens_per_rank, rank, experts, slot_o
         raise NotImplementedError('ferry_amd runs on one GPU (world = 1)')
     if destinations is not None and np.any(np.asarray(destinations) != 0):
         raise AssertionError('expert scheduled on this rank is not cached here')
-    lay = ops.layout(sel, weights, experts, check=True)   # the reference's index checks
-    starts = lay.starts.cpu().numpy()
-    groups = []
-    for e in np.flatnonzero(starts[1:] > starts[:-1]):
-        slot = int(slot_of[e])
-        assert slot >= 0, 'expert scheduled on this rank is not cached here'
-        a, b = int(starts[e]), int(starts[e + 1])
-        groups.append((int(e), lay.rows[a:b], lay.cols[a:b], slot))
+    lay, starts = ops.layout_on_host(sel, weights, experts)   # the reference's index checks
+    sizes = np.diff(starts)
+    active = np.flatnonzero(sizes)
+    slots = np.asarray(slot_of)[active]
+    assert np.all(slots >= 0), 'expert scheduled on this rank is not cached here'
+    split = sizes[active].tolist()
+    groups = list(zip(active.tolist(), lay.rows.split(split), lay.cols.split(split), slots.tolist()))
     return dict(send_idx=torch.arange(T, device='cuda'), send_ids=lay.send_ids,
                 send_counts=[T], recv_counts=[T], groups=groups, layout=lay)

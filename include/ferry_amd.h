@@ -103,6 +103,11 @@ int ferry_layout_noalloc(const int64_t* selected, const void* weights_bf16, int6
                          int64_t* starts, int64_t* rows, int64_t* cols, int32_t* pair_pos,
                          void* stream);
 
+/* starts[0 .. n] (int64, device memory) = exclusive prefix of the n <= FERRY_MAX_EXPERTS group sizes
+ * (host memory, read before the call returns): the starts argument of ferry_expert_ffn for groups
+ * that the host forms (execute_experts, ferry/csrc/expert_ops.cpp:13-45), without a copy. */
+int ferry_starts(const int32_t* sizes, int32_t n, int64_t* starts, void* stream);
+
 /*
  * Grouped SwiGLU over resident cache slots.  Replaces ferry/csrc/expert_ops.cpp:13-45
  * (execute_experts: per expert x = in[rows]; g = x Wg^T; u = x Wu^T; a = silu(g) * u;
@@ -172,6 +177,20 @@ int ferry_combine(const void* part, const int32_t* pair_pos, int64_t tokens, int
  */
 int ferry_combine_add(const void* part, const int32_t* pair_pos, int64_t tokens, int64_t topk,
                       int64_t hidden, const void* addend, void* out, void* stream);
+
+/*
+ * reduce_partials on expert outputs in any order: out[r, :] = bf16( sum over the entries p with
+ * row_of[p] == r of fp32(part[p, :]) ), p ascending, 0 for a row without entries.
+ * Replaces ferry/csrc/expert_ops.cpp:75-83 (fp32 index_add_ of every group's rows in group order,
+ * then bf16).  part is bf16 [entries, hidden], row_of int64 [entries], out bf16 [rows, hidden].
+ * After the call int32 word `rows` of `workspace` (device memory, at least
+ * ferry_reduce_rows_workspace_bytes(rows) bytes) holds the number of entries whose row lies outside
+ * [0, rows) (they are left out), for the caller to read when it wants the check.
+ */
+int64_t ferry_reduce_rows_workspace_bytes(int64_t rows);
+int ferry_reduce_rows(const void* part, int64_t entries, int64_t hidden, const int64_t* row_of,
+                      int64_t rows, void* out, void* workspace, int64_t workspace_bytes,
+                      void* stream);
 
 /*
  * Dispatch packets (the reference's exchange format).  Replaces ferry/csrc/expert_ops.cpp:88-104

@@ -173,3 +173,86 @@ def test_dispatch_combine_steps_bit_exact(device, T, E, k, H, I):
     assert torch.equal(back, partial)   # world = 1: an fp32 round trip of every row
     oracle = moe_layer_ref(lambda e: rows_w[e], x, sel, w, E, H, I)
     torch.testing.assert_close(back.cpu().float(), oracle.float(), rtol=2e-2, atol=1e-2)
+
+
+@pytest.mark.parametrize('T,H,k', [(3, 64, 1), (5, 256, 2), (7, 256, 3), (65, 512, 4), (9, 2048, 6),
+                                   (33, 2048, 8), (4, 20, 5)])
+def test_packets_of_every_alignment(device, T, H, k):
+    """Packet pitches 2H + 3k that are odd and multiples of 2, 4, 8 and 16, a payload that starts at
+    an odd address, hidden rows that are no multiple of 16 bytes: packets bit-equal to the closed
+    form, and split back into the same rows and weights."""
+    from ferry_amd import expert_ops as ops
+    from ferry_amd._lib import last_error, lib
+    rng = np.random.default_rng(T * H + k)
+    E = 4 * k
+    sel, w = _routing(T, E, k, E, rng)
+    x = torch.randn((T, H), generator=torch.Generator().manual_seed(k)).to(torch.bfloat16)
+    ref = layout_closed_form(sel.numpy(), E, w.view(torch.int16).numpy())
+    want = torch.from_numpy(packets_closed_form(x, ref['send_ids'], ref['w_sorted']))
+    xd, seld, wd = x.to(device), sel.to(device), w.to(device)
+    idx, ids = torch.arange(T, device=device), torch.from_numpy(ref['send_ids']).to(device)
+    payload = ops.pack_dispatch(xd, seld, wd, idx, ids, E)
+    assert torch.equal(payload.cpu(), want)
+    pitch = 2 * H + 3 * k
+    flat = torch.full((T * pitch + 1,), 77, dtype=torch.uint8, device=device)
+    stream = torch.cuda.current_stream().cuda_stream
+    assert lib().ferry_pack_dispatch(xd.data_ptr(), T, H, seld.data_ptr(), wd.data_ptr(), k, idx.data_ptr(),
+                                     ids.data_ptr(), T, k, E, flat[1:].data_ptr(), stream) == 0, last_error()
+    assert torch.equal(flat[1:].view(T, pitch).cpu(), want) and int(flat[0]) == 77
+    for raw in (payload, flat[1:].view(T, pitch)):
+        hx, hw = ops.unpack_dispatch(raw, H, k)
+        ux, uw = unpack_dispatch_ref(want, H, k)
+        assert torch.equal(hx.cpu(), ux) and torch.equal(hw.cpu().view(torch.int16), uw.view(torch.int16))
+
+
+@pytest.mark.parametrize('sizes,received,H', [([1], 1, 8), ([5, 0, 3, 7], 6, 64), ([40, 40, 40], 3, 2056),
+                                              ([300] * 20, 300, 256), ([16] * 17, 16, 4096)])
+@pytest.mark.parametrize('adjacent', [True, False])
+def test_reduce_partials_any_rows(device, sizes, received, H, adjacent):
+    """Rows in any order, repeated within a group, up to 16 and more entries a row, rows without
+    entries, parts and rows that split one tensor and that do not: bit-equal to the fp32 sums in
+    group order."""
+    from ferry_amd import expert_ops as ops
+    rng = np.random.default_rng(sum(sizes) + received)
+    rows = [torch.from_numpy(rng.integers(0, received, n)) for n in sizes]
+    if len(sizes) == 17:
+        rows = [torch.randperm(16) for _ in sizes]     # 17 entries in every row
+    g = torch.Generator().manual_seed(H)
+    parts = [torch.randn((n, H), generator=g).to(torch.bfloat16) for n in sizes]
+    want = reduce_partials_ref(parts, rows, received, H)
+    if adjacent:
+        dp = torch.cat(parts).to(device).split(sizes)
+        dr = torch.cat(rows).to(device).split(sizes)
+    else:
+        dp, dr = [p.to(device) for p in parts], [r.to(device) for r in rows]
+    got = ops.reduce_partials(list(dp), list(dr), received, H, dp[0])
+    assert torch.equal(got.cpu().view(torch.int16), want.view(torch.int16))
+    for bad in (-1, received):
+        r0 = dr[0].clone()
+        r0[0] = bad
+        with pytest.raises(RuntimeError):
+            ops.reduce_partials(list(dp), [r0] + list(dr[1:]), received, H, dp[0])
+
+
+def test_execute_experts_row_lists(device):
+    """Row and column lists that split one tensor and that do not give the same bits, empty groups
+    included; int32 lists are taken as before; a list on the host is refused."""
+    from ferry_amd import expert_ops as ops
+    H, I, T, sizes = 256, 128, 90, [3, 0, 20, 70, 1]
+    g = torch.Generator().manual_seed(4)
+    cache = (torch.randn((6, 3 * H * I), generator=g) * 0.05).to(torch.bfloat16).to(device)
+    x = torch.randn((T, H), generator=g).to(torch.bfloat16).to(device)
+    w = torch.rand((T, 2), generator=g).to(torch.bfloat16).to(device)
+    rows = torch.randint(T, (sum(sizes),), generator=g).to(device)
+    cols = torch.randint(2, (sum(sizes),), generator=g).to(device)
+    slots = [5, 1, 0, 2, 3]
+    base = ops.execute_experts(cache, x, w, slots, rows.split(sizes), cols.split(sizes), H, I)
+    assert [tuple(b.shape) for b in base] == [(n, H) for n in sizes]
+    for f in (torch.clone, lambda t: t.to(torch.int32)):
+        other = ops.execute_experts(cache, x, w, slots, [f(t) for t in rows.split(sizes)],
+                                    [f(t) for t in cols.split(sizes)], H, I)
+        assert all(torch.equal(a, b) for a, b in zip(base, other))
+    with pytest.raises(RuntimeError):
+        ops.execute_experts(cache, x, w, slots, [t.cpu() for t in rows.split(sizes)], cols.split(sizes), H, I)
+    with pytest.raises(RuntimeError):
+        ops.execute_experts(cache, x, w, [6, 1, 0, 2, 3], rows.split(sizes), cols.split(sizes), H, I)
