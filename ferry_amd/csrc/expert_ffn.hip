@@ -822,6 +822,93 @@ __device__ __forceinline__ void down_skinny_p(const FfnArgs& a, int li, int64_t 
   }
 }
 
+// Phase 2, skinny, short lists: one workgroup = (expert, 16 hidden rows), K split over the four
+// wavefronts as in down_skinny, walked in chunks of 64 elements (up to NC each).  With 64 hidden rows a workgroup, a list of one
+// to eight experts starts 32 to 256 workgroups, each a chain of load latencies over its K range; here
+// a wavefront loads all of its weights at once, before the workgroup waits for the activation rows
+// (which they do not depend on), and what is left after the wait is one load of the rows and the
+// products.  The weights go through the wavefront's 2 KiB LDS tile (16 rows x 128 B) as in
+// down_skinny_t.  load() takes the weights, the output rows and the routing weights, finish() the rest.
+template <int NC, bool COH>
+struct DownRows16 {
+  bf16x8 w[2 * NC];
+  int k0, ns;           // first element, 32-element steps (an odd count ends with half a chunk)
+  int32_t lane_orow;    // of the expert's row lane % 16
+  float lane_wt;
+  __device__ __forceinline__ void load(const FfnArgs& a, int li, int64_t start, int n, int bx) {
+    const int lane = threadIdx.x & 63, ks = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int steps = (int)a.I / 32, s0 = ks * steps / 4;
+    k0 = 32 * s0;
+    ns = (ks + 1) * steps / 4 - s0;
+    const char* wd = reinterpret_cast<const char*>(
+        uniform_ptr(a.cache + (int64_t)a.list.slot[li] * 3 * a.H * a.I + 2 * a.H * a.I +
+                    (int64_t)bx * 16 * a.I + k0));
+    const uint32_t r8 = (uint32_t)((lane >> 3) * (int)a.I * 2), half = (uint32_t)(16 * a.I);
+    const uint32_t row = r8 + (lane & 7) * 16, row_half = r8 + (lane & 3) * 16;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      // the second half of a half chunk is its first again, a chunk past the last the first half
+      // chunk: no load leaves the wavefront's range
+      const char* b = wd + (2 * c < ns ? 128 * c : 0);
+      const uint32_t at = 2 * c + 1 < ns ? row : row_half;
+      w[2 * c] = *reinterpret_cast<const bf16x8*>(b + at);
+      w[2 * c + 1] = *reinterpret_cast<const bf16x8*>(b + at + half);
+    }
+    const int64_t p = start + ((lane & 15) < n ? lane & 15 : 0);
+    const int64_t tj = a.rows[p] * a.k + a.cols[p];
+    lane_wt = bf16_to_f32(a.w[tj]);
+    lane_orow = a.out_mode == 0 ? (int32_t)tj : (int32_t)p;
+    // all landed here: not sunk below the wait
+#pragma unroll
+    for (int c = 0; c < 2 * NC; ++c) asm volatile("" : "+v"(w[c]));
+    asm volatile("" : "+v"(lane_wt), "+v"(lane_orow));
+  }
+  __device__ __forceinline__ void finish(const FfnArgs& a, int64_t start, int n, int bx, floatx4* red,
+                                         char* tile) {
+    const int lane = threadIdx.x & 63, ks = threadIdx.x >> 6;
+    const int lr = lane >> 3, lc = lane & 7, r16 = lane & 15, kg = (lane >> 4) * 8;
+    const bool ok = r16 < n;
+    // 16-byte loads through a buffer descriptor of the expert's activation rows, agent-coherent
+    // (sc1) under COH; steps past the wavefront's last load what it does not use, or zero past the rows
+    const auto rows = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<bf16_t*>(uniform_ptr(a.act + start * a.I)), 0, (int)(n * a.I * 2), 0x00020000);
+    const int off = ((ok ? r16 : 0) * (int)a.I + k0 + kg) * 2;
+    bf16x8 xa[2 * NC];
+#pragma unroll
+    for (int st = 0; st < 2 * NC; ++st)
+      xa[st] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rows, off + 64 * st, 0, COH ? 16 : 0));
+    const bf16x8 zero8 = {};
+    floatx4 acc[1][1] = {{floatx4{0, 0, 0, 0}}};
+    uint32_t woff[2], roff[2];
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const int row = 8 * g + lr;
+      woff[g] = (uint32_t)(row * 128 + ((lc ^ ((row >> 1) & 7)) << 4));
+      roff[g] = (uint32_t)(r16 * 128 + (((4 * g + (lane >> 4)) ^ ((r16 >> 1) & 7)) << 4));
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+      if (2 * c < ns) {
+#pragma unroll
+        for (int g = 0; g < 2; ++g) *reinterpret_cast<bf16x8*>(tile + woff[g]) = w[2 * c + g];
+#pragma unroll
+        for (int st = 0; st < 2; ++st)
+          if (2 * c + st < ns) {
+            const bf16x8 b = *reinterpret_cast<const bf16x8*>(tile + roff[st]);
+            acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ok ? xa[2 * c + st] : zero8, b, acc[0][0], 0, 0, 0);
+          }
+      }
+    if (!skinny_reduce<4, 1>(acc, ks, 0, lane, red)) return;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int r = (lane >> 4) * 4 + q;
+      const int64_t orow = __shfl(lane_orow, r);
+      const float wt = __shfl(lane_wt, r);
+      if (r < n) a.out[orow * a.H + bx * 16 + (lane & 15)] = f32_to_bf16(bf16r(acc[0][0][q]) * wt);
+    }
+  }
+};
+
 // =============================================================================================
 // Mid kernels
 // =============================================================================================
@@ -1119,7 +1206,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void f
 // of kSyncSets sets (set = epoch % kSyncSets); calls that run at the same time on one GPU use
 // different sets unless kSyncSets of them overlap.
 constexpr int kSyncSets = 8;
-constexpr int kMaxUpWgs = 128;   // up workgroups per expert (I / 16): I <= 2048
+constexpr int kMaxUpWgs = 256;   // up workgroups per expert (I / 16): I <= 4096
 constexpr int kSyncSpinLimit = 1 << 21;
 static __device__ __align__(256) uint32_t g_sync[kSyncSets][kListMax][kMaxUpWgs];
 static __device__ int32_t g_sync_timeouts;
@@ -1129,7 +1216,7 @@ struct FusedSync {
   int32_t* timeouts;
   uint32_t epoch;
   int32_t up_wgs;    // up workgroups per expert (I / 16)
-  int32_t down_wgs;  // down workgroups per expert (H / 64)
+  int32_t down_wgs;  // down workgroups per expert (H / 64, or H / 16 with DownRows16)
   int32_t spin_limit;  // polls before a down workgroup gives up (0: gives up at once)
 };
 
@@ -1156,7 +1243,8 @@ __device__ __forceinline__ bool sync_wait(const FusedSync& fs, int li) {
   }
 }
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void ffn_skinny_fused(
+template <int NC>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NC > 6 ? 2 : (NC > 3 ? 3 : 4)))) void ffn_skinny_fused(
     FfnArgs a, FusedSync fs) {
   // phase 2's K-reduction buffer (16 KiB; phase 1 uses 8) and four 4 KiB weight tiles
   __shared__ __attribute__((aligned(1024))) char sm[16384 + 4 * 4096];
@@ -1185,12 +1273,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void f
     if (threadIdx.x == 0) sync_arrive(fs, li, bx);
     return;
   }
-  if (threadIdx.x < 64) {
-    const bool ok = sync_wait(fs, li);
-    if (threadIdx.x == 0) ok_s = ok ? 1 : 0;
+  auto wait = [&]() {
+    if (threadIdx.x < 64) {
+      const bool ok = sync_wait(fs, li);
+      if (threadIdx.x == 0) ok_s = ok ? 1 : 0;
+    }
+    __syncthreads();
+    return ok_s != 0;
+  };
+  if constexpr (NC > 0) {
+    DownRows16<NC, true> d;
+    d.load(a, li, start, n, bx);
+    if (!wait()) return;
+    d.finish(a, start, n, bx, reinterpret_cast<floatx4*>(sm), sm + 16384 + (threadIdx.x >> 6) * 4096);
+    return;
   }
-  __syncthreads();
-  if (!ok_s) return;
+  if (!wait()) return;
   if (a.I == 768)
     down_skinny_p<3, true>(a, li, start, n, bx, reinterpret_cast<floatx4*>(sm),
                      sm + 16384 + (threadIdx.x >> 6) * 4096);
@@ -2103,9 +2201,20 @@ static int ffn_launch_list(FfnArgs& args, const int32_t* expert_list, const int3
       fs.epoch = epoch;
       fs.flags = sync + (int64_t)(epoch % kSyncSets) * kListMax * kMaxUpWgs;
       fs.up_wgs = (int32_t)(inter / 16);
-      fs.down_wgs = (int32_t)(hidden / 64);
       fs.spin_limit = g_spin_limit.load();
-      launch("ffn_skinny_fused", ffn_skinny_fused,
+      // Down workgroups of 16 hidden rows where those of 64 would leave CUs idle: up to one a CU, or
+      // an eighth of that where a wavefront's K range is three chunks (they pay only for the
+      // launch's emptiest CUs: the activation rows are read by four times as many workgroups).  us
+      // for 16 rows an expert, 64 -> 16 hidden rows a workgroup: H x I = 2048 x 1408, 1 expert 19.7
+      // -> 13.5, 3 experts 26.0 -> 21.1, 8 experts 36.2 -> 33.1; 2048 x 768, 1 expert 12.6 -> 11.3,
+      // 3 experts 14.6 -> 14.5, 6 experts 20.5 -> 22.6; the 2048 x 2816 shared expert, in two
+      // launches before, 17.7 + a launch gap -> 16.3 (1 row: 18.4 -> 13.3).
+      const int64_t chunks = ceil_div(ceil_div(inter / 32, 4), 2);   // of 64 columns, per wavefront
+      const bool narrow = cnt * (hidden / 64) <= (chunks <= 3 ? grid_cap / 8 : grid_cap) && chunks <= 11;
+      fs.down_wgs = (int32_t)(hidden / (narrow ? 16 : 64));
+      launch("ffn_skinny_fused",
+             !narrow ? ffn_skinny_fused<0>
+                     : (chunks <= 3 ? ffn_skinny_fused<3> : (chunks <= 6 ? ffn_skinny_fused<6> : ffn_skinny_fused<11>)),
              dim3((unsigned)((fs.up_wgs + fs.down_wgs) * cnt)), dim3(256), 0, s, args, fs);
       FERRY_LAUNCHED("ffn_skinny_fused");
       continue;

@@ -504,6 +504,39 @@ def test_tiled_kernels_tile_shapes_bit_identical(device, E, n):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))
 
 
+@pytest.mark.parametrize('H,I,counts', [
+    # one-launch decode with down workgroups of 16 hidden rows: K ranges of 1, 3 (odd), 6, 11 (odd), 12
+    # and 22 steps a wavefront, one and several experts, an expert without rows
+    (256, 128, [16]), (256, 384, [1, 0, 16]), (2048, 768, [7]), (512, 1408, [1, 16, 5, 2, 9, 3, 4, 16]),
+    (256, 1536, [3, 8]), (256, 2816, [16, 1]),
+    # ... and of 64: more workgroups than that, and the longest K range
+    (2048, 768, [2] * 9), (256, 4096, [16]), (256, 3072, [5]),
+])
+def test_one_launch_decode_bit_identical(device, H, I, counts):
+    """Both phases in one launch give the bits of the two launches, for every split of the down
+    projection; the rows after the last expert's stay as they were."""
+    ops = _ops()
+    E, P = len(counts), sum(counts)
+    cache = _pool(E, H, I, seed=H + I).to(device)
+    g = torch.Generator().manual_seed(P)
+    x = torch.randn((P, H), generator=g).to(torch.bfloat16).to(device)
+    w = (torch.rand((P, 1), generator=g) + 0.5).to(torch.bfloat16).to(device)
+    starts = torch.tensor(np.concatenate([[0], np.cumsum(counts)]), device=device)
+    rows, cols = torch.randperm(P, generator=g).to(device), torch.zeros(P, dtype=torch.int64, device=device)
+    outs = []
+    for phases in ((ops.PHASE_BOTH,), (ops.PHASE_UP, ops.PHASE_DOWN)):
+        act = torch.full((P + 1, I), float('nan'), dtype=torch.bfloat16, device=device)
+        out = torch.full((P + 1, H), float('nan'), dtype=torch.bfloat16, device=device)
+        for ph in phases:
+            ops.expert_ffn(cache, x, w, starts, rows, cols, np.arange(E), np.arange(E, dtype=np.int32), H, I,
+                           act, out, out_mode=1, experts=E, counts=counts, phases=ph)
+        outs.append((act.cpu(), out.cpu()))
+    assert ops.ffn_sync_timeouts() == 0
+    for a, b in zip(*outs):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+        assert not torch.isnan(a[:P].float()).any() and torch.isnan(a[P].float()).all()
+
+
 def _list_rows_counts_400():
     # 400 experts: the small ones fill more than one launch's list of 256, and the 17-64-row
     # experts (issued first) outnumber it, so the split falls among them
