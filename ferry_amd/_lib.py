@@ -42,11 +42,17 @@ SIGNATURES = [
     ('ferry_history_update', ctypes.c_int,
      [_c_p, _i64, _i64, _i64, _i64, _i64, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _i32, _c_p]),
     ('ferry_history_ready_words', _i64, [_i64, _i64]),
+    ('ferry_history_count', ctypes.c_int,
+     [_c_p, _i64, _i64, _i64, _i64, _i64, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _i32, _c_p]),
+    ('ferry_history_count_blocks', _i64, [_i64]),
+    ('ferry_history_count_words', _i64, [_i64]),
     ('ferry_plan_layer', _i64,
      [_i64, _i64, _c_p, _i64, _i64, _c_p, _c_p, _i64, _c_p, _c_p, _c_p, _i64, _c_p, _c_p]),
     ('ferry_plan_fetch', _i64,
      [_i64, _i64, _c_p, _i64, _i64, _c_p, _c_p, _i64, _c_p, _c_p, _c_p, _i64, _c_p, _c_p, _c_p,
       _c_p]),
+    ('ferry_plan_fetch_counts', _i64,
+     [_i64, _i64, _c_p, _i64, _c_p, _c_p, _i64, _c_p, _c_p, _c_p, _i64, _c_p, _c_p, _c_p]),
     ('ferry_choose_slot', _i64, [_i64, _c_p, _c_p, _i64, _c_p, _c_p, _i64]),
     ('ferry_layer_slots', None, [_c_p, _i64, _i64, _i64, _c_p]),
     ('ferry_h2d_create', ctypes.c_int, [_c_p, _i64, _c_p, _i64, _i64, _i32, ctypes.POINTER(_c_p)]),

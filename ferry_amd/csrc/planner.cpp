@@ -8,8 +8,10 @@
 // (fp32 score of the key's own layer, last-use tick, key) over slots that do not hold an
 // expert the current layer needs; the first empty slot wins outright.  ferry_choose_slot is
 // that rule for one miss; a layer call applies it to all of its misses through one partial
-// sort of the slots (the same choices, see plan_core).  The call's routing IDs are scanned
-// once, which validates them and counts each expert's demand (returned by ferry_plan_fetch).
+// sort of the slots (the same choices, see plan_demand).  The call's routing IDs are scanned
+// once, which validates them and counts each expert's demand (returned by ferry_plan_fetch); of a
+// large call the device does both (ferry_history_count) and the planner sums its records: the scan
+// of 65,536 tokens x 6 IDs took 348 us, of 8192 x 8 about 60 us, with the GPU waiting.
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
@@ -17,6 +19,7 @@
 #include <vector>
 
 #include "../../include/ferry_amd.h"
+#include "count_records.h"
 
 namespace ferry {
 void set_error(const char* fmt, ...);
@@ -49,21 +52,13 @@ extern "C" int64_t ferry_choose_slot(int64_t layer, const uint8_t* active, const
 
 namespace {
 
-// plan_layer over routing IDs of type T (int64 from the Python API, uint8 from the mapped
-// staging buffer).  One pass over the IDs validates them (every ID in [0, E), none repeated
-// within a token: the reference's demand count and layout assume both) and counts each
-// expert's demand, before any state changes; the misses, slot choices and state updates then
-// work on the E demand counts.
+// Demand scan over routing IDs of type T (int64 from the Python API, uint8 from the mapped
+// staging buffer): one pass validates them (every ID in [0, E), none repeated within a token:
+// the reference's demand count and layout assume both) and counts each expert's demand.
+// 0, or -3 with the error set.
 template <typename T>
-int64_t plan_core(int64_t event, int64_t layer, const T* ids, int64_t tokens, int64_t topk,
-                  const float* gate_scores, int64_t* slots, int64_t cap, int64_t* owner,
-                  int64_t* last, float* scores, int64_t experts, int64_t* fetches_out,
-                  int64_t* destinations_out, int64_t* demand_out, const char* who) {
-  ferry::clear_error();
-  if (experts <= 0 || topk <= 0 || tokens < 0 || cap < 0 || layer < 0) {
-    ferry::set_error("%s: bad sizes", who);
-    return -1;
-  }
+int64_t scan_ids(const T* ids, int64_t tokens, int64_t topk, int64_t experts,
+                 std::vector<int64_t>* demand, const char* who) {
   // Four demand histograms, by token mod 4, so that consecutive tokens naming the same expert
   // do not chain their increments through one memory word; a token's repeated IDs are found
   // with a per-expert last-token array.
@@ -90,10 +85,41 @@ int64_t plan_core(int64_t event, int64_t layer, const T* ids, int64_t tokens, in
       ++h[e];
     }
   }
-  std::vector<int64_t> demand((size_t)experts);
+  demand->resize((size_t)experts);
   for (int64_t e = 0; e < experts; ++e)
-    demand[(size_t)e] = hist[(size_t)e] + hist[(size_t)(experts + e)] +
-                        hist[(size_t)(2 * experts + e)] + hist[(size_t)(3 * experts + e)];
+    (*demand)[(size_t)e] = hist[(size_t)e] + hist[(size_t)(experts + e)] +
+                           hist[(size_t)(2 * experts + e)] + hist[(size_t)(3 * experts + e)];
+  return 0;
+}
+
+// The demand of a call whose IDs ferry_history_count checked and counted on the device: the sum
+// of its records.  0, or -3 with the error set.
+int64_t sum_records(const int32_t* records, int64_t tokens, int64_t experts,
+                    std::vector<int64_t>* demand, const char* who) {
+  const int64_t blocks = (tokens + ferry::kCountTokens - 1) / ferry::kCountTokens;
+  const int64_t words = ferry::count_record_words(experts);
+  std::vector<int32_t> sum((size_t)(2 * (words - 1)), 0);
+  for (int64_t b = 0; b < blocks; ++b) {
+    const int32_t* rec = records + b * words;
+    if (rec[0] != 0) {
+      ferry::set_error("%s: an expert id of token %lld is out of range [0, %lld) or repeated", who,
+                       (long long)(b * ferry::kCountTokens + rec[0] - 1), (long long)experts);
+      return -3;
+    }
+    for (int64_t w = 0; w < words - 1; ++w) {
+      const uint32_t pair = (uint32_t)rec[1 + w];
+      sum[(size_t)(2 * w)] += (int32_t)(pair & 0xFFFF);
+      sum[(size_t)(2 * w + 1)] += (int32_t)(pair >> 16);
+    }
+  }
+  demand->assign(sum.begin(), sum.begin() + experts);
+  return 0;
+}
+
+// plan_layer on each expert's demand: the misses, slot choices and state updates.
+int64_t plan_demand(int64_t event, int64_t layer, const std::vector<int64_t>& demand,
+                    const float* gate_scores, int64_t* slots, int64_t cap, int64_t* owner,
+                    int64_t* last, float* scores, int64_t experts, int64_t* fetches_out) {
   const int64_t base = layer * experts;
   std::memcpy(scores + base, gate_scores, (size_t)experts * sizeof(float));
   std::vector<uint8_t> active((size_t)experts, 0);
@@ -164,11 +190,41 @@ int64_t plan_core(int64_t event, int64_t layer, const T* ids, int64_t tokens, in
   }
   for (int64_t e = 0; e < experts; ++e)
     if (active[(size_t)e]) last[base + e] = event + 1;
+  return m;
+}
+
+template <typename T>
+int64_t plan_core(int64_t event, int64_t layer, const T* ids, int64_t tokens, int64_t topk,
+                  const float* gate_scores, int64_t* slots, int64_t cap, int64_t* owner,
+                  int64_t* last, float* scores, int64_t experts, int64_t* fetches_out,
+                  int64_t* destinations_out, int64_t* demand_out, const char* who) {
+  ferry::clear_error();
+  if (experts <= 0 || topk <= 0 || tokens < 0 || cap < 0 || layer < 0) {
+    ferry::set_error("%s: bad sizes", who);
+    return -1;
+  }
+  std::vector<int64_t> demand;
+  const int64_t rc = scan_ids(ids, tokens, topk, experts, &demand, who);
+  if (rc != 0) return rc;
+  const int64_t m = plan_demand(event, layer, demand, gate_scores, slots, cap, owner, last, scores,
+                                experts, fetches_out);
+  if (m < 0) return m;
   if (destinations_out)
     for (int64_t i = 0; i < tokens * topk; ++i)
-      destinations_out[i] = owner[base + (int64_t)ids[i]];
+      destinations_out[i] = owner[layer * experts + (int64_t)ids[i]];
   if (demand_out) std::memcpy(demand_out, demand.data(), (size_t)experts * sizeof(int64_t));
   return m;
+}
+
+// Queue the copies of a plan's misses on the fetch engine (null: plan only).
+int64_t fetch_planned(ferry_h2d* h2d, const int64_t* fetches, int64_t m) {
+  if (m <= 0 || !h2d) return m;
+  std::vector<int64_t> fs((size_t)m), fk((size_t)m);
+  for (int64_t j = 0; j < m; ++j) {
+    fk[(size_t)j] = fetches[3 * j + 1];
+    fs[(size_t)j] = fetches[3 * j + 2];
+  }
+  return ferry_h2d_fetch(h2d, fs.data(), fk.data(), m) == 0 ? m : -2;
 }
 
 }  // namespace
@@ -200,11 +256,26 @@ extern "C" int64_t ferry_plan_fetch(int64_t event, int64_t layer, const uint8_t*
   const int64_t m = plan_core(event, layer, ids, tokens, topk, gate_scores, slots, cap, owner,
                               last, scores, experts, fetches_out, destinations_out, demand_out,
                               "plan_fetch");
-  if (m <= 0 || !h2d) return m;
-  std::vector<int64_t> fs((size_t)m), fk((size_t)m);
-  for (int64_t j = 0; j < m; ++j) {
-    fk[(size_t)j] = fetches_out[3 * j + 1];
-    fs[(size_t)j] = fetches_out[3 * j + 2];
+  return fetch_planned(h2d, fetches_out, m);
+}
+
+extern "C" int64_t ferry_plan_fetch_counts(int64_t event, int64_t layer, const int32_t* records,
+                                           int64_t tokens, const float* gate_scores,
+                                           int64_t* slots, int64_t cap, int64_t* owner,
+                                           int64_t* last, float* scores, int64_t experts,
+                                           int64_t* fetches_out, int64_t* demand_out,
+                                           ferry_h2d* h2d) {
+  ferry::clear_error();
+  if (experts <= 0 || tokens < 0 || cap < 0 || layer < 0) {
+    ferry::set_error("plan_fetch_counts: bad sizes");
+    return -1;
   }
-  return ferry_h2d_fetch(h2d, fs.data(), fk.data(), m) == 0 ? m : -2;
+  std::vector<int64_t> demand;
+  const int64_t rc = sum_records(records, tokens, experts, &demand, "plan_fetch_counts");
+  if (rc != 0) return rc;
+  const int64_t m = plan_demand(event, layer, demand, gate_scores, slots, cap, owner, last, scores,
+                                experts, fetches_out);
+  if (m < 0) return m;
+  if (demand_out) std::memcpy(demand_out, demand.data(), (size_t)experts * sizeof(int64_t));
+  return fetch_planned(h2d, fetches_out, m);
 }

@@ -319,7 +319,7 @@ class SharedExpert:
 
 
 def history_update(selected, experts, window, layer, ring, counts, meta, scores, ids_out=None,
-                   timeouts_out=None, ready_out=None, ready_value=0):
+                   timeouts_out=None, ready_out=None, ready_value=0, records_out=None):
     """Device GateHistory update of ``layer`` (ferry/metadata.py:15-38, frequency rows).
 
     ``scores`` (fp32 [E]), ``ids_out`` (uint8 [T*k]) and ``timeouts_out`` (int32 [1]: the
@@ -327,7 +327,9 @@ def history_update(selected, experts, window, layer, ring, counts, meta, scores,
     CUDA tensors or raw device addresses (ints), e.g. of a mapped host buffer that the kernel
     writes directly.  ``ready_out`` (device address of ``history_ready_words(T, k)`` int32
     words, with ``ids_out``) receives ``ready_value`` in every word once the launch's other
-    writes are visible to the host."""
+    writes are visible to the host.  ``records_out`` (device address of ``history_count_blocks(T)``
+    records of ``history_count_words(E)`` int32, instead of ``ids_out``) receives each expert's
+    demand per 512 tokens; ``ready_out`` then has 1 + ``history_count_blocks(T)`` words."""
     T, k = selected.shape
     sp = scores if isinstance(scores, int) else _dev(scores, 'scores', torch.float32)
     ip = (ids_out if isinstance(ids_out, int) or ids_out is None
@@ -336,6 +338,15 @@ def history_update(selected, experts, window, layer, ring, counts, meta, scores,
           else _dev(timeouts_out, 'timeouts_out', torch.int32))
     rp = (ready_out if isinstance(ready_out, int) or ready_out is None
           else _dev(ready_out, 'ready_out', torch.int32))
+    if records_out is not None:
+        if ids_out is not None:
+            raise RuntimeError('history_update writes either IDs or demand records')
+        check(lib().ferry_history_count(
+            _dev(selected, 'selected', torch.int64), T, k, experts, window, layer,
+            _dev(ring, 'ring', torch.int32), _dev(counts, 'counts', torch.int32),
+            _dev(meta, 'meta', torch.int32), sp, int(records_out), tp, rp, int(ready_value),
+            current_stream(selected.device)), 'history_count')
+        return
     check(lib().ferry_history_update(
         _dev(selected, 'selected', torch.int64), T, k, experts, window, layer,
         _dev(ring, 'ring', torch.int32), _dev(counts, 'counts', torch.int32),
@@ -347,6 +358,16 @@ def history_update(selected, experts, window, layer, ring, counts, meta, scores,
 def history_ready_words(tokens, topk):
     """Number of int32 ready words ``history_update`` writes for a call of ``tokens``."""
     return int(lib().ferry_history_ready_words(int(tokens), int(topk)))
+
+
+def history_count_blocks(tokens):
+    """Number of demand records (512 tokens each) of a call of ``tokens``."""
+    return int(lib().ferry_history_count_blocks(int(tokens)))
+
+
+def history_count_words(experts):
+    """int32 words of one demand record."""
+    return int(lib().ferry_history_count_words(int(experts)))
 
 
 # ------------------------------------------------------------------------------------------

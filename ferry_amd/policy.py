@@ -109,17 +109,32 @@ class Controller:
         the same native call.  Returns fetches[m, 3] (a view of a buffer reused by the next
         call) and the per-rank fetch counts; ``self.demand`` then holds each expert's
         (token, expert) pair count of the call (int64 [E], reused by the next call)."""
-        experts = self.spec.experts
+        fetch_ptr, demand_ptr, cap = self._fetch_pointers()
+        m = lib().ferry_plan_fetch(event, layer, ids_ptr, tokens, topk, scores_ptr,
+                                   self._slots_ptr, cap, self._owner_ptr, self._last_ptr,
+                                   self._scores_ptr, self.spec.experts, fetch_ptr, None,
+                                   demand_ptr, h2d_handle)
+        return self._fetched(m)
+
+    def plan_fetch_counts(self, event, layer, records_ptr, tokens, scores_ptr, h2d_handle):
+        """plan_fetch from the demand records of ``ferry_history_count`` instead of the IDs."""
+        fetch_ptr, demand_ptr, cap = self._fetch_pointers()
+        m = lib().ferry_plan_fetch_counts(event, layer, records_ptr, tokens, scores_ptr,
+                                          self._slots_ptr, cap, self._owner_ptr, self._last_ptr,
+                                          self._scores_ptr, self.spec.experts, fetch_ptr,
+                                          demand_ptr, h2d_handle)
+        return self._fetched(m)
+
+    def _fetch_pointers(self):
         if self._fetch_buf is None:
+            experts = self.spec.experts
             self._fetch_buf = np.empty((experts, 3), np.int64)
             self.demand = np.zeros(experts, np.int64)
             self._fetch_ptrs = (self._fetch_buf.ctypes.data, self.demand.ctypes.data,
                                 int(self.capacities[0]))
-        fetch_ptr, demand_ptr, cap = self._fetch_ptrs
-        m = lib().ferry_plan_fetch(event, layer, ids_ptr, tokens, topk, scores_ptr,
-                                   self._slots_ptr, cap, self._owner_ptr, self._last_ptr,
-                                   self._scores_ptr, experts, fetch_ptr, None, demand_ptr,
-                                   h2d_handle)
+        return self._fetch_ptrs
+
+    def _fetched(self, m):
         if m == -1:
             raise AssertionError(last_error())
         if m == INVALID_ROUTING:

@@ -2,8 +2,9 @@
 
 Per MoE layer call (world = 1):
   1. history: the device window counters of the layer are updated from ``selected``; the
-     same kernel writes the expert IDs (uint8) and the layer's scores straight into mapped
-     host memory -- the host must know the misses to enqueue fetches;
+     same kernel writes the expert IDs (uint8; of a large call each expert's demand instead) and
+     the layer's scores straight into mapped host memory -- the host must know the misses to
+     enqueue fetches;
   2. the layout kernel is enqueued before the host waits for those results, so it overlaps
      the host planning;
   3. the C++ planner picks the misses (ascending expert) and their slots (routing-aware
@@ -48,6 +49,12 @@ from .transport import Transport
 # the step by about 1 % but adds a launch's fixed cost of GPU time for each.
 CHUNK_MIN_PAIRS = 16384
 CHUNKS = 6
+
+# A call with at least this many pairs has the device check its IDs and count each expert's demand
+# instead of the host planner, for which the GPU waits: from launch to plan 512 tokens x 8 of 128
+# took 25.4 us with the IDs and 24.2 with the counts, 8192 x 8 53 and 29, 256 x 8 23.7 and 23.2
+# (about the same), 16 x 8 22.3 and 23.1.
+COUNT_MIN_PAIRS = 2048
 
 
 def expert_ops():
@@ -94,8 +101,10 @@ class OffloadRuntime:
         self.controller = Controller(spec, capacities, policy, topology, balance_tol_bps, salt)
         self.gather = RouteGather(spec.topk, spec.experts, history_window, eviction_score)
         self.transport = Transport(self.ops, spec.topk, spec.experts)
-        # mapped host staging: [scores f32 E | IDs u8 T*k | pad | timeouts i32 | ready i32 ...]
+        # mapped host staging: [scores f32 E | IDs u8 T*k or demand records i32], and
+        # [timeouts i32 | ready i32 ...]
         self._stage_host = None
+        self._ready_host = None
         self._bufs = {}
         self._ready_seq = 0
         # calls wait for their routing IDs by polling the history kernel's ready words (False:
@@ -161,10 +170,6 @@ class OffloadRuntime:
                 f'those experts were not written, so the output of an earlier layer call is '
                 f'invalid')
 
-    def _status_offset(self, tokens):
-        """Byte offset of the timeout word in the staging buffer of a ``tokens``-token call."""
-        return 4 * self.spec.experts + (tokens * self.spec.topk + 3) // 4 * 4
-
     def _buffers(self, tokens):
         b = self._bufs.get(tokens)
         if b is None:
@@ -173,19 +178,31 @@ class OffloadRuntime:
                                      device=self.device),
                      part=torch.empty((tokens * k, spec.hidden), dtype=torch.bfloat16,
                                       device=self.device),
-                     layout=None, ready_n=self.ops.history_ready_words(tokens, k))
+                     layout=None)
+            # a large call plans from demand records instead of IDs (frequency scores only)
+            b['stage'] = tokens * k
+            b['ready_n'] = b['ready_counted'] = self.ops.history_ready_words(tokens, k)
+            b['counted'] = tokens * k >= COUNT_MIN_PAIRS
+            if b['counted']:
+                blocks = self.ops.history_count_blocks(tokens)
+                b['stage'] = max(b['stage'], 4 * blocks * self.ops.history_count_words(spec.experts))
+                b['ready_counted'] = 1 + blocks
             self._bufs[tokens] = b
-        # staging layout: scores | IDs | timeout word | the history kernel's ready words
-        n = self._status_offset(tokens) + 4 + 4 * b['ready_n']
+        # coherent mapped host memory: the history kernel writes the layer's scores, the uint8 IDs
+        # or demand records, the timeout count and its ready words straight into it, so the host
+        # needs no D2H copy.  The timeout word and the ready words have a buffer of their own, in
+        # which no other data of an earlier call can look like this call's number.
+        n = 4 * self.spec.experts + b['stage']
         if self._stage_host is None or self._stage_host.numel() < n:
-            # coherent mapped host memory: the history kernel writes the layer's scores, the
-            # uint8 IDs, the timeout count and its ready words straight into it, so the host
-            # needs no D2H copy
             self._stage_host, self._stage_ptr = mapped_buffer(max(n, 4096))
-            self._stage_host_ptr = self._stage_host.data_ptr()
+        n = 4 + 4 * max(b['ready_n'], b['ready_counted'])
+        if self._ready_host is None or self._ready_host.numel() < n:
+            self._ready_host, self._ready_ptr = mapped_buffer(max(n, 4096))
+            self._ready_host.zero_()   # no call's number
+            self._ready_host_ptr = self._ready_host.data_ptr()
             # int32 view for the timeout word (read right after the routing readback, on the
             # path to the first copy: a torch slice and view there cost about 10 us)
-            self._stage_i32 = self._stage_host.numpy().view(np.int32)
+            self._ready_i32 = self._ready_host.numpy().view(np.int32)
         return b
 
     # -- one layer call ------------------------------------------------------------------------
@@ -208,15 +225,15 @@ class OffloadRuntime:
         # 1. history; the kernel writes scores, IDs and the device's decode FFN timeout count
         # into the mapped host staging buffer (with probability scores its scores go unused)
         frequency = self.gather.score == 'frequency'
-        nbytes = 4 * E + T * k
-        stage_host = self._stage_host[:nbytes]
-        status = self._status_offset(T)
+        counted = frequency and buf['counted']
         # the ready words after the timeout word carry this call's number once the kernel's
         # host-memory writes are visible
         self._ready_seq = self._ready_seq % 0x7FFFFFFF + 1
         seq = self._ready_seq
-        self.device_history.update(layer, selected, self._stage_ptr, self._stage_ptr + 4 * E,
-                                   self._stage_ptr + status, self._stage_ptr + status + 4, seq)
+        staged = self._stage_ptr + 4 * E
+        self.device_history.update(layer, selected, self._stage_ptr, None if counted else staged,
+                                   self._ready_ptr, self._ready_ptr + 4, seq,
+                                   staged if counted else None)
         tail_host = None
         if not frequency:
             tail = min(T, self.window)
@@ -236,7 +253,8 @@ class OffloadRuntime:
         if self._poll_ids:
             # poll the history kernel's ready words: they are seen about 5 us before the event's
             # wait returns, and they show the previous call's slot reads complete
-            words, nw = self._stage_host_ptr + status + 4, buf['ready_n']
+            words = self._ready_host_ptr + 4
+            nw = buf['ready_counted' if counted else 'ready_n']
             wait_ids = lambda: self.h2d.wait_ready(ids_event, words, nw, seq)   # noqa: E731
         else:
             wait_ids = lambda: self.h2d.event_synchronize(ids_event)   # noqa: E731
@@ -258,7 +276,7 @@ class OffloadRuntime:
         t_sync = time.perf_counter_ns()
         wait_ids()
         t_ready = time.perf_counter_ns()
-        count = int(self._stage_i32[status // 4])
+        count = int(self._ready_i32[0])
         if count != self._timeouts_seen:
             late, self._timeouts_seen = count - self._timeouts_seen, count
             raise RuntimeError(self._timeout_message(late))
@@ -266,20 +284,24 @@ class OffloadRuntime:
         # with chunks or timing the copies are queued here; otherwise the planner's native call
         # queues them itself, right after planning
         queue_here = chunked or self.timing
-        if frequency:
+        if counted:
+            fetches, counts = self.controller.plan_fetch_counts(
+                self.event, layer, staged, T, self._stage_ptr,
+                None if queue_here else self.h2d.handle)
+        elif frequency:
             fetches, counts = self.controller.plan_fetch(
-                self.event, layer, self._stage_ptr + 4 * E, T, k, self._stage_ptr,
+                self.event, layer, staged, T, k, self._stage_ptr,
                 None if queue_here else self.h2d.handle)
         else:
             self.history.update(layer, tail_host.numpy())
             scores = self.history.scores(layer)
-            ids = stage_host.numpy()[4 * E:].astype(np.int64).reshape(T, k)
+            ids = self._stage_host.numpy()[4 * E:4 * E + T * k].astype(np.int64).reshape(T, k)
             fetches, _, counts = self.controller.plan(self.event, layer, ids, np.zeros(T, np.int64),
                                                       scores)
             queue_here = True
         t_plan = time.perf_counter_ns()
         if frequency:
-            counts_e = self.controller.demand.copy()   # counted by the planner in its ID pass
+            counts_e = self.controller.demand.copy()   # filled by the planner
         else:
             counts_e = np.bincount(ids.reshape(-1), minlength=E)
         missing_keys = fetches[:, 1] - layer * E

@@ -236,6 +236,20 @@ int ferry_history_update(const int64_t* selected, int64_t tokens, int64_t topk, 
 /* Number of int32 ready words a ferry_history_update call with ids_out writes: one per
  * workgroup, 1 + ceil(tokens * topk / 4096); -1 for bad sizes. */
 int64_t ferry_history_ready_words(int64_t tokens, int64_t topk);
+/*
+ * ferry_history_update for a planner that needs each expert's demand, not the IDs (no counterpart
+ * in the reference; experts <= 255): instead of ids_out, records_out receives one record per 512
+ * tokens, ferry_history_count_blocks(T) of them, each of ferry_history_count_words(E) int32:
+ * 0 or 1 + the first of its tokens with an ID outside [0, E) or a repeated one, then E uint16
+ * counts.  ready_out (nullable) has 1 + ferry_history_count_blocks(T) words.
+ */
+int ferry_history_count(const int64_t* selected, int64_t tokens, int64_t topk, int64_t experts,
+                        int64_t window, int64_t layer, int32_t* ring, int32_t* counts,
+                        int32_t* meta, float* scores_out, int32_t* records_out,
+                        int32_t* ffn_timeouts_out, int32_t* ready_out, int32_t ready_value,
+                        void* stream);
+int64_t ferry_history_count_blocks(int64_t tokens);
+int64_t ferry_history_count_words(int64_t experts);
 
 /*
  * Host planner at world = 1.  Replaces ferry/policy.py:130-194 (plan_layer with
@@ -391,6 +405,14 @@ int64_t ferry_plan_fetch(int64_t event, int64_t layer, const uint8_t* ids, int64
                          int64_t* owner, int64_t* last, float* scores, int64_t experts,
                          int64_t* fetches_out, int64_t* destinations_out, int64_t* demand_out,
                          ferry_h2d* h2d);
+/* ferry_plan_fetch on the records of ferry_history_count for the same tokens: the same decisions,
+ * state updates, demand and return values (-3: a record names a token whose IDs are out of range
+ * or repeated). */
+int64_t ferry_plan_fetch_counts(int64_t event, int64_t layer, const int32_t* records,
+                                int64_t tokens, const float* gate_scores, int64_t* slots,
+                                int64_t cap, int64_t* owner, int64_t* last, float* scores,
+                                int64_t experts, int64_t* fetches_out, int64_t* demand_out,
+                                ferry_h2d* h2d);
 
 #ifdef __cplusplus
 }

@@ -289,6 +289,98 @@ def test_device_history_matches_gate_history(device):
         assert np.array_equal(ids[:T * k].cpu().numpy(), sel.reshape(-1).astype(np.uint8))
 
 
+@pytest.mark.parametrize('E,k', [(128, 8), (64, 6), (255, 9), (33, 1), (9, 9), (1, 1)])
+def test_history_demand_records_plan_like_ids(device, E, k):
+    """ferry_history_count's records lead the planner to the decisions, demand and state of the
+    uint8 IDs, at the edges of a record's 512 tokens; an ID out of range or repeated in any token
+    is refused as it is there, with the state untouched; scores and ring are the same bits."""
+    from ferry_amd.hostmem import mapped_buffer
+    from ferry_amd.metadata import DeviceGateHistory
+    from ferry_amd.policy import Controller
+    from ferry_amd.quota import Topology
+    ops = _ops()
+
+    class Spec:
+        layers, experts = 1, E
+    rng = np.random.default_rng(E)
+    hists = [DeviceGateHistory(1, E, k, 128, device) for _ in range(2)]
+    ctls = [Controller(Spec, [E], 'ferry', Topology.uniform(1, E)) for _ in range(2)]
+    words = ops.history_count_words(E)
+    assert words == 1 + -(-E // 2)
+    for event, T in enumerate([1, 511, 512, 513, 1024, 1300]):
+        sel = np.stack([rng.choice(E, k, replace=False) for _ in range(T)]).astype(np.int64)
+        variants = [(sel, False)]
+        for t in sorted({0, T - 1, min(T - 1, 512)}):
+            for j, bad in ((k - 1, E), (0, -1), (k - 1, None)):
+                if bad is None and k == 1:
+                    continue
+                b = sel.copy()
+                b[t, j] = b[t, 0] if bad is None else bad
+                variants.append((b, True))
+        blocks = ops.history_count_blocks(T)
+        assert blocks == -(-T // 512)
+        for s, bad in variants[1:] + variants[:1]:
+            dsel = torch.from_numpy(s).to(device)
+            host, ptr = mapped_buffer(2 * 4 * E + T * k + 4 * (blocks * words + blocks + 1) + 64)
+            hp = host.data_ptr()
+            host.zero_()
+            rec, ready = 4 * E, 4 * E + 4 * blocks * words
+            scores = ready + 4 * (blocks + 1)
+            ids = scores + 4 * E
+            hists[0].update(0, dsel, ptr, None, None, ptr + ready, 7, ptr + rec)
+            hists[1].update(0, dsel, ptr + scores, ptr + ids)
+            torch.cuda.synchronize()
+            v = host.numpy()
+            assert (v[ready:ready + 4 * (blocks + 1)].view(np.int32) == 7).all()
+            assert np.array_equal(v[:4 * E], v[scores:scores + 4 * E])
+            assert torch.equal(hists[0].ring, hists[1].ring)
+            plans = [lambda: ctls[0].plan_fetch_counts(event, 0, hp + rec, T, hp, None),
+                     lambda: ctls[1].plan_fetch(event, 0, hp + ids, T, k, hp + scores, None)]
+            if bad:
+                for p in plans:
+                    with pytest.raises(RuntimeError, match='out of range|repeated'):
+                        p()
+            else:
+                (f0, c0), (f1, c1) = (p() for p in plans)
+                assert np.array_equal(f0, f1) and np.array_equal(c0, c1)
+                assert np.array_equal(ctls[0].demand, np.bincount(s.reshape(-1), minlength=E))
+                assert np.array_equal(ctls[0].demand, ctls[1].demand)
+            for a in ('slots', 'owner', 'last', 'scores'):
+                assert np.array_equal(getattr(ctls[0], a), getattr(ctls[1], a))
+
+
+def test_runtime_rejects_invalid_ids_of_large_calls(device):
+    """As test_runtime_rejects_invalid_ids, for a call that plans from demand records; a smaller
+    call after it, a larger one and the first again read their own ready words."""
+    from ferry_amd.model import ModelSpec
+    from ferry_amd.quota import Topology
+    from ferry_amd.runtime import OffloadRuntime, COUNT_MIN_PAIRS
+    from ferry_amd import workloads
+    spec = ModelSpec('qwen3_moe', (0,), 16, 4, 256, 128)
+    pool = workloads.make_pool(spec, 1, seed=0)
+    rt = OffloadRuntime(spec, pool, [16], 'ferry', Topology.uniform(1, 16))
+    T = COUNT_MIN_PAIRS // 4
+    g = torch.Generator().manual_seed(0)
+
+    def call(tokens, change=None):
+        x = torch.randn((tokens, 256), generator=g).to(torch.bfloat16).to(device)
+        w = torch.full((tokens, 4), 0.25, dtype=torch.bfloat16, device=device)
+        sel = torch.rand((tokens, 16), generator=g).topk(4, dim=1).indices
+        if change:
+            sel[change[0], 3] = sel[change[0], 0] if change[1] is None else change[1]
+        return rt.execute(0, x, sel.to(device), w, None)
+    call(T)
+    for change in ((T - 1, 16), (0, -1), (T // 2, None)):
+        slots = rt.controller.slots[0].copy()
+        with pytest.raises(RuntimeError, match='out of range|repeated'):
+            call(T, change)
+        assert np.array_equal(slots, rt.controller.slots[0])
+    for tokens in (T, T - 1, 3 * T + 5, T):
+        assert call(tokens).shape == (tokens, 256)
+    torch.cuda.synchronize()
+    rt.close()
+
+
 @pytest.mark.parametrize('T', [16, 1000])
 def test_history_ready_words_and_host_wait(device, T):
     """The history kernel's ready words (one per workgroup, after its host-memory writes) end
