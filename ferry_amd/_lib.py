@@ -53,6 +53,8 @@ SIGNATURES = [
       _c_p]),
     ('ferry_plan_fetch_counts', _i64,
      [_i64, _i64, _c_p, _i64, _c_p, _c_p, _i64, _c_p, _c_p, _c_p, _i64, _c_p, _c_p, _c_p]),
+    ('ferry_layer_lists', ctypes.c_int,
+     [_c_p, _i64, _i64, _i64, _c_p, _c_p, _i64, _c_p, _c_p, _c_p, _c_p]),
     ('ferry_choose_slot', _i64, [_i64, _c_p, _c_p, _i64, _c_p, _c_p, _i64]),
     ('ferry_layer_slots', None, [_c_p, _i64, _i64, _i64, _c_p]),
     ('ferry_h2d_create', ctypes.c_int, [_c_p, _i64, _c_p, _i64, _i64, _i32, ctypes.POINTER(_c_p)]),

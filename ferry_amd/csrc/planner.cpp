@@ -247,6 +247,53 @@ extern "C" void ferry_layer_slots(const int64_t* slots, int64_t cap, int64_t lay
   }
 }
 
+extern "C" int ferry_layer_lists(const int64_t* slots, int64_t cap, int64_t layer, int64_t experts,
+                                 const int64_t* demand, const int64_t* fetches, int64_t m,
+                                 int32_t* slot_of, int32_t* lists, int64_t* list_slots,
+                                 int64_t* sizes) {
+  ferry::clear_error();
+  if (!slots || !demand || !slot_of || !lists || !list_slots || !sizes || (m > 0 && !fetches) ||
+      cap < 0 || layer < 0 || experts <= 0 || m < 0) {
+    ferry::set_error("layer_lists: bad arguments");
+    return 2;
+  }
+  for (int64_t e = 0; e < experts; ++e) slot_of[e] = -1;
+  for (int64_t i = 0; i < cap; ++i) {
+    const int64_t key = slots[i];
+    if (key >= 0 && key / experts == layer) slot_of[key % experts] = (int32_t)i;
+  }
+  std::vector<uint8_t> fetched((size_t)experts, 0);
+  for (int64_t j = 0; j < m; ++j) {
+    const int64_t e = fetches[3 * j + 1] - layer * experts;
+    if (e < 0 || e >= experts) {
+      ferry::set_error("layer_lists: a fetch of another layer");
+      return 2;
+    }
+    fetched[(size_t)e] = 1;
+  }
+  // lists: active, resident, fetched experts, each followed by its row counts
+  int64_t n[3] = {0, 0, 0}, most[3] = {0, 0, 0}, least[3] = {0, 0, 0};
+  for (int64_t e = 0; e < experts; ++e) {
+    const int64_t r = demand[e];
+    if (r <= 0) continue;
+    for (const int l : {0, fetched[(size_t)e] ? 2 : 1}) {
+      int32_t* list = lists + 2 * l * experts;
+      list[n[l]] = (int32_t)e;
+      list[experts + n[l]] = (int32_t)r;
+      list_slots[l * experts + n[l]] = slot_of[e];
+      most[l] = n[l] == 0 || r > most[l] ? r : most[l];
+      least[l] = n[l] == 0 || r < least[l] ? r : least[l];
+      ++n[l];
+    }
+  }
+  for (int l = 0; l < 3; ++l) {
+    sizes[3 * l] = n[l];
+    sizes[3 * l + 1] = most[l];
+    sizes[3 * l + 2] = least[l];
+  }
+  return 0;
+}
+
 extern "C" int64_t ferry_plan_fetch(int64_t event, int64_t layer, const uint8_t* ids,
                                     int64_t tokens, int64_t topk, const float* gate_scores,
                                     int64_t* slots, int64_t cap, int64_t* owner, int64_t* last,

@@ -16,7 +16,10 @@ from ._lib import check, lib
 
 
 def _i64(values):
-    return np.ascontiguousarray(np.asarray(values, dtype=np.int64).reshape(-1))
+    """(int64 values as bytes, their number): the native calls read them before they return, and
+    an array's address costs 2 us more than its bytes."""
+    a = np.asarray(values, dtype=np.int64)
+    return a.tobytes(), a.size
 
 
 DMA, KERNEL = 0, 1   # FERRY_H2D_DMA, FERRY_H2D_KERNEL
@@ -60,35 +63,40 @@ class H2DEngine:
         return self._h
 
     def fetch(self, slots, keys):
-        s, k = _i64(slots), _i64(keys)
-        if len(s) != len(k):
+        (s, n), (k, nk) = _i64(slots), _i64(keys)
+        if n != nk:
             raise RuntimeError('slots and keys must have the same length')
-        check(lib().ferry_h2d_fetch(self._h, s.ctypes.data, k.ctypes.data, len(s)), 'H2DEngine.fetch')
+        check(lib().ferry_h2d_fetch(self._h, s, k, n), 'H2DEngine.fetch')
 
     def wait_host(self, slots):
-        s = _i64(slots)
-        check(lib().ferry_h2d_wait_host(self._h, s.ctypes.data, len(s)), 'H2DEngine.wait_host')
+        s, n = _i64(slots)
+        check(lib().ferry_h2d_wait_host(self._h, s, n), 'H2DEngine.wait_host')
 
     def wait_stream(self, slots, stream=None):
-        s = _i64(slots)
+        s, n = _i64(slots)
         st = stream if stream is not None else torch.cuda.current_stream(self._cache.device)
-        check(lib().ferry_h2d_wait_stream(self._h, s.ctypes.data, len(s), st.cuda_stream),
+        check(lib().ferry_h2d_wait_stream(self._h, s, n, st.cuda_stream),
+              'H2DEngine.wait_stream')
+
+    def wait_stream_at(self, slots_ptr, n, stream_handle):
+        """wait_stream on the ``n`` int64 slots at a host address, by the stream's handle."""
+        check(lib().ferry_h2d_wait_stream(self._h, slots_ptr, n, stream_handle),
               'H2DEngine.wait_stream')
 
     def mark_used(self, slots, stream=None):
-        s = _i64(slots)
+        s, n = _i64(slots)
         st = stream if stream is not None else torch.cuda.current_stream(self._cache.device)
-        check(lib().ferry_h2d_mark_used(self._h, s.ctypes.data, len(s), st.cuda_stream),
+        check(lib().ferry_h2d_mark_used(self._h, s, n, st.cuda_stream),
               'H2DEngine.mark_used')
 
     def mark_used_record(self, slots, stream=None):
         """mark_used and a host-waitable event in one record on ``stream``: returns the
         event's handle (owned by the engine, valid until the next call of this method), for
         ``event_synchronize``."""
-        s = _i64(slots)
+        s, n = _i64(slots)
         st = stream if stream is not None else torch.cuda.current_stream(self._cache.device)
         ev = ctypes.c_void_p()
-        check(lib().ferry_h2d_mark_used_record(self._h, s.ctypes.data, len(s), st.cuda_stream,
+        check(lib().ferry_h2d_mark_used_record(self._h, s, n, st.cuda_stream,
                                                ctypes.byref(ev)), 'H2DEngine.mark_used_record')
         return ev.value
 

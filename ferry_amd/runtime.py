@@ -29,6 +29,7 @@ unwritten and counts a timeout on the device.  The history kernel copies that co
 routing IDs, so the next call raises RuntimeError when it grew (an earlier call's output is then
 invalid), and so do ``reset`` and ``close``.
 """
+import ctypes
 import time
 
 import numpy as np
@@ -36,9 +37,11 @@ import torch
 import torch.distributed as dist
 
 from . import expert_ops as ops
+from ._lib import check, lib
+from .h2d import DMA, KERNEL
 from .hostmem import mapped_buffer
 from .metadata import DeviceGateHistory, GateHistory, RouteGather
-from .policy import Controller, layer_slots
+from .policy import Controller
 from .transport import Transport
 
 
@@ -60,6 +63,30 @@ COUNT_MIN_PAIRS = 2048
 def expert_ops():
     """The native op module (reference: ferry/runtime.py:26-31)."""
     return ops
+
+
+class _LayerLists:
+    """Buffers of ferry_layer_lists and their addresses: 0 the active experts, 1 the resident, 2
+    the fetched ones."""
+
+    def __init__(self, experts):
+        self.experts = experts
+        self.slot_of = np.empty(experts, np.int32)
+        self.lists = np.empty((3, 2, experts), np.int32)
+        self.slots = np.empty((3, experts), np.int64)
+        self.sizes_array = np.zeros(9, np.int64)
+        self.sizes = [0] * 9
+        self.slot_of_ptr, self.lists_ptr = self.slot_of.ctypes.data, self.lists.ctypes.data
+        self.slots_ptr, self.sizes_ptr = self.slots.ctypes.data, self.sizes_array.ctypes.data
+
+    def slots_at(self, which):
+        return self.slots_ptr + 8 * which * self.experts
+
+    def entry(self, which):
+        """(experts, row counts, entries, most rows, least rows) of one list."""
+        at = self.lists_ptr + 8 * which * self.experts
+        n, most, least = self.sizes[3 * which:3 * which + 3]
+        return at, at + 4 * self.experts, n, most, least
 
 
 class OffloadRuntime:
@@ -106,6 +133,7 @@ class OffloadRuntime:
         self._stage_host = None
         self._ready_host = None
         self._bufs = {}
+        self._lists = _LayerLists(spec.experts)
         self._ready_seq = 0
         # calls wait for their routing IDs by polling the history kernel's ready words (False:
         # on the event recorded after that kernel)
@@ -217,7 +245,11 @@ class OffloadRuntime:
         E = spec.experts
         if hidden.dtype != torch.bfloat16 or hidden.dim() != 2 or hidden.shape[1] != spec.hidden:
             raise RuntimeError('hidden must be bf16 [tokens, hidden]')
+        if not hidden.is_cuda:
+            raise RuntimeError('hidden must be a CUDA tensor')
+        hidden = hidden.contiguous()
         stream = torch.cuda.current_stream(self.device)
+        handle = stream.cuda_stream
         buf = self._buffers(T)
         selected = selected.contiguous()
         weights = weights.to(torch.bfloat16).contiguous()
@@ -245,19 +277,11 @@ class OffloadRuntime:
         # one event both releases the IDs to the host and marks the slots that the previous call
         # read on this stream (no event of their own between that call's kernels)
         pend = self._pending_used
-        if pend is not None and pend[1] != stream.cuda_stream:
+        if pend is not None and pend[1] != handle:
             self._flush_used()
             pend = None
         self._pending_used = None
         ids_event = self.h2d.mark_used_record(pend[0] if pend is not None else [], stream)
-        if self._poll_ids:
-            # poll the history kernel's ready words: they are seen about 5 us before the event's
-            # wait returns, and they show the previous call's slot reads complete
-            words = self._ready_host_ptr + 4
-            nw = buf['ready_counted' if counted else 'ready_n']
-            wait_ids = lambda: self.h2d.wait_ready(ids_event, words, nw, seq)   # noqa: E731
-        else:
-            wait_ids = lambda: self.h2d.event_synchronize(ids_event)   # noqa: E731
 
         # 2. layout (overlaps the host planning)
         buf['layout'] = self.ops.layout(selected, weights, E, out=buf['layout'])
@@ -274,7 +298,13 @@ class OffloadRuntime:
 
         # 3. plan + fetch
         t_sync = time.perf_counter_ns()
-        wait_ids()
+        if self._poll_ids:
+            # poll the history kernel's ready words: they are seen about 5 us before the event's
+            # wait returns, and they show the previous call's slot reads complete
+            self.h2d.wait_ready(ids_event, self._ready_host_ptr + 4,
+                                buf['ready_counted' if counted else 'ready_n'], seq)
+        else:
+            self.h2d.event_synchronize(ids_event)
         t_ready = time.perf_counter_ns()
         count = int(self._ready_i32[0])
         if count != self._timeouts_seen:
@@ -300,18 +330,17 @@ class OffloadRuntime:
                                                       scores)
             queue_here = True
         t_plan = time.perf_counter_ns()
-        if frequency:
-            counts_e = self.controller.demand.copy()   # filled by the planner
-        else:
-            counts_e = np.bincount(ids.reshape(-1), minlength=E)
-        missing_keys = fetches[:, 1] - layer * E
+        demand = self.controller.demand if frequency else np.bincount(ids.reshape(-1), minlength=E)
+        lists = self._layer_lists(layer, demand, fetches)
+        missing_keys = None
         # copy order: heaviest expert first, so that the compute left after the last copy is
         # the lightest (the planner's slot choices do not depend on the order of the copies)
         if chunked and len(fetches) > 1:
-            order = np.argsort(-counts_e[missing_keys], kind='stable')
+            missing_keys = fetches[:, 1] - layer * E
+            order = np.argsort(-demand[missing_keys], kind='stable')
             groups = [g for g in np.array_split(order, min(CHUNKS, len(fetches))) if len(g)]
         else:
-            groups = [np.arange(len(fetches))]
+            groups = [np.arange(len(fetches))] if queue_here else [None]
         timing = self.timing and len(fetches) > 0
         if timing:
             copy_stream = stream if on_stream else self.h2d.stream
@@ -326,27 +355,20 @@ class OffloadRuntime:
             # last sub-batch's experts follow the call's last copy
             ends = self.h2d.groups()
             if len(ends) > 1:
+                missing_keys = fetches[:, 1] - layer * E
                 groups = [np.arange(a, b) for a, b in zip([0] + ends[:-1], ends)]
         t_fetch = time.perf_counter_ns()
-        self.fetches_per_rank += counts
-        if self.event >= spec.layers:
-            self.decode_fetches_per_rank += counts
         if timing:
             ev[1].record(copy_stream)
 
         # 4. experts: resident first, then the fetched ones (chunk by chunk as they land)
-        slot_of = layer_slots(self.controller.slots[0], self.cap, layer, E)
-        active = counts_e > 0
-        missing = np.zeros(E, bool)
-        missing[missing_keys] = True
-        resident_list = np.flatnonzero(active & ~missing)
-        slot32 = slot_of.astype(np.int32)
-        common = (self.cache, hidden.contiguous(), lay.w_sorted, lay.starts, lay.rows, lay.cols)
+        common = (hidden, lay, buf, T, k, handle)
+        n_active, n_resident = lists.sizes[0], lists.sizes[3]
         if not self.timing:
             # the reads below are marked by the next call's ID event on this stream (or by
             # _flush_used); set before they are queued, so that a call that fails part-way still
             # orders later copies into these slots after whatever it queued
-            self._pending_used = (slot_of[np.flatnonzero(active)], stream.cuda_stream, stream)
+            self._pending_used = (lists.slots[0][:n_active].copy(), handle, stream)
         if not self.overlap and len(fetches):
             started = time.perf_counter_ns()
             self.h2d.wait_host(fetches[:, 2])
@@ -356,32 +378,43 @@ class OffloadRuntime:
         if on_stream:
             # the copies are queued on this stream (the wait on their events costs nothing);
             # resident rows may come from DMA copies of earlier calls
-            active_list = np.flatnonzero(active)
-            self.h2d.wait_stream(slot_of[active_list], stream)
+            self.h2d.wait_stream_at(lists.slots_at(0), n_active, handle)
             if timing:
                 waits.append((ev[0], ev[1]))   # the copy kernel holds this stream
-            self._ffn(common, active_list, slot32, buf, stream, counts_e)
-        elif len(resident_list):
-            self.h2d.wait_stream(slot_of[resident_list], stream)
-            self._ffn(common, resident_list, slot32, buf, stream, counts_e)
-        shared_out = shared(common[1], out=self._shared_out(T)) if shared is not None else None
+            self._ffn(common, *lists.entry(0))
+        elif n_resident:
+            self.h2d.wait_stream_at(lists.slots_at(1), n_resident, handle)
+            self._ffn(common, *lists.entry(1))
+        shared_out = shared(hidden, out=self._shared_out(T)) if shared is not None else None
         if len(fetches) and not on_stream:
             for g in groups:
                 w0 = w1 = None
                 if timing:
                     w0 = torch.cuda.Event(enable_timing=True)
                     w0.record(stream)
-                self.h2d.wait_stream(fetches[g, 2], stream)
+                if len(groups) == 1:
+                    self.h2d.wait_stream_at(lists.slots_at(2), len(fetches), handle)
+                else:
+                    self.h2d.wait_stream(fetches[g, 2], stream)
                 if timing:
                     w1 = torch.cuda.Event(enable_timing=True)
                     w1.record(stream)
                     waits.append((w0, w1))
-                self._ffn(common, np.sort(missing_keys[g]), slot32, buf, stream, counts_e)
+                if len(groups) == 1:
+                    self._ffn(common, *lists.entry(2))
+                else:
+                    el = np.sort(missing_keys[g])
+                    rows = demand[el]
+                    self._ffn(common, el.astype(np.int32).tobytes(), rows.astype(np.int32).tobytes(),
+                              len(el), int(rows.max()), int(rows.min()))
         if self.timing:
-            self.h2d.mark_used(slot_of[np.flatnonzero(active)], stream)
+            self.h2d.mark_used(lists.slots[0][:n_active], stream)
         if timing:
             self.timings.append((ev, waits, (mark, self.ops.timing_mark())))
             self.step_marks.append((d2h, ev[0], ev[1], waits[-1][1] if waits else None))
+        self.fetches_per_rank += counts
+        if self.event >= spec.layers:
+            self.decode_fetches_per_rank += counts
         self.event += 1
 
         # 5. combine (+ the shared experts' output)
@@ -404,7 +437,6 @@ class OffloadRuntime:
 
     def _set_copy_mode(self, on_stream, stream):
         """Copy kernel on ``stream`` for on-stream calls, DMA copies otherwise."""
-        from .h2d import DMA, KERNEL
         mode = (on_stream, stream.cuda_stream if on_stream else None)
         if mode != self._copy_mode:
             self.h2d.engine = KERNEL if on_stream else DMA
@@ -418,16 +450,34 @@ class OffloadRuntime:
                                       device=self.device)
         return b['shared']
 
-    def _ffn(self, common, expert_list, slot32, buf, stream, counts_e):
-        """Phase 1 (gate/up + SwiGLU) and phase 2 (down + weight) for ``expert_list``."""
+    def _layer_lists(self, layer, demand, fetches):
+        """The call's expert lists (ferry_layer_lists) in this runtime's buffers, which the native
+        calls of the same layer call read."""
+        lists, ctl = self._lists, self.controller
+        check(lib().ferry_layer_lists(ctl._slots_ptr, self.cap, layer, self.spec.experts,
+                                      demand.tobytes(), fetches.tobytes(), len(fetches),
+                                      lists.slot_of_ptr, lists.lists_ptr, lists.slots_ptr,
+                                      lists.sizes_ptr), 'layer_lists')
+        lists.sizes = lists.sizes_array.tolist()
+        return lists
+
+    def _ffn(self, common, expert_list, list_rows, n, most, least):
+        """Phase 1 (gate/up + SwiGLU) and phase 2 (down + weight) for the ``n`` experts of
+        ``expert_list`` with ``list_rows`` rows each (int32, host addresses or bytes)."""
+        hidden, lay, buf, T, k, handle = common
         spec = self.spec
-        self.ops.expert_ffn(*common, expert_list, slot32, spec.hidden, spec.intermediate,
-                            buf['act'], buf['part'], out_mode=0, experts=spec.experts,
-                            counts=counts_e)
+        check(lib().ferry_expert_ffn(
+            self.cache.data_ptr(), self.cap, spec.hidden, spec.intermediate, hidden.data_ptr(), T, k,
+            lay.w_sorted.data_ptr(), lay.starts.data_ptr(), lay.rows.data_ptr(),
+            lay.cols.data_ptr(), expert_list, n, self._lists.slot_of_ptr, spec.experts, most, least,
+            list_rows, buf['act'].data_ptr(), buf['part'].data_ptr(), 0, self.ops.PHASE_BOTH,
+            handle), 'expert_ffn')
         if self.timing:
             H, I = spec.hidden, spec.intermediate
-            rows = int(counts_e[expert_list].sum())
-            d = len(expert_list)
+            data = (list_rows if isinstance(list_rows, bytes)
+                    else ctypes.string_at(list_rows, 4 * n))
+            rows = int(np.frombuffer(data, np.int32).sum())
+            d = n
             # algorithmic bytes: weights read once, x / activation rows read, outputs written
             self.kernel_bytes['up'] += d * 2 * I * H * 2 + rows * (H * 2 + I * 2)
             self.kernel_bytes['down'] += d * H * I * 2 + rows * (I * 2 + H * 2 + 2)

@@ -405,6 +405,16 @@ int64_t ferry_plan_fetch(int64_t event, int64_t layer, const uint8_t* ids, int64
                          int64_t* owner, int64_t* last, float* scores, int64_t experts,
                          int64_t* fetches_out, int64_t* destinations_out, int64_t* demand_out,
                          ferry_h2d* h2d);
+/* The expert lists of a planned layer call, for ferry_expert_ffn and the fetch engine (in place of
+ * the host array work of ferry/runtime.py:76-89 and of ferry_layer_slots).  From the planner's
+ * slots, the call's demand and its m fetches: slot_of[E] int32 (-1: not cached) and three lists,
+ * experts ascending: 0 all with demand, 1 those already resident, 2 those fetched.  lists is int32
+ * [3][2][E] (experts, row counts), list_slots int64 [3][E], sizes int64 [3][3] (entries, most rows,
+ * least rows). */
+int ferry_layer_lists(const int64_t* slots, int64_t cap, int64_t layer, int64_t experts,
+                      const int64_t* demand, const int64_t* fetches, int64_t m, int32_t* slot_of,
+                      int32_t* lists, int64_t* list_slots, int64_t* sizes);
+
 /* ferry_plan_fetch on the records of ferry_history_count for the same tokens: the same decisions,
  * state updates, demand and return values (-3: a record names a token whose IDs are out of range
  * or repeated). */

@@ -449,3 +449,39 @@ def test_pack_row_round_trip():
     assert lib().ferry_pack_row(rnd.ctypes.data, n, None, 0, ctypes.byref(nb)) == 1
     assert lib().ferry_pack_row(rnd.ctypes.data, 100, None, 0, ctypes.byref(nb)) == 2
     assert lib().ferry_pack_row(rnd.ctypes.data, 48, None, 0, ctypes.byref(nb)) == 2
+
+
+@pytest.mark.parametrize('E,cap,L', [(1, 1, 1), (7, 5, 2), (128, 128, 3), (255, 300, 2), (512, 40, 4)])
+def test_layer_lists_match_array_code(E, cap, L):
+    """ferry_layer_lists against layer_slots and numpy selections: active, resident and fetched
+    experts (each may be empty), their rows, slots and row bounds; bad arguments are refused."""
+    from ferry_amd._lib import lib
+    from ferry_amd.policy import layer_slots
+    rng = np.random.default_rng(E + cap)
+    for trial in range(12):
+        layer = int(rng.integers(0, L))
+        slots = rng.permutation(np.concatenate([np.arange(L * E), np.full(cap, -1)]))[:cap].astype(np.int64)
+        slot_of = layer_slots(slots, cap, layer, E)
+        cached = np.flatnonzero(slot_of >= 0)
+        active = np.sort(rng.choice(cached, rng.integers(0, len(cached) + 1), replace=False))
+        got = np.sort(rng.choice(active, rng.integers(0, len(active) + 1), replace=False)).astype(np.int64)
+        demand = np.zeros(E, np.int64)
+        demand[active] = rng.integers(1, 70000, len(active))
+        fetches = np.ascontiguousarray(np.stack([0 * got, got + layer * E, slot_of[got]], 1)).astype(np.int64)
+        so, lists = np.empty(E, np.int32), np.empty((3, 2, E), np.int32)
+        ls, sizes = np.empty((3, E), np.int64), np.empty((3, 3), np.int64)
+        args = [slots.ctypes.data, cap, layer, E, demand.ctypes.data, fetches.ctypes.data, len(got),
+                so.ctypes.data, lists.ctypes.data, ls.ctypes.data, sizes.ctypes.data]
+        assert lib().ferry_layer_lists(*args) == 0
+        assert np.array_equal(so, slot_of)
+        for i, want in enumerate((active, np.setdiff1d(active, got), got)):
+            n = len(want)
+            assert sizes[i, 0] == n
+            assert np.array_equal(lists[i, 0, :n], want) and np.array_equal(lists[i, 1, :n], demand[want])
+            assert np.array_equal(ls[i, :n], slot_of[want])
+            if n:
+                assert sizes[i, 1] == demand[want].max() and sizes[i, 2] == demand[want].min()
+        if len(got):
+            fetches[0, 1] = (layer + 1) * E
+            assert lib().ferry_layer_lists(*args) != 0
+        assert lib().ferry_layer_lists(None, *args[1:]) != 0
