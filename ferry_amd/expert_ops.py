@@ -11,14 +11,15 @@ from operator import add, attrgetter
 
 import numpy as np
 import torch
+import torch.nn.functional as F
 
 from ._lib import check, lib
 from ._lib import check as _check_status
 from .h2d import H2DEngine
 
 __all__ = ['execute_experts', 'pack_dispatch', 'unpack_dispatch', 'reduce_partials',
-           'scatter_returned', 'H2DEngine', 'router_topk', 'layout', 'expert_ffn', 'combine',
-           'SharedExpert', 'history_update', 'history_ready_words', 'current_stream', 'PHASE_UP',
+           'scatter_returned', 'H2DEngine', 'router_topk', 'layout', 'gate_logits', 'expert_ffn',
+           'combine', 'SharedExpert', 'history_update', 'history_ready_words', 'current_stream', 'PHASE_UP',
            'PHASE_DOWN', 'PHASE_BOTH']
 
 MAX_EXPERTS = 512
@@ -115,6 +116,28 @@ def router_topk(logits, topk, renorm=True, scale=1.0, sorted=True, return_probs=
         _dev(tie_counter, 'tie_counter', torch.int32) if tie_counter is not None else None,
         _stream_of(logits)), 'router_topk')
     return (w, idx, probs) if return_probs else (w, idx)
+
+
+def gate_logits(x, weight):
+    """fp32 router logits of a gate: ``F.linear(x.float(), weight.float())`` (the DeepSeek-V2 gate
+    feeding ferry/model.py:151-158).
+
+    Plain bf16 CUDA matrices go to a kernel that reads them as they are (another order of the fp32
+    additions); everything else, and a call that autograd or autocast takes part in, is the torch
+    expression."""
+    if (x.dtype is torch.bfloat16 and weight.dtype is torch.bfloat16 and x.is_cuda
+            and x.dim() == 2 and weight.dim() == 2 and x.shape[1] == weight.shape[1]
+            and x.shape[1] % 64 == 0 and x.numel() and weight.numel()
+            and x.get_device() == weight.get_device()
+            and x.is_contiguous() and weight.is_contiguous()
+            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
+            and not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
+            and not torch.is_autocast_enabled() and torch.autograd.forward_ad._current_level < 0):
+        out = torch.empty((x.shape[0], weight.shape[0]), dtype=torch.float32, device=x.device)
+        check(lib().ferry_gate_logits(x.data_ptr(), x.shape[0], x.shape[1], weight.data_ptr(),
+                                      weight.shape[0], out.data_ptr(), _stream_of(x)), 'gate_logits')
+        return out
+    return F.linear(x.float(), weight.float())
 
 
 class Layout:

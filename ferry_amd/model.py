@@ -137,7 +137,10 @@ def deepseek_moe(rt, layer, flat, gate_weight, topk, shared=None, routed_scaling
     HF gate): fp32 logits = fp32(x) fp32(W)^T, fp32 softmax / top-k (sorted=False) / scaling /
     bf16 in the router kernel, the routed experts in the runtime, and the shared experts
     (``expert_ops.SharedExpert``) added in bf16 inside the combine.  Returns (out, logits)."""
-    logits = F.linear(flat.float(), gate_weight.float())
+    # with probability scores the logits' last bits enter the eviction state: torch's own there
+    frequency = getattr(rt.gather, 'score', 'frequency') == 'frequency'
+    logits = (ops.gate_logits(flat, gate_weight) if frequency
+              else F.linear(flat.float(), gate_weight.float()))
     weights, selected, tail = _route(rt, logits, topk, renorm=False, sorted=False,
                                      scale=routed_scaling_factor)
     return rt.execute(layer, flat, selected, weights, tail, shared=shared), logits

@@ -211,6 +211,15 @@ int ferry_unpack_dispatch(const void* payload, int64_t packets, int64_t hidden_s
                           void* hidden_out, void* weights_out, void* stream);
 
 /*
+ * Router logits of a gate with bf16 weights in fp32: out[tokens, experts] = fp32(x) fp32(w)^T for
+ * bf16 x[tokens, hidden] and w[experts, hidden] (the DeepSeek-V2 gate that feeds
+ * ferry/model.py:151-158), fp32 accumulation.  hidden must be a multiple of 64, x and w 16-byte
+ * aligned.
+ */
+int ferry_gate_logits(const void* x, int64_t tokens, int64_t hidden, const void* w,
+                      int64_t experts, float* out, void* stream);
+
+/*
  * Selection-frequency history on the device.  Replaces ferry/metadata.py:15-38 (GateHistory
  * update/scores over one-hot rows built by RouteGather.collect, ferry/metadata.py:67-83).
  * State per layer (device memory, caller-owned, zero-initialised):

@@ -289,6 +289,59 @@ def test_device_history_matches_gate_history(device):
         assert np.array_equal(ids[:T * k].cpu().numpy(), sel.reshape(-1).astype(np.uint8))
 
 
+@pytest.mark.parametrize('T', [1, 15, 16, 17, 513, 1025, 2047, 4100, 8200, 20000])
+@pytest.mark.parametrize('E,H', [(64, 2048), (37, 192), (130, 64)])
+def test_gate_logits(device, T, E, H):
+    """The gate kernel at the edges of its tiles (all five over these sizes) against 64 bits: a
+    product of bf16 values is exact in fp32, so each of fewer than H + 16 additions errs by at most
+    2^-24 of the sum of magnitudes (2^-23 where the adder truncates)."""
+    ops = _ops()
+    g = torch.Generator(device=device).manual_seed(T + E)
+    x = torch.randn((T, H), generator=g, device=device).to(torch.bfloat16)
+    w = torch.randn((E, H), generator=g, device=device).to(torch.bfloat16)
+    out = ops.gate_logits(x, w)
+    assert out.shape == (T, E) and out.dtype == torch.float32
+    want = x.double() @ w.double().t()
+    bound = (x.double().abs() @ w.double().abs().t()) * (H + 16) * 2.0 ** -23
+    assert ((out.double() - want).abs() <= bound).all()
+    assert (out.double() - want).norm() <= 1e-6 * want.norm()
+    assert torch.equal(ops.gate_logits(x, w), out)
+
+
+def test_gate_logits_other_forms(device):
+    """What the gate kernel does not take is torch's expression: other types, strides, alignment,
+    sizes, empty calls, autograd, autocast; infinities and NaN come out as they do there."""
+    import torch.nn.functional as F
+    ops = _ops()
+    g = torch.Generator(device=device).manual_seed(0)
+    x = torch.randn((70, 256), generator=g, device=device).to(torch.bfloat16)
+    w = torch.randn((40, 256), generator=g, device=device).to(torch.bfloat16)
+    forms = [(x.float(), w), (x, w.half()), (x[:, :250], w[:, :250]), (x.t()[:64], w[:, :70]),
+             (x[:, 1:65], w[:, :64]), (x[::2], w), (x[:0], w), (x, w[::3]),
+             (x.reshape(-1)[1:1 + 64 * 64].view(64, 64), w[:, :64].contiguous())]
+    for a, b in forms:
+        if a.shape[1] != b.shape[1]:
+            with pytest.raises(RuntimeError):
+                ops.gate_logits(a, b)
+            continue
+        torch.testing.assert_close(ops.gate_logits(a, b), F.linear(a.float(), b.float()),
+                                   rtol=1e-4, atol=1e-3)
+    wg = w.clone().requires_grad_()
+    y = ops.gate_logits(x, wg)
+    y.sum().backward()
+    assert wg.grad is not None and wg.grad.shape == w.shape
+    with torch.no_grad():
+        assert not ops.gate_logits(x, wg).requires_grad
+    with torch.autocast('cuda', dtype=torch.bfloat16):
+        assert ops.gate_logits(x, w).dtype == torch.bfloat16
+    for v in (float('inf'), float('-inf'), float('nan')):
+        xb = x.clone()
+        xb[3, 5] = v
+        a, b = ops.gate_logits(xb, w), F.linear(xb.float(), w.float())
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isinf(), b.isinf())
+        assert torch.equal(a[a.isinf()], b[b.isinf()])
+
+
 @pytest.mark.parametrize('E,k', [(128, 8), (64, 6), (255, 9), (33, 1), (9, 9), (1, 1)])
 def test_history_demand_records_plan_like_ids(device, E, k):
     """ferry_history_count's records lead the planner to the decisions, demand and state of the
