@@ -1182,7 +1182,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void f
 // =============================================================================================
 
 // The workgroups of ffn_up_skinny<1> (I/16 per expert) come first in the grid, those of
-// ffn_down_skinny<1> (H/64 per expert) after them.  A down workgroup needs every intermediate
+// ffn_down_skinny<1> (H/64 per expert; H/16 with DownRows16) after them.  A down workgroup needs every intermediate
 // column of its expert's activation rows, so it waits for all of that expert's up workgroups:
 // each up workgroup, once its rows are stored, sets its arrival flag; a down workgroup's first
 // wavefront waits for all flags of its expert.  The L2s of the XCDs are not coherent with
@@ -1200,7 +1200,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void f
 //
 // Arrival flags: one 32-bit word per up workgroup, holding the epoch (a number unique to the
 // call) once that workgroup's rows are stored.  A down workgroup's first wavefront checks all
-// flags of its expert at once (one lane per flag) until every one holds the call's epoch.  Flags
+// flags of its expert at once (a lane takes every 64th) until every one holds the call's epoch.  Flags
 // from earlier calls hold older epochs, so nothing is ever cleared, and no word is written by
 // two workgroups (no read-modify-write contention).  The flags live in a static per-device ring
 // of kSyncSets sets (set = epoch % kSyncSets); calls that run at the same time on one GPU use
