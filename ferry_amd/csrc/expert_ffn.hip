@@ -2004,16 +2004,16 @@ struct MTiles {
 static int ffn_launch_list(FfnArgs& args, const int32_t* expert_list, const int32_t* slot_of,
                            int32_t n_list, int32_t n_mid, int64_t maxn, int64_t min_rows,
                            int64_t pairs, const MTiles& mt, int32_t phases, int64_t hidden,
-                           int64_t inter, hipStream_t s);
+                           int64_t inter, int64_t tiled_cus, hipStream_t s);
 
-extern "C" int ferry_expert_ffn(const void* cache, int64_t cache_rows, int64_t hidden,
+static int expert_ffn_call(const void* cache, int64_t cache_rows, int64_t hidden,
                                 int64_t inter, const void* x, int64_t rows_in, int64_t topk,
                                 const void* w_sorted, const int64_t* starts, const int64_t* rows,
                                 const int64_t* cols, const int32_t* expert_list, int32_t n_list,
                                 const int32_t* slot_of, int64_t experts,
                                 int64_t max_rows_per_expert, int64_t min_rows_per_expert,
                                 const int32_t* list_rows, void* act, void* out,
-                                int32_t out_mode, int32_t phases, void* stream) {
+                                int32_t out_mode, int32_t phases, int32_t spare_cus, void* stream) {
   clear_error();
   FERRY_CHECK_ARG(phases >= 1 && phases <= 3, "phases must be 1 (up), 2 (down) or 3 (both)");
   FERRY_CHECK_ARG(hidden > 0 && hidden % 128 == 0, "hidden must be a positive multiple of 128");
@@ -2025,6 +2025,7 @@ extern "C" int ferry_expert_ffn(const void* cache, int64_t cache_rows, int64_t h
   FERRY_CHECK_ARG(experts >= 1 && experts <= FERRY_MAX_EXPERTS, "experts must be in [1, %d]",
                   FERRY_MAX_EXPERTS);
   FERRY_CHECK_ARG(out_mode == 0 || out_mode == 1, "out_mode must be 0 or 1");
+  FERRY_CHECK_ARG(spare_cus >= 0 && spare_cus <= 128, "spare_cus must be in [0, 128]");
   // the tiled down projection covers the hidden dimension in 256-column tiles
   FERRY_CHECK_ARG(hidden % 256 == 0 || max_rows_per_expert <= kSkinnyMax,
                   "hidden must be a multiple of 256 when an expert has more than %d rows",
@@ -2071,6 +2072,7 @@ extern "C" int ferry_expert_ffn(const void* cache, int64_t cache_rows, int64_t h
   args.I = inter;
   args.k = topk;
   args.out_mode = out_mode;
+  const int64_t tiled_cus = g_num_cus > 2 * spare_cus ? g_num_cus - spare_cus : g_num_cus;
   // max_rows_per_expert must bound every n_e from above (rows_in does for a layout from
   // ferry_layout) and min_rows_per_expert from below (0 when unknown); the kernels size their
   // work from the device starts, the bounds only select and gate the launches.  With the
@@ -2080,7 +2082,7 @@ extern "C" int ferry_expert_ffn(const void* cache, int64_t cache_rows, int64_t h
   // without rows are left out.
   if (!list_rows)
     return ffn_launch_list(args, expert_list, slot_of, n_list, n_list, max_rows_per_expert,
-                           min_rows_per_expert, rows_in * topk, MTiles{}, phases, hidden, inter, s);
+                           min_rows_per_expert, rows_in * topk, MTiles{}, phases, hidden, inter, tiled_cus, s);
   std::vector<int32_t> small, big;
   int32_t n_mid = 0;
   MTiles mt;
@@ -2104,13 +2106,41 @@ extern "C" int ferry_expert_ffn(const void* cache, int64_t cache_rows, int64_t h
   if (!small.empty()) {
     const int rc = ffn_launch_list(args, small.data(), slot_of, (int32_t)small.size(), n_mid,
                                    small_max, small_min, rows_in * topk, MTiles{}, phases, hidden,
-                                   inter, s);
+                                   inter, tiled_cus, s);
     if (rc != 0) return rc;
   }
   if (!big.empty())
     return ffn_launch_list(args, big.data(), slot_of, (int32_t)big.size(), 0, big_max, big_min,
-                           rows_in * topk, mt, phases, hidden, inter, s);
+                           rows_in * topk, mt, phases, hidden, inter, tiled_cus, s);
   return 0;
+}
+
+extern "C" int ferry_expert_ffn(const void* cache, int64_t cache_rows, int64_t hidden,
+                                int64_t inter, const void* x, int64_t rows_in, int64_t topk,
+                                const void* w_sorted, const int64_t* starts, const int64_t* rows,
+                                const int64_t* cols, const int32_t* expert_list, int32_t n_list,
+                                const int32_t* slot_of, int64_t experts,
+                                int64_t max_rows_per_expert, int64_t min_rows_per_expert,
+                                const int32_t* list_rows, void* act, void* out,
+                                int32_t out_mode, int32_t phases, void* stream) {
+  return expert_ffn_call(cache, cache_rows, hidden, inter, x, rows_in, topk, w_sorted, starts, rows, cols,
+                         expert_list, n_list, slot_of, experts, max_rows_per_expert,
+                         min_rows_per_expert, list_rows, act, out, out_mode, phases, 0, stream);
+}
+
+extern "C" int ferry_expert_ffn_spare(const void* cache, int64_t cache_rows, int64_t hidden,
+                                      int64_t inter, const void* x, int64_t rows_in, int64_t topk,
+                                      const void* w_sorted, const int64_t* starts,
+                                      const int64_t* rows, const int64_t* cols,
+                                      const int32_t* expert_list, int32_t n_list,
+                                      const int32_t* slot_of, int64_t experts,
+                                      int64_t max_rows_per_expert, int64_t min_rows_per_expert,
+                                      const int32_t* list_rows, void* act, void* out,
+                                      int32_t out_mode, int32_t phases, int32_t spare_cus,
+                                      void* stream) {
+  return expert_ffn_call(cache, cache_rows, hidden, inter, x, rows_in, topk, w_sorted, starts, rows, cols,
+                         expert_list, n_list, slot_of, experts, max_rows_per_expert,
+                         min_rows_per_expert, list_rows, act, out, out_mode, phases, spare_cus, stream);
 }
 
 // Which tile a list's tiled experts take: the one whose rounds of one tile per CU cost least.  A
@@ -2176,7 +2206,7 @@ static int tiled_launch(const FfnArgs& args, const MTiles& mt, int64_t pairs, in
 static int ffn_launch_list(FfnArgs& args, const int32_t* expert_list, const int32_t* slot_of,
                            int32_t n_list, int32_t n_mid, int64_t maxn, int64_t min_rows,
                            int64_t pairs, const MTiles& mt, int32_t phases, int64_t hidden,
-                           int64_t inter, hipStream_t s) {
+                           int64_t inter, int64_t tiled_cus, hipStream_t s) {
   const bool any_small = min_rows <= kSkinnyMax;
   for (int32_t off = 0; off < n_list; off += kListMax) {
     const int32_t cnt = (n_list - off) < kListMax ? (n_list - off) : kListMax;
@@ -2188,7 +2218,7 @@ static int ffn_launch_list(FfnArgs& args, const int32_t* expert_list, const int3
       args.list.slot[i] = i < cnt ? slot_of[expert_list[off + i]] : 0;
     }
     const bool any_big = maxn > kSkinnyMax;
-    const int64_t grid_cap = (int64_t)g_num_cus;  // one tiled workgroup per CU
+    const int64_t grid_cap = tiled_cus;  // one tiled workgroup per CU
     if (phases == 3 && any_small && !any_big && maxn <= 16 && inter / 16 <= kMaxUpWgs) {
       // decode: both phases in one launch, each expert's down projection as soon as its up
       // projection is stored

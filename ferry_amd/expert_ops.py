@@ -220,7 +220,7 @@ SKINNY_MAX_ROWS = 64   # experts with at most this many rows run the small-exper
 
 def expert_ffn(cache, x, w_sorted, starts, rows, cols, expert_list, slot_of, hidden,
                intermediate, act, out, out_mode=0, max_rows=None, experts=None, phases=PHASE_BOTH,
-               counts=None):
+               counts=None, spare_cus=0):
     """Grouped SwiGLU over cache slots for the experts in ``expert_list`` (host ints).
 
     phases: PHASE_UP (gate/up + SwiGLU into ``act``), PHASE_DOWN (down + routing weight from
@@ -228,7 +228,8 @@ def expert_ffn(cache, x, w_sorted, starts, rows, cols, expert_list, slot_of, hid
     the row count of every expert, ``starts[e+1] - starts[e]``: the library then issues the
     experts with at most 64 rows (small-expert kernels, 17-64 rows first) and the larger ones
     (tiled kernels) as separate launches with exact row bounds, and skips experts without rows.
-    ``rows`` and ``cols`` are CUDA tensors or raw device addresses (ints).
+    ``rows`` and ``cols`` are CUDA tensors or raw device addresses (ints).  ``spare_cus`` keeps the
+    tiled kernels off that many CUs, for kernels on other streams.
     """
     R, k = w_sorted.shape
     el = np.ascontiguousarray(expert_list, dtype=np.int32)
@@ -240,19 +241,19 @@ def expert_ffn(cache, x, w_sorted, starts, rows, cols, expert_list, slot_of, hid
             rows if isinstance(rows, int) else _dev(rows, 'rows', torch.int64),
             cols if isinstance(cols, int) else _dev(cols, 'cols', torch.int64))
     tail = (_dev(act, 'act', torch.bfloat16), _dev(out, 'out', torch.bfloat16), int(out_mode),
-            int(phases), _stream_of(x))
+            int(phases), int(spare_cus), _stream_of(x))
 
     # the host lists as bytes: an array's address costs 2 us more
     n, el_at, so_at = len(el), el.tobytes(), so.tobytes()
     if counts is None:
-        check(lib().ferry_expert_ffn(*args, el_at, n, so_at, E,
+        check(lib().ferry_expert_ffn_spare(*args, el_at, n, so_at, E,
                                      int(max_rows if max_rows is not None else R), 0, None, *tail),
               'expert_ffn')
         return out
     c = np.ascontiguousarray(np.asarray(counts, dtype=np.int64)[el], dtype=np.int32)
     if n:
         rows_of = c.tolist()
-        check(lib().ferry_expert_ffn(*args, el_at, n, so_at, E, max(rows_of), min(rows_of),
+        check(lib().ferry_expert_ffn_spare(*args, el_at, n, so_at, E, max(rows_of), min(rows_of),
                                      c.tobytes(), *tail), 'expert_ffn')
     return out
 
@@ -341,7 +342,7 @@ class SharedExpert:
             self._bufs[T] = b
         return b
 
-    def __call__(self, x, out=None):
+    def __call__(self, x, out=None, spare_cus=0):
         """bf16 [T, H] -> bf16 [T, H] = down(silu(x Wg^T) * (x Wu^T))."""
         T = x.shape[0]
         if out is None:
@@ -351,7 +352,7 @@ class SharedExpert:
         b = self._buffers(T, x.device)
         return expert_ffn(self.row, x.contiguous(), b['w'], b['starts'], b['rows'], b['cols'], [0],
                           np.zeros(1, np.int32), self.hidden, self.intermediate, b['act'], out,
-                          out_mode=1, experts=1, counts=[T])
+                          out_mode=1, experts=1, counts=[T], spare_cus=spare_cus)
 
 
 def history_update(selected, experts, window, layer, ring, counts, meta, scores, ids_out=None,

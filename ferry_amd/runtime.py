@@ -52,6 +52,13 @@ from .transport import Transport
 # the step by about 1 % but adds a launch's fixed cost of GPU time for each.
 CHUNK_MIN_PAIRS = 16384
 CHUNKS = 6
+# Packed chunked calls: CUs that the tiled kernels leave to the unpacking of the rows still being
+# copied.  A tiled workgroup holds its CU's registers for the whole launch, so without them a row's
+# unpacking, and the copies behind it, wait for a launch to end: 26 DeepSeek-V2-Lite layers of 65,536
+# tokens, every expert fetched, take 372.5 ms with 0, 362.7 with 8, 362.2 with 16, 360.7 with 32 (FFN
+# 7.7, 7.9, 8.1, 8.3 ms a layer, which the copies of 13.2 ms hide); 48 Qwen3 layers of 8192 tokens
+# 703.1, 703.5, 702.9 and 701.5.
+UNPACK_CUS = 16
 
 # A call with at least this many pairs has the device check its IDs and count each expert's demand
 # instead of the host planner, for which the GPU waits: from launch to plan 512 tokens x 8 of 128
@@ -363,6 +370,8 @@ class OffloadRuntime:
 
         # 4. experts: resident first, then the fetched ones (chunk by chunk as they land)
         common = (hidden, lay, buf, T, k, handle)
+        # CUs that the tiled kernels leave to the unpacking of rows still being copied
+        spare = UNPACK_CUS if chunked and self.packed is not None and len(fetches) else 0
         n_active, n_resident = lists.sizes[0], lists.sizes[3]
         if not self.timing:
             # the reads below are marked by the next call's ID event on this stream (or by
@@ -384,8 +393,11 @@ class OffloadRuntime:
             self._ffn(common, *lists.entry(0))
         elif n_resident:
             self.h2d.wait_stream_at(lists.slots_at(1), n_resident, handle)
-            self._ffn(common, *lists.entry(1))
-        shared_out = shared(hidden, out=self._shared_out(T)) if shared is not None else None
+            self._ffn(common, *lists.entry(1), spare)
+        shared_out = None
+        if shared is not None:
+            out = self._shared_out(T)
+            shared_out = shared(hidden, out=out, spare_cus=spare) if spare else shared(hidden, out=out)
         if len(fetches) and not on_stream:
             for g in groups:
                 w0 = w1 = None
@@ -406,7 +418,8 @@ class OffloadRuntime:
                     el = np.sort(missing_keys[g])
                     rows = demand[el]
                     self._ffn(common, el.astype(np.int32).tobytes(), rows.astype(np.int32).tobytes(),
-                              len(el), int(rows.max()), int(rows.min()))
+                              len(el), int(rows.max()), int(rows.min()),
+                              spare if g is not groups[-1] else 0)
         if self.timing:
             self.h2d.mark_used(lists.slots[0][:n_active], stream)
         if timing:
@@ -461,17 +474,17 @@ class OffloadRuntime:
         lists.sizes = lists.sizes_array.tolist()
         return lists
 
-    def _ffn(self, common, expert_list, list_rows, n, most, least):
+    def _ffn(self, common, expert_list, list_rows, n, most, least, spare=0):
         """Phase 1 (gate/up + SwiGLU) and phase 2 (down + weight) for the ``n`` experts of
         ``expert_list`` with ``list_rows`` rows each (int32, host addresses or bytes)."""
         hidden, lay, buf, T, k, handle = common
         spec = self.spec
-        check(lib().ferry_expert_ffn(
+        check(lib().ferry_expert_ffn_spare(
             self.cache.data_ptr(), self.cap, spec.hidden, spec.intermediate, hidden.data_ptr(), T, k,
             lay.w_sorted.data_ptr(), lay.starts.data_ptr(), lay.rows.data_ptr(),
             lay.cols.data_ptr(), expert_list, n, self._lists.slot_of_ptr, spec.experts, most, least,
             list_rows, buf['act'].data_ptr(), buf['part'].data_ptr(), 0, self.ops.PHASE_BOTH,
-            handle), 'expert_ffn')
+            spare, handle), 'expert_ffn')
         if self.timing:
             H, I = spec.hidden, spec.intermediate
             data = (list_rows if isinstance(list_rows, bytes)

@@ -157,6 +157,16 @@ int ferry_expert_ffn(const void* cache, int64_t cache_rows, int64_t hidden, int6
                      int64_t experts, int64_t max_rows_per_expert,
                      int64_t min_rows_per_expert, const int32_t* list_rows, void* act, void* out,
                      int32_t out_mode, int32_t phases, void* stream);
+/* ferry_expert_ffn with the tiled kernels' workgroups, which stay for a whole launch and leave no
+ * registers for others on their CU, on all CUs but spare_cus (0 to 128; 0: the same call), so that
+ * kernels on other streams (the unpacking of rows that are still being fetched) run beside them. */
+int ferry_expert_ffn_spare(const void* cache, int64_t cache_rows, int64_t hidden, int64_t inter,
+                     const void* x, int64_t rows_in, int64_t topk, const void* w_sorted,
+                     const int64_t* starts, const int64_t* rows, const int64_t* cols,
+                     const int32_t* expert_list, int32_t n_list, const int32_t* slot_of,
+                     int64_t experts, int64_t max_rows_per_expert,
+                     int64_t min_rows_per_expert, const int32_t* list_rows, void* act, void* out,
+                     int32_t out_mode, int32_t phases, int32_t spare_cus, void* stream);
 int ferry_expert_ffn_sync_timeouts(int64_t* count);
 int ferry_expert_ffn_set_sync_spin_limit(int64_t limit);
 

@@ -289,6 +289,35 @@ def test_device_history_matches_gate_history(device):
         assert np.array_equal(ids[:T * k].cpu().numpy(), sel.reshape(-1).astype(np.uint8))
 
 
+@pytest.mark.parametrize('counts', [[70], [300, 65, 128, 2000, 20, 3], [1500] * 24])
+def test_tiled_kernels_spare_cus_bit_identical(device, counts):
+    """The tiled kernels on fewer CUs (more tiles a workgroup, other workgroups for a tile) give the
+    same bits; a number of spare CUs outside [0, 128] is refused."""
+    ops = _ops()
+    H, I, E, R = 512, 256, len(counts), sum(counts)
+    g = torch.Generator(device=device).manual_seed(R)
+    cache = (torch.randn((E, 3 * H * I), generator=g, device=device) * 0.05).to(torch.bfloat16)
+    x = torch.randn((R, H), generator=g, device=device).to(torch.bfloat16)
+    w = torch.rand((R, 1), generator=g, device=device).to(torch.bfloat16)
+    starts = torch.tensor(np.concatenate([[0], np.cumsum(counts)]), dtype=torch.int64, device=device)
+    rows = torch.randperm(R, generator=g, device=device)
+    cols = torch.zeros(R, dtype=torch.int64, device=device)
+
+    def run(spare, counts_arg):
+        act = torch.full((R, I), 7.0, dtype=torch.bfloat16, device=device)
+        out = torch.full((R, H), 7.0, dtype=torch.bfloat16, device=device)
+        ops.expert_ffn(cache, x, w, starts, rows, cols, np.arange(E), np.arange(E, dtype=np.int32), H, I,
+                       act, out, out_mode=1, experts=E, counts=counts_arg, spare_cus=spare)
+        return out
+    for counts_arg in (counts, None):
+        base = run(0, counts_arg)
+        for spare in (1, 5, 16, 128):
+            assert torch.equal(run(spare, counts_arg), base), spare
+    for spare in (-1, 129):
+        with pytest.raises(RuntimeError, match='spare_cus'):
+            run(spare, counts)
+
+
 @pytest.mark.parametrize('T', [1, 15, 16, 17, 513, 1025, 2047, 4100, 8200, 20000])
 @pytest.mark.parametrize('E,H', [(64, 2048), (37, 192), (130, 64)])
 def test_gate_logits(device, T, E, H):
@@ -400,6 +429,38 @@ def test_history_demand_records_plan_like_ids(device, E, k):
                 assert np.array_equal(ctls[0].demand, ctls[1].demand)
             for a in ('slots', 'owner', 'last', 'scores'):
                 assert np.array_equal(getattr(ctls[0], a), getattr(ctls[1], a))
+
+
+def test_first_call_ignores_words_of_earlier_runtimes(device):
+    """A runtime whose host buffers reuse an earlier runtime's memory (its ready words hold call
+    number 1, its IDs every expert) waits for its own first call's IDs."""
+    import gc
+    from ferry_amd.model import ModelSpec
+    from ferry_amd.quota import Topology
+    from ferry_amd.runtime import OffloadRuntime
+    from ferry_amd import workloads
+    spec = ModelSpec('qwen3_moe', (0,), 128, 8, 256, 128)
+    pool = workloads.make_pool(spec, 1, seed=0)
+
+    def call(rt, sel):
+        x = torch.ones((sel.shape[0], 256), dtype=torch.bfloat16, device=device)
+        w = torch.full(sel.shape, 0.125, dtype=torch.bfloat16, device=device)
+        return rt.execute(0, x, sel, w, None)
+    every = torch.arange(128, device=device).reshape(16, 8)
+    eight = torch.arange(40, 48, device=device).expand(16, 8).contiguous()
+    for _ in range(4):
+        rt = OffloadRuntime(spec, pool, [128], 'ferry', Topology.uniform(1, 128))
+        call(rt, every)
+        call(rt, every.repeat(64, 1))
+        torch.cuda.synchronize()
+        rt.close()
+        del rt
+        gc.collect()
+        rt = OffloadRuntime(spec, pool, [38], 'ferry', Topology.uniform(1, 128))
+        call(rt, eight)
+        torch.cuda.synchronize()
+        assert sorted(rt.controller.slots[0][rt.controller.slots[0] >= 0]) == list(range(40, 48))
+        rt.close()
 
 
 def test_runtime_rejects_invalid_ids_of_large_calls(device):
