@@ -459,6 +459,9 @@ def execute_experts(cache, input, routing_weights, slots, rows, cols, hidden, in
     slots = np.asarray(slots, np.int64)
     if slots.min() < 0 or slots.max() >= cache.shape[0]:
         raise RuntimeError('slot out of range')
+    # before anything is queued: the group starts are written to memory on the input's device
+    _dev(input, 'input', torch.bfloat16, contiguous=False)
+    _dev(routing_weights, 'routing_weights', torch.bfloat16, contiguous=False)
     sizes = [r.numel() for r in rows]
     dev = input.device
     rows_at, P, _rows = _joined(rows, torch.int64, dev)
@@ -513,6 +516,7 @@ def reduce_partials(parts, rows, received, hidden, like):
     """fp32 sum of expert outputs per received row, ascending group order, then bf16 (:76-83)."""
     if len(parts) == 0:
         return torch.zeros((received, hidden), dtype=torch.bfloat16, device=like.device)
+    _dev(parts[0], 'parts', contiguous=False)   # the sums are written to memory on this device
     dev = parts[0].device
     part_at, n, _parts = _joined(parts, torch.bfloat16, dev)
     if part_at % 16:

@@ -485,3 +485,28 @@ def test_layer_lists_match_array_code(E, cap, L):
             fetches[0, 1] = (layer + 1) * E
             assert lib().ferry_layer_lists(*args) != 0
         assert lib().ferry_layer_lists(None, *args[1:]) != 0
+
+
+@pytest.mark.parametrize('rows', [0, 3])
+def test_host_tensors_are_refused_before_any_launch(monkeypatch, rows):
+    """Host tensors, with and without rows: the drop-in calls raise before a native call could hand
+    the address of a host tensor to a kernel."""
+    import torch
+    from ferry_amd import expert_ops as ops
+
+    class NoNative:
+        def __getattr__(self, name):
+            raise AssertionError(f'{name} was called')
+    monkeypatch.setattr(ops, 'lib', NoNative)
+    monkeypatch.setattr(ops, '_raw_stream', lambda device: 0)
+    dev = ops._dev      # takes the cache here, so that the other tensors' checks are reached
+    monkeypatch.setattr(ops, '_dev', lambda t, name, *a, **kw: 0 if name == 'cache' else dev(t, name, *a, **kw))
+    H, I = 128, 128
+    cache = torch.zeros((2, 3 * H * I), dtype=torch.bfloat16)
+    x, w = torch.zeros((4, H), dtype=torch.bfloat16), torch.zeros((4, 1), dtype=torch.bfloat16)
+    idx = torch.zeros(rows, dtype=torch.int64)
+    part = torch.zeros((rows, H), dtype=torch.bfloat16)
+    with pytest.raises(RuntimeError, match='must be a CUDA tensor'):
+        ops.execute_experts(cache, x, w, [0], [idx], [idx], H, I)
+    with pytest.raises(RuntimeError, match='must be a CUDA tensor'):
+        ops.reduce_partials([part], [idx], 4, H, part)
