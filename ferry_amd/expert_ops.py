@@ -522,8 +522,8 @@ def reduce_partials(parts, rows, received, hidden, like):
     if part_at % 16:
         _parts = torch.cat([p.reshape(-1) for p in parts])
         part_at = _parts.data_ptr()
-    if n % hidden:
-        raise RuntimeError('parts must hold rows of hidden elements')
+    if any(map(hidden.__rmod__, map(_numel, parts))):
+        raise RuntimeError('every part must hold whole rows of hidden elements')
     rows_at, entries, _rows = _joined(rows, torch.int64, dev)
     if entries > n // hidden:
         raise RuntimeError('rows must not outnumber the rows of parts')

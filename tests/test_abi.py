@@ -510,3 +510,19 @@ def test_host_tensors_are_refused_before_any_launch(monkeypatch, rows):
         ops.execute_experts(cache, x, w, [0], [idx], [idx], H, I)
     with pytest.raises(RuntimeError, match='must be a CUDA tensor'):
         ops.reduce_partials([part], [idx], 4, H, part)
+
+
+def test_reduce_partials_refuses_parts_of_broken_rows(monkeypatch):
+    """Parts that are not whole rows each are refused, also where they add up to whole rows."""
+    import torch
+    from ferry_amd import expert_ops as ops
+
+    class NoNative:
+        def __getattr__(self, name):
+            raise AssertionError(f'{name} was called')
+    monkeypatch.setattr(ops, 'lib', NoNative)
+    monkeypatch.setattr(ops, '_dev', lambda t, *a, **kw: t.data_ptr())
+    parts = [torch.zeros(n, dtype=torch.bfloat16) for n in (12, 4)]
+    rows = [torch.zeros(1, dtype=torch.int64)] * 2
+    with pytest.raises(RuntimeError, match='whole rows'):
+        ops.reduce_partials(parts, rows, 2, 8, parts[0])
