@@ -2200,6 +2200,17 @@ static int tiled_launch(const FfnArgs& args, const MTiles& mt, int64_t pairs, in
   return 0;
 }
 
+// Is work on s being captured into a graph?  (The null stream cannot be captured, and is not asked.)
+static bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (s == nullptr) return false;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();   // the launch that follows reports what is wrong with the stream
+    return false;
+  }
+  return st != hipStreamCaptureStatusNone;
+}
+
 // The launches of one list: n_mid of its leading entries are known to hold 17-64 rows (the
 // small-expert up launch gives them 64-column workgroups; the others get 16-column ones unless
 // the bounds allow no expert of more than 16 rows, n_mid = n_list when unknown).
@@ -2219,9 +2230,10 @@ static int ffn_launch_list(FfnArgs& args, const int32_t* expert_list, const int3
     }
     const bool any_big = maxn > kSkinnyMax;
     const int64_t grid_cap = tiled_cus;  // one tiled workgroup per CU
-    if (phases == 3 && any_small && !any_big && maxn <= 16 && inter / 16 <= kMaxUpWgs) {
+    if (phases == 3 && any_small && !any_big && maxn <= 16 && inter / 16 <= kMaxUpWgs && !capturing(s)) {
       // decode: both phases in one launch, each expert's down projection as soon as its up
-      // projection is stored
+      // projection is stored.  Not in a graph: its replays would all carry the captured epoch, whose
+      // flags the first of them leaves set, so a later one's down projections would not wait.
       FusedSync fs;
       uint32_t* sync = nullptr;
       const int rc = sync_addresses(&sync, &fs.timeouts);

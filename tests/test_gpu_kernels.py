@@ -710,6 +710,48 @@ def test_tiled_kernels_tile_shapes_bit_identical(device, E, n):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))
 
 
+@pytest.mark.parametrize('H,I,counts', [(2048, 2816, [16]), (2048, 768, [16, 3, 0, 9]), (256, 4096, [5] * 9),
+                                        (512, 1408, [1, 16])])
+def test_decode_ffn_graph_replays(device, H, I, counts):
+    """A captured decode call with both phases, replayed with new rows and weights each time and
+    eager calls in between: every replay gives the eager call's bits."""
+    ops = _ops()
+    E, P = len(counts), sum(counts)
+    cache = _pool(E, H, I, seed=I).to(device)
+    g = torch.Generator(device=device).manual_seed(P)
+    x = torch.empty((P, H), dtype=torch.bfloat16, device=device)
+    w = torch.empty((P, 1), dtype=torch.bfloat16, device=device)
+    starts = torch.tensor(np.concatenate([[0], np.cumsum(counts)]), device=device)
+    rows, cols = torch.randperm(P, device=device), torch.zeros(P, dtype=torch.int64, device=device)
+    act = torch.empty((P, I), dtype=torch.bfloat16, device=device)
+    out = torch.empty((P, H), dtype=torch.bfloat16, device=device)
+
+    def call(out):
+        ops.expert_ffn(cache, x, w, starts, rows, cols, np.arange(E), np.arange(E, dtype=np.int32), H, I,
+                       act, out, out_mode=1, experts=E, counts=counts)
+        return out
+
+    def fresh():
+        x.normal_(generator=g)
+        w.uniform_(0.5, 1.5, generator=g)
+    fresh()
+    call(out)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(out)
+    for replay in range(6):
+        fresh()
+        out.fill_(float('nan'))
+        graph.replay()
+        torch.cuda.synchronize()
+        want = call(torch.empty_like(out))
+        assert torch.equal(out.view(torch.int16), want.view(torch.int16)), replay
+        for _ in range(replay):
+            call(torch.empty_like(out))
+    assert ops.ffn_sync_timeouts() == 0
+
+
 @pytest.mark.parametrize('H,I,counts', [
     # one-launch decode with down workgroups of 16 hidden rows: K ranges of 1, 3 (odd), 6, 11 (odd), 12
     # and 22 steps a wavefront, one and several experts, an expert without rows
