@@ -17,7 +17,9 @@
 // a NaN or +inf logit has all-NaN probabilities, i.e. all elements compare equal.
 // Selection runs on order-preserving uint32 keys of the probabilities.
 //
-// Every row replays the CPU algorithm exactly, on a whole wavefront:
+// Sorted rows without ties have one possible result, which k wavefront arg-max rounds find
+// (distinct_select; taken first where ties are rare, see ferry_router_topk).  Every other row
+// replays the CPU algorithm exactly, on a whole wavefront:
 //  * introselect: the row is held 1, 2 or 4 keys per lane (position p = 64 * slot + lane); each
 //    median-of-3 / Hoare partition step is evaluated in one pass -- the j-th left stop (ascending
 //    position holding a key <= pivot) is exchanged with the j-th right stop (descending position
@@ -29,12 +31,13 @@
 //    k*64 <= n; k - 1 > 16) runs the sequential algorithm on lane 0 over the row in LDS.
 //
 // A decode call is bound by this chain's latency (one wavefront a row, a step of it about 1,000
-// clocks), a large batch by its instruction issue.  Finding sorted rows without ties by k arg-max
-// rounds first, and replaying the others with ranks staged in LDS, took 10.7 us for 16 rows (k = 8
-// of 128, bf16: a quarter of the rows have ties), 24.0 us for 8192 and, unsorted (k = 6 of 64, fp32),
-// 7.4 us for 256 and 108 us for 65,536 rows; now 7.6, 19.7, 5.4 and 68.8 us.  Always replaying costs
-// a single row without ties 5.0 -> 6.8 us.
+// clocks), a large batch by its instruction issue.  With the stops' ranks staged in LDS and the
+// arg-max rounds first for every sorted row, 16 rows (k = 8 of 128, bf16) took 10.7 us, 8192 rows 24.0
+// and, unsorted (k = 6 of 64, fp32), 256 rows 7.4 us and 65,536 rows 108 us; now 7.6, 19.7, 5.4 and
+// 68.8 us.
 #include "common.h"
+
+#include <type_traits>
 
 // every rounding step below is the reference's: no contraction of a*b+c into one FMA
 #pragma clang fp contract(off)
@@ -520,6 +523,45 @@ __device__ __forceinline__ float wave_max(float v) {
   v = fmaxf(v, dpp_asf(dpp_u<0x143, 0xc>(u, u)));
   return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), 63));
 }
+__device__ __forceinline__ uint32_t umax_(uint32_t a, uint32_t b) { return a > b ? a : b; }
+__device__ __forceinline__ uint32_t wave_max_u(uint32_t v) {
+  v = umax_(v, dpp_u<0xB1>(v, v));
+  v = umax_(v, dpp_u<0x4E>(v, v));
+  v = umax_(v, dpp_u<0x141>(v, v));
+  v = umax_(v, dpp_u<0x140>(v, v));
+  v = umax_(v, dpp_u<0x142, 0xa>(v, v));
+  v = umax_(v, dpp_u<0x143, 0xc>(v, v));
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// The selection where order and membership do not depend on the algorithm: kk arg-max rounds, lane
+// j < kk receives the j-th largest key's index.  False (e undefined) where a round's largest key is
+// not the only one, i.e. two of the kk + 1 largest are equal.  Keys of elements are above 0, the
+// padding's 0.
+template <int NS>
+__device__ __forceinline__ bool distinct_select(const uint32_t (&k)[NS], int kk, int lane, int& e) {
+  uint32_t cur[NS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s) cur[s] = k[s];
+  for (int r = 0; r < kk; ++r) {
+    uint32_t most = cur[0];
+#pragma unroll
+    for (int s = 1; s < NS; ++s) most = umax_(most, cur[s]);
+    most = wave_max_u(most);
+    int hits = 0, pos = 0;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const uint64_t hit = __ballot(cur[s] == most);
+      hits += __popcll(hit);
+      if (hit) pos = 64 * s + __ffsll((long long)hit) - 1;
+      cur[s] = cur[s] == most ? 0u : cur[s];
+    }
+    if (hits != 1) return false;
+    e = lane == r ? pos : e;
+  }
+  return true;
+}
+
 // SLEEF's single-precision exp with 1.0-ulp bound (xexpf of SLEEF 3, sleefsimdsp.c; the
 // published Cody-Waite reduction by ln 2 in two parts, a degree-6 polynomial for e^s - 1 - s in
 // Horner form with fused multiply-adds, and a two-step scaling by 2^q).  Restated from that
@@ -628,7 +670,8 @@ __device__ __forceinline__ float load_logit<bf16_t>(const bf16_t* p) {
   return bf16_to_f32(*p);
 }
 
-template <typename T, int NS>
+// ARGMAX: sorted rows of the introselect regime, which distinct_select tries first
+template <typename T, int NS, bool ARGMAX>
 __global__ __launch_bounds__(64 * kWaves) void router_kernel(
     const T* __restrict__ logits, int64_t tokens, int n, int kk, int renorm, float scale,
     int sorted, int64_t* __restrict__ idx_out, bf16_t* __restrict__ w_out,
@@ -677,7 +720,9 @@ __global__ __launch_bounds__(64 * kWaves) void router_kernel(
       key[s] = e < n ? (row_bad ? 0xffffffffu : ordered_key(p)) : 0u;
       ix[s] = e;
     }
-    const int e = exact_select(key, ix, n, kk, sorted != 0, lane, ws);
+    int e = 0;
+    if (!ARGMAX || row_bad || !distinct_select(key, kk, lane, e))
+      e = exact_select(key, ix, n, kk, sorted != 0, lane, ws);
     if (tie_rows) {
       // rows whose result depends on the algorithm's order: unsorted, NaN and partial_sort rows, and
       // those with a chosen key that another element has too
@@ -733,17 +778,29 @@ extern "C" int ferry_router_topk(const void* logits, int32_t logits_dtype, int64
     launch("router_kernel", kernel, dim3(grid), dim3(64 * kWaves), 0, s, lg, tokens, (int)experts,
            (int)topk, renorm, scale, sorted, idx_out, (bf16_t*)w_out_bf16, probs_out, tie_rows);
   };
-  if (logits_dtype == FERRY_BF16) {
-    const bf16_t* lg = (const bf16_t*)logits;
-    if (experts <= 64) go(router_kernel<bf16_t, 1>, lg);
-    else if (experts <= 128) go(router_kernel<bf16_t, 2>, lg);
-    else go(router_kernel<bf16_t, 4>, lg);
-  } else {
-    const float* lg = (const float*)logits;
-    if (experts <= 64) go(router_kernel<float, 1>, lg);
-    else if (experts <= 128) go(router_kernel<float, 2>, lg);
-    else go(router_kernel<float, 4>, lg);
-  }
+  auto pick = [&](auto argmax, const auto* lg) {
+    typedef std::decay_t<decltype(*lg)> T;
+    constexpr bool A = decltype(argmax)::value;
+    if (experts <= 64) go(router_kernel<T, 1, A>, lg);
+    else if (experts <= 128) go(router_kernel<T, 2, A>, lg);
+    else go(router_kernel<T, 4, A>, lg);
+  };
+  // Arg-max rounds first where most rows have no ties: fp32 logits, and few bf16 rows (about a quarter
+  // of the rows of 128 bf16 logits has one among its 9 largest, and the rows of a small call are done
+  // when the slowest is).  us, rounds first / replay at once: fp32, k = 8 of 128, 1 row 4.8 / 6.7,
+  // 8192 rows 13 / 20, k = 24 of 128 8.5 / 43 and 25 / 98; bf16 (mean of 100 inputs), k = 8 of 128,
+  // 1 row 4.9 / 6.2, 4 rows 6.4 / 7.1, 8 rows 7.5 / 7.3, 16 rows 7.8 / 7.6.
+  const bool argmax = sorted && topk * 64 > experts && (logits_dtype == FERRY_F32 || tokens <= 4);
+  auto typed = [&](const auto* lg) {
+    if (argmax)
+      pick(std::true_type{}, lg);
+    else
+      pick(std::false_type{}, lg);
+  };
+  if (logits_dtype == FERRY_BF16)
+    typed((const bf16_t*)logits);
+  else
+    typed((const float*)logits);
   FERRY_LAUNCHED("router_kernel");
   return 0;
 }

@@ -55,6 +55,38 @@ def test_router_sorted_matches_torch_cpu_topk(device, E, k, dtype, ties):
         assert int(counter.item()) > 0, 'the exact tie path was not exercised'
 
 
+@pytest.mark.parametrize('E,k', [(1, 1), (9, 9), (60, 4), (64, 6), (65, 7), (128, 8), (128, 24), (129, 18), (256, 32)])
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize('T', [4, 5, 40])
+def test_router_sorted_rows_with_and_without_ties(device, E, k, dtype, T):
+    """Sorted rows of distinct probabilities, and rows whose two equal ones stand at the first, a
+    middle, the k-th and (k+1)-th and the last places; a row with NaN and one with +inf: indices and
+    weights equal to torch's CPU topk, bit for bit, and the rows with ties counted."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(E * 64 + k + T)
+    base = (torch.arange(E).float() - E) * 0.0625      # distinct in bf16 and as probabilities
+    x = torch.stack([base[torch.randperm(E, generator=g)] for _ in range(T)])
+    pairs = [(0, 1), (k // 2, k // 2 + 1), (k - 1, k), (E - 2, E - 1)]
+    ties = 0
+    for row, (a, b) in zip(range(1, T), pairs):
+        if 0 <= a < b < E:
+            order = x[row].argsort(descending=True)
+            x[row, order[b]] = x[row, order[a]]
+            ties += a < k
+    if T > 6:
+        x[5, 0], x[6, E // 2] = float('nan'), float('inf')
+        ties += 2
+    x = x.to(dtype)
+    count = torch.zeros(1, dtype=torch.int32, device=device)
+    w, idx = ops.router_topk(x.to(device), k, tie_counter=count)
+    ref_w, ref_idx, _ = qwen3_router(x, k)
+    assert torch.equal(idx.cpu(), ref_idx)
+    nan = ref_w.isnan()
+    assert torch.equal(w.cpu().isnan(), nan)
+    assert torch.equal(w.cpu().view(torch.int16)[~nan], ref_w.view(torch.int16)[~nan])
+    assert int(count) == (T if k * 64 <= E else ties)
+
+
 @pytest.mark.parametrize('E,k', [(63, 6), (64, 2), (65, 7), (127, 9), (128, 17), (129, 5), (192, 12),
                                  (255, 8), (256, 17)])
 @pytest.mark.parametrize('sorted_', [False, True])
