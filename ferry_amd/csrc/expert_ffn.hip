@@ -1206,7 +1206,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void f
 // of kSyncSets sets (set = epoch % kSyncSets); calls that run at the same time on one GPU use
 // different sets unless kSyncSets of them overlap.
 constexpr int kSyncSets = 8;
-constexpr int kMaxUpWgs = 256;   // up workgroups per expert (I / 16): I <= 4096
+constexpr int kMaxUpWgs = 176;   // up workgroups per expert (I / 16): I <= 2816
 constexpr int kSyncSpinLimit = 1 << 21;
 static __device__ __align__(256) uint32_t g_sync[kSyncSets][kListMax][kMaxUpWgs];
 static __device__ int32_t g_sync_timeouts;
@@ -2200,6 +2200,36 @@ static int tiled_launch(const FfnArgs& args, const MTiles& mt, int64_t pairs, in
   return 0;
 }
 
+// One-launch decode: down workgroups of 16 hidden rows (DownRows16) instead of 64 for a list of cnt
+// experts?  They shorten each workgroup's chain of loads, and pay while the workgroups of 64 rows
+// (wgs) leave CUs idle; past that, four times as many workgroups read the activation rows.  The limit
+// also depends on what they replace: workgroups of 64 rows, which read whole 128-byte pieces of the
+// weight rows only where I is a multiple of 256, and above kWideInter two launches.  Measured for 32
+// H x I of 512-7168 x 512-2816, 1 to 16 experts of 1 and of 16 rows, time relative to those, 1 row an
+// expert - 16 rows:
+//   K range of up to 3 chunks (of 64 columns, per wavefront): 0.87-0.95 up to an eighth of the CUs,
+//     768 x 2048 then 1.02-1.10
+//   I a multiple of 256, up to 2048: at half the CUs 0.87-0.92 (H = 2048), 0.93-1.00 (4096); at 3/4
+//     0.97-1.03 and 0.95-1.04, at all of them 1.03-1.14 and 0.96-1.04
+//   I of 2304 to 2816: below half the CUs 0.75-1.00, at half 0.85-0.99 (H = 2048) and 0.93-1.07
+//     (4096); 8 experts 0.83-1.02, 12 experts 0.93-1.07 (H = 512)
+//   other I: at 5/8 of the CUs 0.79-1.02; 1152 to 1920 at all of them 0.84-1.01 (H up to 5120), 7168 x
+//     1408 already 1.00-1.05 at 7/8; 896 at 3/4 0.97-1.05; 2688 at all of them 0.94-1.04
+// e.g. us, 64 -> 16 rows, 16 rows an expert, H = 2048: I = 1408, 1 expert 17.9 -> 12.7, 3 experts 26.4
+// -> 21.4, 8 experts 37.0 -> 34.4; I = 768, 1 expert 11.0 -> 10.5; the 2048 x 2816 shared expert, from
+// two launches, 20.7 -> 17.2 (1 row: 19.8 -> 14.4).  I = 3072 to 4096 in one launch of 64-row workgroups
+// took 1.04 to 1.23 times the two launches (1 to 6 experts of 16 rows), so they keep those.
+constexpr int kNarrowChunks = 11;    // the longest K range of DownRows16: I <= 2816
+constexpr int kWideInter = 2048;     // largest I of a launch with workgroups of 64 rows
+static bool narrow_down(int64_t cnt, int64_t hidden, int64_t inter) {
+  const int64_t chunks = ceil_div(ceil_div(inter / 32, 4), 2), wgs = cnt * (hidden / 64), cus = g_num_cus;
+  if (chunks <= 3) return wgs <= cus / 8;
+  if (chunks > kNarrowChunks) return false;
+  if (inter % 256 == 0 && inter <= kWideInter) return wgs <= cus / 2;
+  if (inter % 256 == 0) return wgs <= (hidden <= 2048 ? cus / 2 : cus / 2 - 1) && cnt <= 8;
+  return wgs <= (chunks >= 5 && chunks <= 8 && hidden <= 5120 ? cus : cus * 5 / 8);
+}
+
 // Is work on s being captured into a graph?  (The null stream cannot be captured, and is not asked.)
 static bool capturing(hipStream_t s) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
@@ -2230,10 +2260,11 @@ static int ffn_launch_list(FfnArgs& args, const int32_t* expert_list, const int3
     }
     const bool any_big = maxn > kSkinnyMax;
     const int64_t grid_cap = tiled_cus;  // one tiled workgroup per CU
-    if (phases == 3 && any_small && !any_big && maxn <= 16 && inter / 16 <= kMaxUpWgs && !capturing(s)) {
-      // decode: both phases in one launch, each expert's down projection as soon as its up
-      // projection is stored.  Not in a graph: its replays would all carry the captured epoch, whose
-      // flags the first of them leaves set, so a later one's down projections would not wait.
+    // Decode: both phases in one launch, each expert's down projection as soon as its up projection is
+    // stored.  Not in a graph: its replays would all carry the captured epoch, whose flags the first
+    // of them leaves set, so a later one's down projections would not wait.
+    const bool narrow = narrow_down(cnt, hidden, inter);
+    if (phases == 3 && any_small && !any_big && maxn <= 16 && (inter <= kWideInter || narrow) && !capturing(s)) {
       FusedSync fs;
       uint32_t* sync = nullptr;
       const int rc = sync_addresses(&sync, &fs.timeouts);
@@ -2244,15 +2275,7 @@ static int ffn_launch_list(FfnArgs& args, const int32_t* expert_list, const int3
       fs.flags = sync + (int64_t)(epoch % kSyncSets) * kListMax * kMaxUpWgs;
       fs.up_wgs = (int32_t)(inter / 16);
       fs.spin_limit = g_spin_limit.load();
-      // Down workgroups of 16 hidden rows where those of 64 would leave CUs idle: up to one a CU, or
-      // an eighth of that where a wavefront's K range is three chunks (they pay only for the
-      // launch's emptiest CUs: the activation rows are read by four times as many workgroups).  us
-      // for 16 rows an expert, 64 -> 16 hidden rows a workgroup: H x I = 2048 x 1408, 1 expert 19.7
-      // -> 13.5, 3 experts 26.0 -> 21.1, 8 experts 36.2 -> 33.1; 2048 x 768, 1 expert 12.6 -> 11.3,
-      // 3 experts 14.6 -> 14.5, 6 experts 20.5 -> 22.6; the 2048 x 2816 shared expert, in two
-      // launches before, 17.7 + a launch gap -> 16.3 (1 row: 18.4 -> 13.3).
-      const int64_t chunks = ceil_div(ceil_div(inter / 32, 4), 2);   // of 64 columns, per wavefront
-      const bool narrow = cnt * (hidden / 64) <= (chunks <= 3 ? grid_cap / 8 : grid_cap) && chunks <= 11;
+      const int64_t chunks = ceil_div(ceil_div(inter / 32, 4), 2);
       fs.down_wgs = (int32_t)(hidden / (narrow ? 16 : 64));
       launch("ffn_skinny_fused",
              !narrow ? ffn_skinny_fused<0>

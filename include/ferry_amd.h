@@ -136,8 +136,8 @@ int ferry_starts(const int32_t* sizes, int32_t n, int64_t* starts, void* stream)
  * than 4 GiB.
  */
 enum { FERRY_MAX_EXPERTS = 512 };
-/* A call with phases = 3 whose experts all have at most 16 rows (decode, intermediate <= 4096)
- * runs both phases in one launch, unless `stream` is being captured into a graph (replays of one
+/* A call with phases = 3 whose experts all have at most 16 rows (decode, intermediate <= 2048, for
+ * few experts <= 2816) runs both phases in one launch, unless `stream` is being captured into a graph (replays of one
  * launch would share its call number): an expert's down projection starts once its up projection is
  * stored, through arrival flags in a static device ring of 8 sets, one per call in turn.  Calls
  * on one GPU whose kernels run at the same time must number fewer than 8 (calls on one stream

@@ -784,12 +784,41 @@ def test_decode_ffn_graph_replays(device, H, I, counts):
     assert ops.ffn_sync_timeouts() == 0
 
 
+@pytest.mark.parametrize('H,I,n,fused', [(2048, 768, 8, True), (512, 2048, 40, True), (2048, 2816, 4, True),
+                                         (2048, 2816, 5, False), (512, 2688, 20, True), (512, 2688, 21, False),
+                                         (256, 2944, 1, False), (256, 4096, 1, False)])
+def test_decode_launches(device, H, I, n, fused):
+    """Decode lists take one launch up to an intermediate of 2048, above it only while short lists up
+    to 2816 let down workgroups of 16 rows pay, and two launches else; the same bits either way."""
+    ops = _ops()
+    cache = _pool(n, H, I, seed=I).to(device)
+    g = torch.Generator().manual_seed(n)
+    x = torch.randn((2 * n, H), generator=g).to(torch.bfloat16).to(device)
+    w = (torch.rand((2 * n, 1), generator=g) + 0.5).to(torch.bfloat16).to(device)
+    starts = torch.arange(0, 2 * n + 1, 2, device=device)
+    rows, cols = torch.randperm(2 * n, generator=g).to(device), torch.zeros(2 * n, dtype=torch.int64, device=device)
+    outs = []
+    for phases in ((ops.PHASE_BOTH,), (ops.PHASE_UP, ops.PHASE_DOWN)):
+        act = torch.empty((2 * n, I), dtype=torch.bfloat16, device=device)
+        out = torch.full((2 * n, H), float('nan'), dtype=torch.bfloat16, device=device)
+        ops.timing_enable(True)
+        for ph in phases:
+            ops.expert_ffn(cache, x, w, starts, rows, cols, np.arange(n), np.arange(n, dtype=np.int32), H, I,
+                           act, out, out_mode=1, experts=n, counts=[2] * n, phases=ph)
+        torch.cuda.synchronize()
+        launches = [ops.timing_summary(k)[0] for k in ('ffn_skinny_fused', 'ffn_up_skinny', 'ffn_down_skinny')]
+        ops.timing_enable(False)
+        assert launches == ([1, 0, 0] if fused and len(phases) == 1 else [0, 1, 1])
+        outs.append(out.cpu().view(torch.int16))
+    assert torch.equal(*outs)
+
+
 @pytest.mark.parametrize('H,I,counts', [
     # one-launch decode with down workgroups of 16 hidden rows: K ranges of 1, 3 (odd), 6, 11 (odd), 12
     # and 22 steps a wavefront, one and several experts, an expert without rows
     (256, 128, [16]), (256, 384, [1, 0, 16]), (2048, 768, [7]), (512, 1408, [1, 16, 5, 2, 9, 3, 4, 16]),
     (256, 1536, [3, 8]), (256, 2816, [16, 1]),
-    # ... and of 64: more workgroups than that, and the longest K range
+    # ... and of 64: more workgroups than that; longer K ranges (two launches)
     (2048, 768, [2] * 9), (256, 4096, [16]), (256, 3072, [5]),
 ])
 def test_one_launch_decode_bit_identical(device, H, I, counts):
