@@ -28,6 +28,7 @@ SIGNATURES = [
      [_c_p, _c_p, _i64, _i64, _i64, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p]),
     ('ferry_starts', ctypes.c_int, [_c_p, _i32, _c_p, _c_p]),
     ('ferry_reduce_rows_workspace_bytes', _i64, [_i64]),
+    ('ferry_reduce_rows_full_workspace_bytes', _i64, [_i64, _i64]),
     ('ferry_reduce_rows', ctypes.c_int, [_c_p, _i64, _i64, _c_p, _i64, _c_p, _c_p, _i64, _c_p]),
     ('ferry_expert_ffn', ctypes.c_int,
      [_c_p, _i64, _i64, _i64, _c_p, _i64, _i64, _c_p, _c_p, _c_p, _c_p, _c_p, _i32, _c_p, _i64,

@@ -69,23 +69,39 @@ __global__ __launch_bounds__(kThreads) void combine_kernel(const bf16_t* __restr
 
 // reduce_partials on lists of expert outputs, whose rows come in any order and number.  Three small
 // launches: the counters are cleared; every entry p takes one of its row's 16 slots (a layout gives a
-// row at most 16 entries); a workgroup per row sorts its slots and sums.  A row with more entries
-// looks for them in row_of instead, 256 at a time, in order.  Bound by latency (three dependent
-// launches) for decode-sized calls, by the reads of part in the last launch for large ones.
+// row at most 16 entries), and those after the 16th are chained; a workgroup per row puts its entries
+// in order and sums.  Bound by latency (three dependent launches) for decode-sized calls, by the reads
+// of part in the last launch for large ones.
 // Building the inverse of row_of with a concatenation of part, a sort, a histogram, a scan and
 // gathers took 24 launches, two of them waited for, 108 us of GPU time for 64 rows of 8 entries
 // (H = 2048) and 170 us for 2000 of 6; these three take 12.4 and 22.1 us.
-constexpr int kSlots = 16;
+//
+// A row of up to 1024 entries walks its chain with one lane (half a microsecond a step, rows side by
+// side) and ranks the entries in LDS.  It looks for them in row_of instead, 256 at a time, in order,
+// where that is no longer (fewer than 128 entries of the call for each step: few rows can be so), where
+// it has more, or where the workspace has no room for chains.  Looking in row_of for every row of more
+// than 16 entries grows with rows * entries: 20,000 rows of 20 (H = 512) took 7480 us and take 164, 8192
+// of 32 (H = 2048) 2140 us and 265.
+constexpr int kSlots = 16;            // entries of a row with a place of their own
+constexpr int kListed = 1024;         // most entries of a row listed in LDS
+constexpr int kEntriesPerStep = 128;  // entries of the call per step of a chain
 
-__global__ __launch_bounds__(kThreads) void reduce_clear(int32_t* __restrict__ count, int64_t n) {
-  for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads)
+// head (nullable): 0, or 1 + the first entry of row r's chain; next[p] likewise the one after p
+__global__ __launch_bounds__(kThreads) void reduce_clear(int32_t* __restrict__ count, int64_t rows,
+                                                         int32_t* __restrict__ head) {
+  for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i <= rows;
+       i += (int64_t)gridDim.x * kThreads) {
     count[i] = 0;
+    if (head && i < rows) head[i] = 0;
+  }
 }
 // count[r]: entries of row r; count[rows]: entries outside [0, rows) (left out)
 __global__ __launch_bounds__(kThreads) void reduce_slots(const int64_t* __restrict__ row_of,
                                                          int64_t entries, int64_t rows,
                                                          int32_t* __restrict__ count,
-                                                         int32_t* __restrict__ slots) {
+                                                         int32_t* __restrict__ slots,
+                                                         int32_t* __restrict__ head,
+                                                         int32_t* __restrict__ next) {
   for (int64_t p = (int64_t)blockIdx.x * kThreads + threadIdx.x; p < entries;
        p += (int64_t)gridDim.x * kThreads) {
     const int64_t r = row_of[p];
@@ -93,7 +109,10 @@ __global__ __launch_bounds__(kThreads) void reduce_slots(const int64_t* __restri
       atomicAdd(&count[rows], 1);
     } else {
       const int32_t c = atomicAdd(&count[r], 1);
-      if (c < kSlots) slots[r * kSlots + c] = (int32_t)p;
+      if (c < kSlots)
+        slots[r * kSlots + c] = (int32_t)p;
+      else if (head)
+        next[p] = atomicExch(&head[r], (int32_t)p + 1);
     }
   }
 }
@@ -108,8 +127,8 @@ __device__ __forceinline__ void add8(float (&acc)[kVec], const bf16_t* p) {
 __global__ __launch_bounds__(kThreads) void reduce_rows_kernel(
     const bf16_t* __restrict__ part, const int64_t* __restrict__ row_of, int64_t entries,
     int64_t rows, int64_t H, const int32_t* __restrict__ count, const int32_t* __restrict__ slots,
-    bf16_t* __restrict__ out) {
-  __shared__ int32_t order[kThreads];
+    const int32_t* __restrict__ head, const int32_t* __restrict__ next, bf16_t* __restrict__ out) {
+  __shared__ int32_t order[kListed], found[kListed];
   __shared__ int32_t wave_n[kThreads / 64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {
@@ -120,6 +139,25 @@ __global__ __launch_bounds__(kThreads) void reduce_rows_kernel(
       for (int j = 0; j < n; ++j) rank += __shfl(mine, j) < mine;
       if (lane < n) order[rank] = mine;
     }
+    const bool listed =
+        n > kSlots && n <= kListed && head && (int64_t)(n - kSlots) * kEntriesPerStep <= entries;
+    if (listed) {
+      if (threadIdx.x < kSlots) found[threadIdx.x] = slots[r * kSlots + threadIdx.x];
+      if (threadIdx.x == 64) {
+        int32_t p = head[r];
+        for (int i = kSlots; i < n; ++i) {
+          found[i] = p - 1;
+          p = next[p - 1];
+        }
+      }
+      __syncthreads();
+      for (int i = threadIdx.x; i < n; i += kThreads) {
+        const int32_t mine = found[i];
+        int rank = 0;
+        for (int j = 0; j < n; ++j) rank += found[j] < mine;
+        order[rank] = mine;
+      }
+    }
     __syncthreads();
     for (int64_t h0 = 0; h0 < H; h0 += kThreads * kVec) {
       const int64_t h = h0 + threadIdx.x * kVec;
@@ -128,6 +166,10 @@ __global__ __launch_bounds__(kThreads) void reduce_rows_kernel(
       for (int i = 0; i < kVec; ++i) acc[i] = 0.f;
       if (n <= kSlots) {
         if (h < H)
+          for (int j = 0; j < n; ++j) add8(acc, part + (int64_t)order[j] * H + h);
+      } else if (listed) {
+        if (h < H)
+#pragma unroll 4
           for (int j = 0; j < n; ++j) add8(acc, part + (int64_t)order[j] * H + h);
       } else {
         for (int64_t p0 = 0; p0 < entries; p0 += kThreads) {
@@ -144,6 +186,7 @@ __global__ __launch_bounds__(kThreads) void reduce_rows_kernel(
           if (hit) order[before + __popcll(hits & ((1ull << lane) - 1))] = (int32_t)p;
           __syncthreads();
           if (h < H)
+#pragma unroll 4
             for (int j = 0; j < all; ++j) add8(acc, part + (int64_t)order[j] * H + h);
           __syncthreads();
         }
@@ -169,6 +212,10 @@ extern "C" int64_t ferry_reduce_rows_workspace_bytes(int64_t rows) {
   return (rows * (kSlots + 1) + 1) * (int64_t)sizeof(int32_t);
 }
 
+extern "C" int64_t ferry_reduce_rows_full_workspace_bytes(int64_t rows, int64_t entries) {
+  return ferry_reduce_rows_workspace_bytes(rows) + (rows + entries) * (int64_t)sizeof(int32_t);
+}
+
 extern "C" int ferry_reduce_rows(const void* part, int64_t entries, int64_t hidden,
                                  const int64_t* row_of, int64_t rows, void* out, void* workspace,
                                  int64_t workspace_bytes, void* stream) {
@@ -183,21 +230,25 @@ extern "C" int ferry_reduce_rows(const void* part, int64_t entries, int64_t hidd
                   "workspace too small (%lld < %lld bytes)", (long long)workspace_bytes,
                   (long long)ferry_reduce_rows_workspace_bytes(rows));
   hipStream_t s = (hipStream_t)stream;
-  // words: [count of each row | entries outside the rows | slots]
+  // words: [count of each row | entries outside the rows | slots | chain heads | chains]
   int32_t* count = (int32_t*)workspace;
   int32_t* slots = count + rows + 1;
+  int32_t* head = workspace_bytes >= ferry_reduce_rows_full_workspace_bytes(rows, entries)
+                      ? slots + rows * kSlots
+                      : nullptr;
+  int32_t* next = head ? head + rows : nullptr;
   auto blocks = [](int64_t n) { return dim3((unsigned)(n < 1 ? 1 : (ceil_div(n, kThreads) < 4096 ? ceil_div(n, kThreads) : 4096))); };
-  launch("reduce_clear", reduce_clear, blocks(rows + 1), dim3(kThreads), 0, s, count, rows + 1);
+  launch("reduce_clear", reduce_clear, blocks(rows + 1), dim3(kThreads), 0, s, count, rows, head);
   FERRY_LAUNCHED("reduce_clear");
   if (entries > 0) {
     launch("reduce_slots", reduce_slots, blocks(entries), dim3(kThreads), 0, s, row_of, entries, rows,
-           count, slots);
+           count, slots, head, next);
     FERRY_LAUNCHED("reduce_slots");
   }
   if (rows > 0) {
     launch("reduce_rows_kernel", reduce_rows_kernel, dim3((unsigned)(rows < (1 << 30) ? rows : (1 << 30))),
            dim3(kThreads), 0, s, (const bf16_t*)part, row_of, entries, rows, hidden, count, slots,
-           (bf16_t*)out);
+           head, next, (bf16_t*)out);
     FERRY_LAUNCHED("reduce_rows_kernel");
   }
   return 0;

@@ -528,8 +528,8 @@ def reduce_partials(parts, rows, received, hidden, like):
     if entries > n // hidden:
         raise RuntimeError('rows must not outnumber the rows of parts')
     out = torch.empty((received, hidden), dtype=torch.bfloat16, device=dev)
-    ws = torch.empty(int(lib().ferry_reduce_rows_workspace_bytes(received)) // 4, dtype=torch.int32,
-                     device=dev)
+    ws = torch.empty(lib().ferry_reduce_rows_full_workspace_bytes(received, entries) // 4,
+                     dtype=torch.int32, device=dev)
     check(lib().ferry_reduce_rows(part_at, entries, hidden, rows_at, received, out.data_ptr(),
                                   ws.data_ptr(), ws.numel() * 4, _stream_of(out)),
           'reduce_partials')

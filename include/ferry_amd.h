@@ -196,9 +196,12 @@ int ferry_combine_add(const void* part, const int32_t* pair_pos, int64_t tokens,
  * then bf16).  part is bf16 [entries, hidden], row_of int64 [entries], out bf16 [rows, hidden].
  * After the call int32 word `rows` of `workspace` (device memory, at least
  * ferry_reduce_rows_workspace_bytes(rows) bytes) holds the number of entries whose row lies outside
- * [0, rows) (they are left out), for the caller to read when it wants the check.
+ * [0, rows) (they are left out), for the caller to read when it wants the check.  A workspace of
+ * ferry_reduce_rows_full_workspace_bytes(rows, entries) bytes gives the same bits and saves rows of
+ * more than 16 entries a search of the whole of row_of each.
  */
 int64_t ferry_reduce_rows_workspace_bytes(int64_t rows);
+int64_t ferry_reduce_rows_full_workspace_bytes(int64_t rows, int64_t entries);
 int ferry_reduce_rows(const void* part, int64_t entries, int64_t hidden, const int64_t* row_of,
                       int64_t rows, void* out, void* workspace, int64_t workspace_bytes,
                       void* stream);

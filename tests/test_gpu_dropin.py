@@ -256,3 +256,37 @@ def test_execute_experts_row_lists(device):
         ops.execute_experts(cache, x, w, slots, [t.cpu() for t in rows.split(sizes)], cols.split(sizes), H, I)
     with pytest.raises(RuntimeError):
         ops.execute_experts(cache, x, w, [6, 1, 0, 2, 3], rows.split(sizes), cols.split(sizes), H, I)
+
+
+@pytest.mark.parametrize('counts,entries', [
+    ([16, 17, 20, 0, 24], 2048),          # chains of 1, 4 and 8; the longest that 2048 entries allow is 16
+    ([32, 33, 15], 2048),                 # 16 and 17 steps
+    ([1024, 1025, 1023, 16], 130000),     # the longest listed row
+    ([1, 2000], 2001),
+])
+def test_reduce_rows_of_many_entries(device, counts, entries):
+    """Rows of up to and past 16 and 1024 entries among others, in any order, with the workspace that
+    holds chains of them and with the smallest: bit-equal to the fp32 sums in order, nothing written
+    past the workspace's size."""
+    from ferry_amd._lib import last_error, lib
+    H = 24
+    rng = np.random.default_rng(entries + len(counts))
+    rows = len(counts) + -(-(entries - sum(counts)) // 7)
+    row_of = np.concatenate([np.repeat(np.arange(len(counts)), counts),
+                             len(counts) + np.arange(entries - sum(counts)) // 7])
+    row_of = torch.from_numpy(rng.permutation(row_of))
+    part = torch.randn((entries, H), generator=torch.Generator().manual_seed(entries)).to(torch.bfloat16)
+    want = reduce_partials_ref([part], [row_of], rows, H)
+    dp, dr = part.to(device), row_of.to(device)
+    small, full = lib().ferry_reduce_rows_workspace_bytes(rows), lib().ferry_reduce_rows_full_workspace_bytes(rows, entries)
+    assert small < full
+    stream = torch.cuda.current_stream().cuda_stream
+    for nbytes in (full, full - 4, small):
+        out = torch.full((rows, H), float('nan'), dtype=torch.bfloat16, device=device)
+        ws = torch.full((full // 4 + 1,), -5, dtype=torch.int32, device=device)
+        assert lib().ferry_reduce_rows(dp.data_ptr(), entries, H, dr.data_ptr(), rows, out.data_ptr(), ws.data_ptr(),
+                                       nbytes, stream) == 0, last_error()
+        assert torch.equal(out.cpu().view(torch.int16), want.view(torch.int16)), nbytes
+        assert int(ws[rows]) == 0 and int(ws[-1]) == -5
+        if nbytes != full:
+            assert (ws[small // 4:] == -5).all()
