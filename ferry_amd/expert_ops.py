@@ -7,6 +7,7 @@ so that call sites written against the reference work unchanged; the fused hot-p
 points (router_topk, layout, expert_ffn, combine, history_update) are exposed next to them.
 All tensors are CUDA (HIP) tensors; every op runs on the current stream.
 """
+import math
 from operator import add, attrgetter
 
 import numpy as np
@@ -415,12 +416,14 @@ _get_device, _is_contiguous = torch.Tensor.get_device, torch.Tensor.is_contiguou
 _dtype = attrgetter('dtype')
 
 
-def _joined(tensors, dtype, device):
+def _joined(tensors, dtype, device, unit=1):
     """(address, elements, owner) of the tensors one after the other, as ``dtype``: in place where
     they already follow each other in memory (views that split one tensor), else concatenated.
-    ``owner`` keeps the memory alive."""
+    ``owner`` keeps the memory alive.  Each tensor must hold a multiple of ``unit`` elements."""
     # builtin calls over the whole list: a Python loop over 100 views takes twice the time
     sizes = list(map(_numel, tensors))
+    if math.gcd(unit, *sizes) != unit:
+        raise RuntimeError(f'every part must hold whole rows of {unit} elements')
     parts = tensors if all(sizes) else [t for t in tensors if t.numel()]
     if not parts:
         return 0, 0, None
@@ -518,12 +521,10 @@ def reduce_partials(parts, rows, received, hidden, like):
         return torch.zeros((received, hidden), dtype=torch.bfloat16, device=like.device)
     _dev(parts[0], 'parts', contiguous=False)   # the sums are written to memory on this device
     dev = parts[0].device
-    part_at, n, _parts = _joined(parts, torch.bfloat16, dev)
+    part_at, n, _parts = _joined(parts, torch.bfloat16, dev, unit=hidden)
     if part_at % 16:
         _parts = torch.cat([p.reshape(-1) for p in parts])
         part_at = _parts.data_ptr()
-    if any(map(hidden.__rmod__, map(_numel, parts))):
-        raise RuntimeError('every part must hold whole rows of hidden elements')
     rows_at, entries, _rows = _joined(rows, torch.int64, dev)
     if entries > n // hidden:
         raise RuntimeError('rows must not outnumber the rows of parts')
