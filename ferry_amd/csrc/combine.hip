@@ -246,7 +246,7 @@ extern "C" int ferry_reduce_rows(const void* part, int64_t entries, int64_t hidd
     FERRY_LAUNCHED("reduce_slots");
   }
   if (rows > 0) {
-    launch("reduce_rows_kernel", reduce_rows_kernel, dim3((unsigned)(rows < (1 << 30) ? rows : (1 << 30))),
+    launch("reduce_rows_kernel", reduce_rows_kernel, dim3((unsigned)(rows < kMaxGrid ? rows : kMaxGrid)),
            dim3(kThreads), 0, s, (const bf16_t*)part, row_of, entries, rows, hidden, count, slots,
            head, next, (bf16_t*)out);
     FERRY_LAUNCHED("reduce_rows_kernel");

@@ -71,6 +71,10 @@ __host__ __device__ inline bf16_t f32_to_bf16(float f) {
 // the float value of v rounded to bf16
 __host__ __device__ inline float bf16r(float v) { return bf16_to_f32(f32_to_bf16(v)); }
 
+// Most workgroups (of up to 512 threads) that a grid-stride kernel is launched with: a launch's
+// threads are counted in 32 bits (2^24 + 3 workgroups of 256 ran as 3).
+constexpr int64_t kMaxGrid = 1 << 22;
+
 __host__ __device__ inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Per-launch kernel timing (ferry_timing_enable): when on, kernels are launched with

@@ -152,7 +152,7 @@ extern "C" int ferry_unpack_dispatch(const void* payload, int64_t packets, int64
   FERRY_CHECK_ARG(payload && hidden_out && weights_out, "null pointer argument");
   const int64_t hbytes = 2 * hidden_size, wbytes = 2 * topk, pitch = hbytes + wbytes + topk;
   const int vec16 = ((uintptr_t)hidden_out & 15) == 0 && (hbytes & 15) == 0;
-  const int64_t grid = packets < (1 << 30) ? packets : (1 << 30);
+  const int64_t grid = packets < kMaxGrid ? packets : kMaxGrid;
   launch("unpack_dispatch_kernel", unpack_dispatch_kernel, dim3((unsigned)grid), dim3(kThreads), 0,
          (hipStream_t)stream, (const uint8_t*)payload, packets, hbytes, wbytes, pitch,
          (uint8_t*)hidden_out, (uint8_t*)weights_out, vec16);

@@ -290,3 +290,21 @@ def test_reduce_rows_of_many_entries(device, counts, entries):
         assert int(ws[rows]) == 0 and int(ws[-1]) == -5
         if nbytes != full:
             assert (ws[small // 4:] == -5).all()
+
+
+def test_more_rows_than_one_grid_holds(device):
+    """2^24 packets and received rows (2^32 threads, where a launch's thread count wraps, if each had a
+    workgroup of its own): the first, the last and those about the largest grid."""
+    from ferry_amd import expert_ops as ops
+    n, H, k = 1 << 24, 8, 1
+    raw = torch.randint(256, (n, 2 * H + 3 * k), dtype=torch.uint8, device=device)
+    x, w = ops.unpack_dispatch(raw, H, k)
+    for a in (0, (1 << 22) - 2, n - 4):
+        b = slice(a, a + 4)
+        assert torch.equal(x[b].view(torch.uint8), raw[b, :2 * H]) and torch.equal(w[b].view(torch.uint8), raw[b, 2 * H:-k])
+    del raw, w
+    rows = torch.arange(n, device=device)
+    out = ops.reduce_partials([x], [rows.flip(0)], n, H, x)
+    for a in (0, (1 << 22) - 2, n - 4):
+        want = x[n - a - 4:n - a].flip(0)
+        assert ((out[a:a + 4] == want) | want.isnan()).all()
