@@ -10,6 +10,13 @@ import torch
 from . import expert_ops as ops
 
 
+def _slots_of(slot_of, experts):
+    """``int(slot_of[e])`` of each expert; ``slot_of`` is anything that can be indexed so."""
+    if isinstance(slot_of, np.ndarray) and slot_of.dtype.kind in 'iu' and slot_of.ndim == 1:
+        return slot_of[experts].tolist()
+    return [int(slot_of[e]) for e in experts]
+
+
 def device_layout(selected, destinations, tokens_per_rank, rank, experts, slot_of, weights=None):
     """Same contract as ferry/layout.py:78-94 at world = 1.
 
@@ -32,9 +39,9 @@ def device_layout(selected, destinations, tokens_per_rank, rank, experts, slot_o
     lay, starts = ops.layout_on_host(sel, weights, experts)   # the reference's index checks
     sizes = np.diff(starts)
     active = np.flatnonzero(sizes)
-    slots = np.asarray(slot_of)[active]
-    assert np.all(slots >= 0), 'expert scheduled on this rank is not cached here'
+    slots = _slots_of(slot_of, active)
+    assert all(s >= 0 for s in slots), 'expert scheduled on this rank is not cached here'
     split = sizes[active].tolist()
-    groups = list(zip(active.tolist(), lay.rows.split(split), lay.cols.split(split), slots.tolist()))
+    groups = list(zip(active.tolist(), lay.rows.split(split), lay.cols.split(split), slots))
     return dict(send_idx=torch.arange(T, device='cuda'), send_ids=lay.send_ids,
                 send_counts=[T], recv_counts=[T], groups=groups, layout=lay)

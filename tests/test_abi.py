@@ -526,3 +526,16 @@ def test_reduce_partials_refuses_parts_of_broken_rows(monkeypatch):
     rows = [torch.zeros(1, dtype=torch.int64)] * 2
     with pytest.raises(RuntimeError, match='whole rows'):
         ops.reduce_partials(parts, rows, 2, 8, parts[0])
+
+
+def test_group_slots_of_any_mapping():
+    """device_layout takes slot_of as whatever can be indexed by an expert."""
+    import torch
+    from ferry_amd.layout import _slots_of
+    table = [5, -1, 3, 0, 9]
+    active = np.array([0, 2, 3])
+    for slot_of in (table, tuple(table), dict(enumerate(table)), {0: 5, 2: 3, 3: 0}, np.array(table),
+                    np.array(table, np.int16), np.array(table, float), torch.tensor(table)):
+        got = _slots_of(slot_of, active)
+        assert got == [5, 3, 0] and all(type(s) is int for s in got)
+    assert _slots_of({}, active[:0]) == []

@@ -308,3 +308,21 @@ def test_more_rows_than_one_grid_holds(device):
     for a in (0, (1 << 22) - 2, n - 4):
         want = x[n - a - 4:n - a].flip(0)
         assert ((out[a:a + 4] == want) | want.isnan()).all()
+
+
+def test_device_layout_slot_tables(device):
+    """slot_of as an array, list, dict and CUDA tensor leads to the same groups; an active expert
+    without a slot is refused."""
+    from ferry_amd.layout import device_layout
+    E, k, T = 12, 3, 20
+    sel, _ = _routing(T, E, k, 6, np.random.default_rng(0))
+    active = sorted(set(sel.reshape(-1).tolist()))
+    table = np.full(E, -1)
+    table[active] = np.arange(len(active))[::-1]
+    forms = (table, table.tolist(), {e: table[e] for e in active}, torch.from_numpy(table).to(device))
+    for slot_of in forms:
+        groups = device_layout(sel.numpy(), None, T, 0, E, slot_of)['groups']
+        assert [(g[0], g[3]) for g in groups] == [(e, int(table[e])) for e in active]
+    table[active[1]] = -1
+    with pytest.raises(AssertionError, match='not cached'):
+        device_layout(sel.numpy(), None, T, 0, E, table)
