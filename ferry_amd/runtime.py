@@ -370,8 +370,10 @@ class OffloadRuntime:
 
         # 4. experts: resident first, then the fetched ones (chunk by chunk as they land)
         common = (hidden, lay, buf, T, k, handle)
-        # CUs that the tiled kernels leave to the unpacking of rows still being copied
-        spare = UNPACK_CUS if chunked and self.packed is not None and len(fetches) else 0
+        # CUs that the tiled kernels leave to the unpacking of rows still being copied (without
+        # overlap the call waits for all of them before its first expert)
+        spare = (UNPACK_CUS if chunked and self.overlap and self.packed is not None and len(fetches)
+                 else 0)
         n_active, n_resident = lists.sizes[0], lists.sizes[3]
         if not self.timing:
             # the reads below are marked by the next call's ID event on this stream (or by

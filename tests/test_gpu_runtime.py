@@ -378,3 +378,31 @@ def test_runtime_raises_after_decode_ffn_timeout(device):
         ops.ffn_set_sync_spin_limit(None)
     with pytest.raises(RuntimeError, match='gave up'):
         rt.close()
+
+
+@pytest.mark.parametrize('overlap', [True, False])
+def test_spare_cus_only_beside_copies(device, overlap):
+    """A large packed call with misses leaves CUs to the unpacking only where it runs beside the
+    copies; serial calls, which have waited for them, use all CUs.  The same output both ways."""
+    from ferry_amd import workloads
+    from ferry_amd.model import ModelSpec
+    from ferry_amd.quota import Topology
+    from ferry_amd.runtime import CHUNK_MIN_PAIRS, UNPACK_CUS, OffloadRuntime
+    spec = ModelSpec('qwen3_moe', (0,), 16, 4, 256, 128)
+    rt = OffloadRuntime(spec, workloads.make_pool(spec, 1, seed=3), [16], 'ferry', Topology.uniform(1, 16),
+                        overlap=overlap, pack=True)
+    T = CHUNK_MIN_PAIRS // 4
+    g = torch.Generator().manual_seed(0)
+    x = torch.randn((T, 256), generator=g).to(torch.bfloat16).to(device)
+    w = torch.full((T, 4), 0.25, dtype=torch.bfloat16, device=device)
+    sel = torch.rand((T, 16), generator=g).topk(4, dim=1).indices.to(device)
+    seen = []
+
+    def shared(rows, out, spare_cus=0):
+        seen.append(spare_cus)
+        return out.zero_()
+    outs = [rt.execute(0, x, sel, w, None, shared=shared).clone() for _ in range(2)]
+    torch.cuda.synchronize()
+    assert seen == [UNPACK_CUS if overlap else 0, 0]      # the second call has no misses
+    assert torch.equal(*outs)
+    rt.close()
