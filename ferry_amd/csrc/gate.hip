@@ -120,7 +120,7 @@ extern "C" int ferry_gate_logits(const void* x, int64_t tokens, int64_t hidden, 
   FERRY_CHECK_ARG(tokens >= 0 && experts >= 1 && experts <= 65536, "bad sizes");
   FERRY_CHECK_ARG(hidden >= 64 && hidden % 64 == 0 && hidden <= (1 << 24),
                   "hidden must be a multiple of 64 in [64, 2^24]");
-  FERRY_CHECK_ARG(tokens <= (int64_t)1 << 34, "too many tokens");
+  FERRY_CHECK_ARG(tokens < (int64_t)1 << 30, "too many tokens");   // 256 threads for each 64 of them
   if (tokens == 0) return 0;
   FERRY_CHECK_ARG(x && w && out, "null pointer argument");
   FERRY_CHECK_ARG(((uintptr_t)x | (uintptr_t)w) % 16 == 0, "x and w must be 16-byte aligned");

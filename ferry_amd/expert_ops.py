@@ -13,6 +13,7 @@ from operator import add, attrgetter
 import numpy as np
 import torch
 import torch.nn.functional as F
+from torch.autograd.forward_ad import unpack_dual
 
 from ._lib import check, lib
 from ._lib import check as _check_status
@@ -119,21 +120,30 @@ def router_topk(logits, topk, renorm=True, scale=1.0, sorted=True, return_probs=
     return (w, idx, probs) if return_probs else (w, idx)
 
 
+def _gate_operand(t):
+    """A bf16 CUDA matrix that the gate kernel can read as it is, and that torch does not watch
+    (autograd, forward mode, a transform: those tensors' address is not theirs to ask)."""
+    if not (t.dtype is torch.bfloat16 and t.is_cuda and t.dim() == 2 and t.numel() and t.is_contiguous()
+            and not (t.requires_grad and torch.is_grad_enabled())
+            and unpack_dual(t).tangent is None):
+        return False
+    try:
+        return t.data_ptr() % 16 == 0
+    except RuntimeError:
+        return False
+
+
 def gate_logits(x, weight):
     """fp32 router logits of a gate: ``F.linear(x.float(), weight.float())`` (the DeepSeek-V2 gate
     feeding ferry/model.py:151-158).
 
     Plain bf16 CUDA matrices go to a kernel that reads them as they are (another order of the fp32
-    additions); everything else, and a call that autograd or autocast takes part in, is the torch
-    expression."""
-    if (x.dtype is torch.bfloat16 and weight.dtype is torch.bfloat16 and x.is_cuda
-            and x.dim() == 2 and weight.dim() == 2 and x.shape[1] == weight.shape[1]
-            and x.shape[1] % 64 == 0 and x.numel() and weight.numel()
-            and x.get_device() == weight.get_device()
-            and x.is_contiguous() and weight.is_contiguous()
-            and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
-            and not (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
-            and not torch.is_autocast_enabled() and torch.autograd.forward_ad._current_level < 0):
+    additions); everything else, and a call that autograd, autocast, a transform or a trace takes part
+    in, is the torch expression."""
+    if (not torch.jit.is_tracing() and not torch.is_autocast_enabled()
+            and _gate_operand(x) and _gate_operand(weight) and x.shape[1] == weight.shape[1]
+            and x.shape[1] % 64 == 0 and x.shape[1] <= 1 << 24 and x.shape[0] < 1 << 30
+            and weight.shape[0] <= 65536 and x.get_device() == weight.get_device()):
         out = torch.empty((x.shape[0], weight.shape[0]), dtype=torch.float32, device=x.device)
         check(lib().ferry_gate_logits(x.data_ptr(), x.shape[0], x.shape[1], weight.data_ptr(),
                                       weight.shape[0], out.data_ptr(), _stream_of(x)), 'gate_logits')

@@ -227,8 +227,8 @@ int ferry_unpack_dispatch(const void* payload, int64_t packets, int64_t hidden_s
 /*
  * Router logits of a gate with bf16 weights in fp32: out[tokens, experts] = fp32(x) fp32(w)^T for
  * bf16 x[tokens, hidden] and w[experts, hidden] (the DeepSeek-V2 gate that feeds
- * ferry/model.py:151-158), fp32 accumulation.  hidden must be a multiple of 64, x and w 16-byte
- * aligned.
+ * ferry/model.py:151-158), fp32 accumulation.  hidden must be a multiple of 64 (at most 2^24), x and w
+ * 16-byte aligned, with fewer than 2^30 tokens and at most 65,536 experts.
  */
 int ferry_gate_logits(const void* x, int64_t tokens, int64_t hidden, const void* w,
                       int64_t experts, float* out, void* stream);

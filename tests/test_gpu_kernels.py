@@ -402,6 +402,32 @@ def test_gate_logits_other_forms(device):
         assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isinf(), b.isinf())
         assert torch.equal(a[a.isinf()], b[b.isinf()])
 
+def test_gate_logits_transforms_and_limits(device):
+    """Calls that torch traces or transforms (forward mode, vmap, jit.trace), and more experts than
+    the gate kernel takes, are torch's expression."""
+    import torch.autograd.forward_ad as fwd
+    import torch.nn.functional as F
+    ops = _ops()
+    g = torch.Generator(device=device).manual_seed(1)
+    x, tx = (torch.randn((3, 20, 128), generator=g, device=device).to(torch.bfloat16) for _ in range(2))
+    w, tw = (torch.randn((40, 128), generator=g, device=device).to(torch.bfloat16) for _ in range(2))
+    want = F.linear(x.float(), w.float())
+    close = dict(rtol=1e-4, atol=1e-3)
+    with fwd.dual_level():
+        for a, b, t in ((fwd.make_dual(x[0], tx[0]), w, F.linear(tx[0].float(), w.float())),
+                        (x[0], fwd.make_dual(w, tw), F.linear(x[0].float(), tw.float()))):
+            y, ty = fwd.unpack_dual(ops.gate_logits(a, b))
+            torch.testing.assert_close(y, want[0], **close)
+            torch.testing.assert_close(ty, t, **close)
+    torch.testing.assert_close(torch.vmap(lambda a: ops.gate_logits(a, w))(x), want, **close)
+    _, ty = torch.func.jvp(lambda a: ops.gate_logits(a, w), (x[0],), (tx[0],))
+    torch.testing.assert_close(ty, F.linear(tx[0].float(), w.float()), **close)
+    traced = torch.jit.trace(ops.gate_logits, (x[0], w))
+    torch.testing.assert_close(traced(x[1], w), want[1], **close)
+    many = torch.randn((65537, 64), generator=g, device=device).to(torch.bfloat16)
+    y = ops.gate_logits(x[0, :, :64].contiguous(), many)
+    torch.testing.assert_close(y, F.linear(x[0, :, :64].float(), many.float()), **close)
+
 
 @pytest.mark.parametrize('E,k', [(128, 8), (64, 6), (255, 9), (33, 1), (9, 9), (1, 1)])
 def test_history_demand_records_plan_like_ids(device, E, k):
