@@ -11,7 +11,7 @@
 // Design: one token per lane.  Within a wavefront the rank of a token among the earlier tokens that
 // chose the same expert is a popcount of a 64-bit per-expert lane mask built with LDS atomic ORs;
 // the wavefront and block offsets come from exclusive scans.  No global atomics are used, so the
-// permutation is deterministic.  Up to 512 tokens a single block (of as many wavefronts as the
+// permutation is deterministic.  For few tokens a single block (of as many wavefronts as the
 // tokens need) does everything in one launch; more take two: per-block histograms, then the
 // scatter, in which every block sums the histograms before its own.
 //
@@ -20,9 +20,13 @@
 // and blocks of 256 tokens where the histograms then stay small (256 blocks at 65,536 tokens
 // instead of 64 of 1024).  us, with one sort width, a one-thread scan, 1024-token blocks and a scan
 // launch of its own -> now: 16 tokens (k = 8, 128 experts) 10.2 -> 6.5; 512 tokens 15.8 -> 12.1; 1024
-// tokens 25.0 -> 13.4; 8192 tokens 34.9 -> 14.4; 65,536 tokens (k = 6, 64 experts) 39 -> 16.  The one
-// launch is left at 512 tokens, where both take 12 us: one CU then spends its time on the scattered
-// stores (22.5 us at 1024 tokens).
+// tokens 25.0 -> 13.4; 8192 tokens 34.9 -> 14.4; 65,536 tokens (k = 6, 64 experts) 39 -> 16.
+//
+// The one launch is bound by one CU's scattered stores, so its line is drawn in (token, expert) pairs:
+// us, one launch - two, 8 IDs of 128: 400 tokens 10.2 - 10.8, 512 tokens 11.8 - 10.9, 1024 tokens 21 -
+// 11.5; 6 of 64: 512 tokens 7.8 - 9.0, 640 tokens 9.1 - 9.0; 2 of 8: 768 tokens 5.7 - 7.5, 1024 tokens
+// 6.6 - 7.8; 16 of 256, where the two launches sort twice as much: 300 tokens 20.5 - 23.2, 400 tokens
+// 25.2 - 23.2.
 #include "common.h"
 
 #include <mutex>
@@ -32,7 +36,9 @@ namespace {
 
 constexpr int kMaxE = 512;
 constexpr int kMaxK = 16;
-constexpr int kSingleTokens = 512;    // most tokens of the one-launch layout
+constexpr int kSingleTokens = 1024;   // most tokens of the one-launch layout
+constexpr int kSinglePairs8 = 3200;   // ... and of (token, expert) pairs, for up to 8 IDs a token
+constexpr int kSinglePairs16 = 5120;  // ... and for up to 16
 constexpr int kMaxBlock = 1024;       // most tokens of a block of the two-launch layout
 
 template <int KM>
@@ -377,7 +383,7 @@ extern "C" int ferry_layout(const int64_t* selected, const void* weights_bf16, i
   const int k = (int)topk, E = (int)experts;
   const bf16_t* w = (const bf16_t*)weights_bf16;
   bf16_t* ws = (bf16_t*)w_sorted_bf16;
-  if (tokens <= kSingleTokens) {
+  if (tokens <= kSingleTokens && tokens * topk <= (topk <= 8 ? kSinglePairs8 : kSinglePairs16)) {
     const int waves = (int)ceil_div(tokens > 0 ? tokens : 1, 64);
     launch("layout_single", k <= 8 ? layout_single<8> : layout_single<16>, dim3(1), dim3(64 * waves),
            (uint32_t)BlockLds::bytes(waves, E), s, selected, w, tokens, k, E, send_ids, ws, starts,

@@ -222,7 +222,10 @@ def test_layout_bit_exact(device, T, E, k):
 
 
 @pytest.mark.parametrize('T,E,k', [(1, 3, 3), (63, 130, 9), (65, 512, 16), (1024, 512, 16),
-                                   (1025, 5, 5), (2049, 130, 7), (66000, 512, 8), (140000, 64, 6)])
+                                   (1025, 5, 5), (2049, 130, 7), (66000, 512, 8), (140000, 64, 6),
+                                   # about the last call of one launch, by pairs and by tokens
+                                   (400, 128, 8), (401, 128, 8), (320, 256, 16), (321, 256, 16),
+                                   (1024, 512, 3), (1025, 512, 3)])
 def test_layout_blocks_and_workspaces(device, T, E, k):
     """One launch and two, expert counts that are no multiple of 4 or 64, more than 8 IDs a token,
     and the two-launch layout's 256-, 512- and 1024-token blocks: the recommended workspace and one
