@@ -380,8 +380,8 @@ def run_prefill(args, device, w):
     for _ in range(args.prefill_reps):
         layer()
     torch.cuda.synchronize()
-    names = ('router_kernel', 'layout_count', 'layout_scan', 'layout_scatter', 'ffn_up_skinny',
-             'ffn_tiled_up', 'ffn_down_skinny', 'ffn_tiled_down', 'combine_kernel')
+    names = ('router_kernel', 'layout_count', 'layout_scatter', 'ffn_up_skinny', 'ffn_tiled_up',
+             'ffn_down_skinny', 'ffn_tiled_down', 'combine_kernel')
     kern = {name: launch_stats(ops, name) for name in names}
     ops.timing_enable(False)
     # plain reads of the small experts' weight byte counts where their launches run: the

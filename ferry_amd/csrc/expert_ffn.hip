@@ -20,10 +20,12 @@
 //    the full K; the expert's token rows are staged once per workgroup in LDS, the weights
 //    stream into MFMA B registers.  Launched together with the skinny experts of a list.
 //  * tiled (n_e > 64, prefill): MFMA-bound.  Persistent workgroups walk a device-computed
-//    list of 256x256 output tiles; A (gathered x rows / activation rows) and B (weight rows)
-//    tiles of 64 along K are staged by direct global->LDS loads into a swizzled,
-//    double-buffered LDS layout.  v_mfma_f32_16x16x32_bf16, eight wavefronts, the two of a SIMD
-//    taking turns on the matrix core and on memory.
+//    list of output tiles; A (gathered x rows / activation rows) and B (weight rows) tiles of 64
+//    along K are staged by direct global->LDS loads into a swizzled LDS layout.
+//    v_mfma_f32_16x16x32_bf16.  Tiles of 256x256 (ffn_tiled: two stages in LDS, eight wavefronts,
+//    the two of a SIMD taking turns on the matrix core and on memory), or, for lists that leave CUs
+//    idle with those, one of five from 256x128 down to 64x64 (ffn_tile: a ring of three to nine
+//    stages); choose_tile picks one for the list.
 // Phase 1 ("up") computes the gate and up projections together and applies silu(g)*u in the
 // epilogue; phase 2 ("down") applies the routing weight in the epilogue and writes the
 // per-(token, expert) row that the combine kernel sums.
@@ -41,7 +43,6 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -1329,10 +1330,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NC > 6 ? 2 
 // flight.  A wavefront issues two loads a phase, so "at most 12 outstanding" before the barrier
 // says that its share of the half read next has landed; nothing in the loop waits for all loads.
 // Before this schedule (one barrier and a full drain of the loads per stage, both wavefronts of a
-// SIMD waiting together) a stage took 1.7 us, now 1.31.  One dense expert of
-// 65,536 rows, H x I = 2048 x 768: up 352 -> 299 us (1173 -> 1380 TFLOP/s), down 233 -> 197 us
-// (883 -> 1049); 2048 x 1408: up 1177 -> 1411, down 1048 -> 1232; 2048 x 4096 down 1240 -> 1488.  Of
-// that, running on across tiles gives 2 % (up) and 2-6 % (down); each tile still spends about 6.5 us
+// SIMD waiting together) a stage took 1.7 us, now 1.31.  One dense expert of 65,536 rows, H x I = 2048
+// x 768, both timed in turn: up 372-391 -> 308-321 us (1060-1110 -> 1280-1340 TFLOP/s), down 255-271
+// -> 209-214 us (760-810 -> 960-990); launched back to back, at the clock that the power limit then
+// leaves, 430-455 -> 371-400 and 265-283 -> 216-227 (the card before: up 352 -> 299, down 233 -> 197
+// after idling).  2048 x 1408: up 1177 -> 1411, down 1048 -> 1232 TFLOP/s; 2048 x 4096 down 1240 -> 1488.
+// Of that, running on across tiles gives 2 % (up) and 2-6 % (down); each tile still spends about 6.5 us
 // outside its stages, most of it the SwiGLU of the up epilogue (two quarter-rate transcendentals for
 // each of a lane's 64 outputs).
 // The same products are summed in the same K order as before: results are bit-identical.
@@ -2145,15 +2148,15 @@ extern "C" int ferry_expert_ffn_spare(const void* cache, int64_t cache_rows, int
 
 // Which tile a list's tiled experts take: the one whose rounds of one tile per CU cost least.  A
 // tile costs kt stages of K plus a fixed part (tile table, row indices, first loads, epilogue); the
-// figures are fitted to 2 x 67 launches (1-64 experts of 65-4096 rows, H x I = 2048 x 768 / 1408 /
-// 2816), over which the choice costs 0.8 % more than the best tile on average, 16 % at worst (64
-// experts of 65 rows, 1.5 rounds).  A small tile has less latency, a large one less traffic per
+// figures are fitted to launches of 1-64 experts of 65-4096 rows, H x I = 2048 x 768 / 1408 / 2816.
+// Over 2 x 97 of those the choice costs 0.8 % more than the best tile on average, 14 % at worst (64
+// experts of 65 rows: 1.5 rounds).  A small tile has less latency, a large one less traffic per
 // product; so a list that leaves CUs idle with large tiles takes smaller ones.  us, 256 x 256 ->
-// chosen: shared expert (2048 x 2816) of 256 rows 39.9 -> 18.3 up, 47.4 -> 18.7 down, of 777 rows
-// 50.6 -> 33.0 and 52.3 -> 22.0; 8 experts (2048 x 1408) of 128 rows 39.5 -> 26.0 and 28.5 -> 15.4;
-// 24 experts (2048 x 768) of 100 rows 46.0 -> 41.9.  No choice beats reading the list's weights at
+// chosen: shared expert (2048 x 2816) of 256 rows 36.6 -> 17.2 up, 47.0 -> 18.2 down, of 777 rows
+// 37.8 -> 30.8 and 47.9 -> 20.8; 8 experts (2048 x 1408) of 128 rows 36.3 -> 24.6 and 24.5 -> 13.8;
+// 24 experts (2048 x 768) of 100 rows 43.8 -> 41.9.  No choice beats reading the list's weights at
 // 4.5 TB/s, and the 256 x 256 tile is preferred by 5 % (its loop is the better one when full).
-// Lists without row counts take 256 x 256 tiles.
+// The whole list takes one tile.  Lists without row counts take 256 x 256 tiles.
 struct TileCost {
   int rows_log, cols;    // 64 << rows_log rows, weight rows
   double stage, fixed;   // us
