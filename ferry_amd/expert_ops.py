@@ -13,7 +13,7 @@ from operator import add, attrgetter
 import numpy as np
 import torch
 import torch.nn.functional as F
-from torch.autograd.forward_ad import unpack_dual
+from torch.autograd import forward_ad
 
 from ._lib import check, lib
 from ._lib import check as _check_status
@@ -120,16 +120,24 @@ def router_topk(logits, topk, renorm=True, scale=1.0, sorted=True, return_probs=
     return (w, idx, probs) if return_probs else (w, idx)
 
 
-def _gate_operand(t):
-    """A bf16 CUDA matrix that the gate kernel can read as it is, and that torch does not watch
-    (autograd, forward mode, a transform: those tensors' address is not theirs to ask)."""
-    if not (t.dtype is torch.bfloat16 and t.is_cuda and t.dim() == 2 and t.numel() and t.is_contiguous()
-            and not (t.requires_grad and torch.is_grad_enabled())
-            and unpack_dual(t).tangent is None):
+def _gate_kernel_takes(x, weight):
+    """bf16 CUDA matrices that the gate kernel can read as they are, in a call that torch does not
+    watch (a trace, autocast, autograd, forward mode, a transform)."""
+    if (torch.jit.is_tracing() or x.dtype is not torch.bfloat16 or weight.dtype is not torch.bfloat16
+            or not x.is_cuda or x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1]
+            or x.shape[1] % 64 or x.shape[1] > 1 << 24 or not x.numel() or not weight.numel()
+            or x.shape[0] >= 1 << 30 or weight.shape[0] > 65536
+            or x.get_device() != weight.get_device() or not x.is_contiguous()
+            or not weight.is_contiguous() or torch.is_autocast_enabled()
+            or (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))):
+        return False
+    # outside every dual level no tensor has a tangent (asking each costs 1 us)
+    if (getattr(forward_ad, '_current_level', 0) >= 0
+            and any(forward_ad.unpack_dual(t).tangent is not None for t in (x, weight))):
         return False
     try:
-        return t.data_ptr() % 16 == 0
-    except RuntimeError:
+        return (x.data_ptr() | weight.data_ptr()) % 16 == 0
+    except RuntimeError:   # a transform's tensor: its address is not to be had
         return False
 
 
@@ -140,10 +148,7 @@ def gate_logits(x, weight):
     Plain bf16 CUDA matrices go to a kernel that reads them as they are (another order of the fp32
     additions); everything else, and a call that autograd, autocast, a transform or a trace takes part
     in, is the torch expression."""
-    if (not torch.jit.is_tracing() and not torch.is_autocast_enabled()
-            and _gate_operand(x) and _gate_operand(weight) and x.shape[1] == weight.shape[1]
-            and x.shape[1] % 64 == 0 and x.shape[1] <= 1 << 24 and x.shape[0] < 1 << 30
-            and weight.shape[0] <= 65536 and x.get_device() == weight.get_device()):
+    if _gate_kernel_takes(x, weight):
         out = torch.empty((x.shape[0], weight.shape[0]), dtype=torch.float32, device=x.device)
         check(lib().ferry_gate_logits(x.data_ptr(), x.shape[0], x.shape[1], weight.data_ptr(),
                                       weight.shape[0], out.data_ptr(), _stream_of(x)), 'gate_logits')
