@@ -57,8 +57,10 @@ enum { FERRY_BF16 = 0, FERRY_F32 = 1 };
  * w /= w.sum(), .to(bf16)) and the greedy DeepSeek-V2 gate whose outputs reach
  * ferry/model.py:151-157 (softmax, topk(sorted=False), * routed_scaling_factor, .to(bf16)).
  * Selection reproduces torch's CPU topk exactly, ties included.  probs_out (nullable)
- * receives the fp32 probabilities [T, E]; tie_rows (nullable, one int32 counter) counts
- * rows that took the exact tie-resolution path.
+ * receives the fp32 probabilities [T, E]; tie_rows (nullable, one int32 counter) counts the rows
+ * whose result depends on the algorithm's order: unsorted ones, those with a NaN or +inf logit, those
+ * of torch's partial_sort regime (k * 64 <= E), and those with a chosen probability that another
+ * element has too.
  */
 int ferry_router_topk(const void* logits, int32_t logits_dtype, int64_t tokens, int64_t experts,
                       int64_t topk, int32_t renorm, float scale, int32_t sorted,
